@@ -21,6 +21,7 @@
 //   dL/d map   (Remap) per pixel (g Iu, g Iv).
 // Images of one call share a size; `count` images lie at a fixed byte distance (batch stride).
 #include "mvx_common.hpp"
+#include <type_traits>
 
 namespace mvx {
 
@@ -43,6 +44,11 @@ MVX_DEV float px(const F32Plane &P, uint32_t img, int x, int y)
 {
     return (x >= 0 && y >= 0 && x < (int)P.w && y < (int)P.h) ? row_of(P, img, y)[x] : 0.f;
 }
+
+// two neighbouring pixels at any 4-byte aligned address
+struct __attribute__((packed, aligned(4))) float2a {
+    float x, y;
+};
 
 // one bilinear sample with everything the adjoint needs
 struct Sample {
@@ -138,89 +144,180 @@ k_remap_f32(F32Plane S, float *dst, uint32_t dw, uint32_t dh, uint32_t dStride, 
 }
 
 // ------------------------------------------------------------------ adjoint kernels --------------
-// block sum of WF_SLOTS values: wave shuffles, then LDS across the 4 waves; thread 0 writes
-MVX_DEV void block_sum_store(float (&acc)[WF_SLOTS], float *out)
+// workgroups reach the XCDs round robin; this mapping gives each XCD one contiguous run of tiles, so the
+// 128-byte lines at the edges of a tile's source footprint are in the L2 that its neighbour already filled
+MVX_DEV uint32_t xcd_order(uint32_t id, uint32_t n)
 {
-    __shared__ float part[WF_BY][WF_SLOTS];
+    const uint32_t q = n >> 3, r = n & 7u, xcd = id & 7u, k = id >> 3;
+    return xcd * q + min(xcd, r) + k;
+}
+
+// sum over each row of 16 lanes by DPP lane shifts (one instruction a step): valid in the row's last lane
+MVX_DEV float row16_sum(float v)
+{
+#define MVX_DPP_ADD(ctrl) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true))
+    MVX_DPP_ADD(0x111);   // row_shr:1
+    MVX_DPP_ADD(0x112);
+    MVX_DPP_ADD(0x114);
+    MVX_DPP_ADD(0x118);
+#undef MVX_DPP_ADD
+    return v;
+}
+
+// block sum of WF_SLOTS values: rows of 16 lanes in registers, then the block's 16 rows through LDS; slot k
+// of tile t of image img goes to partials[(img * WF_SLOTS + k) * tiles + t]
+MVX_DEV void block_sum_store(const float (&acc)[WF_SLOTS], float *out, uint32_t tiles)
+{
+    constexpr int ROWS16 = WF_BX * WF_BY / 16;
+    __shared__ float part[ROWS16][WF_SLOTS];
     const int tid = threadIdx.y * WF_BX + threadIdx.x;
 #pragma unroll
     for (int k = 0; k < WF_SLOTS; k++) {
-        float v = acc[k];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-        acc[k] = v;
+        const float v = row16_sum(acc[k]);
+        if ((tid & 15) == 15) part[tid >> 4][k] = v;
     }
-    if ((tid & 63) == 0)
-#pragma unroll
-        for (int k = 0; k < WF_SLOTS; k++) part[tid >> 6][k] = acc[k];
     __syncthreads();
-    if (tid < WF_SLOTS) out[tid] = ((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid];
-}
-
-// MODE 0: g given per pixel (gradient of an arbitrary loss); MODE 1: L2 against `T`, g = 2 weight r
-template <int MODE>
-__global__ void __launch_bounds__(WF_BX * WF_BY)
-k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, const double *Hs, float weight, float *gsrc,
-                   uint32_t gsStride, size_t gsBatch, float *partials)
-{
-    const uint32_t img = blockIdx.z;
-    const int x = blockIdx.x * WF_BX + threadIdx.x;
-    const HomF H = load_hom(Hs + 9 * img);
-    float acc[WF_SLOTS];
+    if (tid < WF_SLOTS) {
+        float v = part[0][tid];
 #pragma unroll
-    for (int k = 0; k < WF_SLOTS; k++) acc[k] = 0.f;
-    for (int r = 0; r < WF_ROWS; r++) {
-        const int y = blockIdx.y * WF_TILE_H + r * WF_BY + threadIdx.y;
-        if (x >= (int)dw || y >= (int)dh) continue;
-        const float X = (float)x, Y = (float)y;
-        float du, dv, z;
-        const bool inFront = project(H, X, Y, du, dv, z);
-        Sample s;
-        s.ok = false;
-        s.val = 0.f;
-        if (inFront) s = bilinear(S, img, x, y, du, dv);
-        float g;
-        if (MODE == 1) {
-            const float res = s.val - row_of(G, img, y)[x];
-            acc[9] += weight * res * res;
-            g = 2.f * weight * res;
-        } else {
-            g = row_of(G, img, y)[x];
-        }
-        if (!s.ok || g == 0.f) continue;
-        const float Iu = (1.f - s.fy) * (s.p01 - s.p00) + s.fy * (s.p11 - s.p10);
-        const float Iv = (1.f - s.fx) * (s.p10 - s.p00) + s.fx * (s.p11 - s.p01);
-        const float u = X + du, v = Y + dv;
-        const float a = g * Iu / z, b = g * Iv / z, c = -(a * u + b * v);
-        acc[0] += a * X; acc[1] += a * Y; acc[2] += a;
-        acc[3] += b * X; acc[4] += b * Y; acc[5] += b;
-        acc[6] += c * X; acc[7] += c * Y; acc[8] += c;
-        if (gsrc) scatter((float *)((uint8_t *)gsrc + img * gsBatch), gsStride, S.w, S.h, s, g);
+        for (int r = 1; r < ROWS16; r++) v += part[r][tid];
+        out[(size_t)tid * tiles] = v;
     }
-    const uint32_t blocks = gridDim.x * gridDim.y;
-    block_sum_store(acc, partials + ((size_t)img * blocks + blockIdx.y * gridDim.x + blockIdx.x) * WF_SLOTS);
 }
 
-// dH[img][0..8] (and loss[img]) = F64 sums of the per-workgroup partials, in a fixed order
+// n / z from a reciprocal r of z that is good to an ulp: the product, its exact remainder, one correction
+MVX_DEV float div_by(float n, float z, float r)
+{
+    const float q = n * r;
+    return fmaf(fmaf(-q, z, n), r, q);
+}
+
+MVX_DEV bool wave_all(bool v) { return __builtin_amdgcn_ballot_w64(v) == __builtin_amdgcn_ballot_w64(true); }
+
+// MODE 0: g given per pixel (gradient of an arbitrary loss); MODE 1: L2 against `G`, g = 2 weight r.
+//
+// A wave owns a strip of 64 columns and ROWS consecutive rows, one row at a time.  Bound by VALU issue
+// (about 90 instructions a row) and for large batches not far from memory (8 bytes a pixel).  What keeps the
+// instructions down: one reciprocal serves all four quotients of a pixel; a column's X is the same in all
+// of a lane's rows, so only the sums of a, b, c and of a Y, b Y, c Y are kept and the X sums formed once;
+// rows whose samples all lie inside the source, in front and with z in [2^-60, 2^60] (the usual case) take
+// their four pixels with two unchecked loads off one 32-bit offset, others clamped loads, and where z or a
+// position is out of the ordinary the plain divisions.  The sample positions follow project() operation by
+// operation, so forward and adjoint sample the same cells.  Eight waves a SIMD hide the loads better than
+// more loads in flight per wave: with two and four rows at a time (58 to 96 and 115 to 155 registers) the
+// batch below took 236 and 286 us in all, with one row 232.
+// 64 pairs of 1024x1024 and their two smaller levels (L2, no source gradient), reductions included: 417 us
+// with four divisions, checked loads, ten sums a pixel and shuffle reductions; 232 us now.
+template <int MODE, int ROWS>
+__global__ void __launch_bounds__(WF_BX * WF_BY, 8)
+k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t tilesX, const double *Hs, float weight,
+                   float *gsrc, uint32_t gsStride, size_t gsBatch, float *partials)
+{
+    const uint32_t tiles = gridDim.x;
+    const uint32_t id = xcd_order(blockIdx.y * tiles + blockIdx.x, tiles * gridDim.y);
+    const uint32_t img = id / tiles, tile = id - img * tiles;
+    const uint32_t ty = tile / tilesX, tx = tile - ty * tilesX;
+    const int yw = (int)((ty * WF_BY + __builtin_amdgcn_readfirstlane(threadIdx.y)) * ROWS);
+    const int xl = (int)(tx * WF_BX + threadIdx.x);
+    const bool inx = xl < (int)dw;
+    const int x = min(xl, (int)dw - 1);   // lanes past the right edge repeat the last column and are left out of the sums
+    const HomF H = load_hom(Hs + 9 * img);
+    const float X = (float)x;
+    const float q0 = H.h6 * X, u0 = H.d0 * X, v0 = H.h3 * X;
+    const uint8_t *gbase = (const uint8_t *)G.p + img * G.batch, *sbase = (const uint8_t *)S.p + img * S.batch;
+    // cells floor(du), floor(dv) whose four pixels lie inside the source: [lo, hi] (none when offsets or
+    // coordinates outgrow 32 bits, a float or a 24-bit product)
+    const bool small = max(max(dw, dh), max(S.w, S.h)) < (1u << 24) && S.stride < (1u << 24) && (uint64_t)S.h * S.stride < (1ull << 32);
+    const float lox = small ? -X : INFINITY, hix = (float)((int)S.w - 2) - X, hiy = (float)((int)S.h - 2);
+    float sa = 0.f, sb = 0.f, sc = 0.f, saY = 0.f, sbY = 0.f, scY = 0.f, loss = 0.f;
+#pragma unroll 1
+    for (int y = yw; y < min(yw + ROWS, (int)dh); y++) {
+        const float target = ((const float *)(gbase + (size_t)y * G.stride))[x];
+        const float Y = (float)y;
+        const float q = q0 + H.h7 * Y, z = q + H.h8;
+        const float nu = (u0 + H.h1 * Y + H.h2) - X * q, nv = (v0 + H.d4 * Y + H.h5) - Y * q;
+        float rz = __builtin_amdgcn_rcpf(z);
+        rz = fmaf(fmaf(-z, rz, 1.f), rz, rz);
+        float du = div_by(nu, z, rz), dv = div_by(nv, z, rz);
+        float fu = floorf(du), fv = floorf(dv);
+        Sample s;
+        s.ok = true;
+        s.x0 = x + (int)fu; s.y0 = y + (int)fv;
+        const bool usual = (z >= 0x1p-60f) & (z <= 0x1p60f);
+        const auto accumulate = [&](auto check) {
+            constexpr bool CHECK = decltype(check)::value;
+            s.fx = du - fu; s.fy = dv - fv;
+            const float gx = 1.f - s.fx, gy = 1.f - s.fy;
+            const float Iu = fmaf(s.fy, s.p11 - s.p10, gy * (s.p01 - s.p00)), Iv = fmaf(s.fx, s.p11 - s.p01, gx * (s.p10 - s.p00));
+            float g = target;
+            if (MODE == 1) {
+                const float top = fmaf(s.fx, s.p01, gx * s.p00), bot = fmaf(s.fx, s.p11, gx * s.p10);
+                const float val = CHECK && !s.ok ? 0.f : fmaf(s.fy, bot, gy * top);
+                const float res = val - g, wr = weight * res;
+                loss += wr * res;
+                g = 2.f * wr;
+            }
+            const bool take = (!CHECK || s.ok) & (g != 0.f);
+            if (take) {
+                const float gz = g * rz;
+                const float a = gz * Iu, b = gz * Iv, c = -fmaf(a, X + du, b * (Y + dv));
+                sa += a; sb += b; sc += c;
+                saY = fmaf(a, Y, saY); sbY = fmaf(b, Y, sbY); scY = fmaf(c, Y, scY);
+            }
+            if (gsrc && take && inx) scatter((float *)((uint8_t *)gsrc + img * gsBatch), gsStride, S.w, S.h, s, g);
+        };
+        if (wave_all(usual & (fu >= lox) & (fu <= hix) & (fv >= -Y) & (fv <= hiy - Y))) {
+            const uint32_t off = __umul24((uint32_t)s.y0, S.stride) + 4u * (uint32_t)s.x0;
+            const float2a t = *(const float2a *)(sbase + off), b = *(const float2a *)(sbase + S.stride + off);
+            s.p00 = t.x; s.p01 = t.y; s.p10 = b.x; s.p11 = b.y;
+            accumulate(std::false_type());
+        } else {
+            if (!wave_all(usual & (fabsf(du) < 1.0e7f) & (fabsf(dv) < 1.0e7f))) {
+                rz = 1.f / z;
+                du = nu / z;
+                dv = nv / z;
+                s.ok = (z > 0.f) & (fabsf(du) < 1.0e7f) & (fabsf(dv) < 1.0e7f);   // also false for NaN
+                if (!s.ok) du = dv = 0.f;
+                fu = floorf(du); fv = floorf(dv);
+                s.x0 = x + (int)fu; s.y0 = y + (int)fv;
+            }
+            // every load inside the source, pixels outside it then 0
+            const int xe = (int)S.w - 1, ye = (int)S.h - 1;
+            const int xa = min(max(s.x0, 0), xe), xb = min(max(s.x0 + 1, 0), xe), ya = min(max(s.y0, 0), ye), yb = min(max(s.y0 + 1, 0), ye);
+            const float *ra = (const float *)(sbase + (size_t)(uint32_t)ya * S.stride), *rb = (const float *)(sbase + (size_t)(uint32_t)yb * S.stride);
+            const float t0 = ra[xa], t1 = ra[xb], t2 = rb[xa], t3 = rb[xb];
+            const bool ia = xa == s.x0, ib = xb == s.x0 + 1, ja = ya == s.y0, jb = yb == s.y0 + 1;
+            s.p00 = (ia & ja) ? t0 : 0.f; s.p01 = (ib & ja) ? t1 : 0.f;
+            s.p10 = (ia & jb) ? t2 : 0.f; s.p11 = (ib & jb) ? t3 : 0.f;
+            accumulate(std::true_type());
+        }
+    }
+    float acc[WF_SLOTS] = {sa * X, saY, sa, sb * X, sbY, sb, sc * X, scY, sc, loss};
+    if (!inx)
+#pragma unroll
+        for (int k = 0; k < WF_SLOTS; k++) acc[k] = 0.f;
+    block_sum_store(acc, partials + (size_t)img * WF_SLOTS * tiles + tile, tiles);
+}
+
+// dH[img][0..8] (and loss[img]) = F64 sums of the per-workgroup partials, in a fixed order; one workgroup
+// per image and slot (64 images, 1024 partials a slot: 18 us when one workgroup took all ten slots in turn,
+// ? us now)
 __global__ void __launch_bounds__(256)
 k_reduce_partials(const float *partials, uint32_t blocks, double *gradH, double *loss, int accumulate)
 {
-    const uint32_t img = blockIdx.x;
-    __shared__ double red[256];
-    for (int k = 0; k < WF_SLOTS; k++) {
-        double v = 0.0;
-        for (uint32_t b = threadIdx.x; b < blocks; b += 256) v += (double)partials[((size_t)img * blocks + b) * WF_SLOTS + k];
-        red[threadIdx.x] = v;
-        __syncthreads();
-        for (int off = 128; off > 0; off >>= 1) {
-            if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) {
-            double *o = (k < 9) ? (gradH ? gradH + 9 * img + k : nullptr) : (loss ? loss + img : nullptr);
-            if (o) *o = accumulate ? *o + red[0] : red[0];
-        }
-        __syncthreads();
+    const uint32_t img = blockIdx.x, k = blockIdx.y;
+    __shared__ double red[4];
+    const float *p = partials + ((size_t)img * WF_SLOTS + k) * blocks;
+    double v = 0.0;
+    for (uint32_t b = threadIdx.x; b < blocks; b += 256) v += (double)p[b];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const double t = ((red[0] + red[1]) + red[2]) + red[3];
+        double *o = (k < 9) ? (gradH ? gradH + 9 * img + k : nullptr) : (loss ? loss + img : nullptr);
+        if (o) *o = accumulate ? *o + t : t;
     }
 }
 
@@ -364,18 +461,28 @@ static int warp_adjoint_common(mvx_stream_t stream, int mode, uint32_t count, ui
     if (!ws || (reinterpret_cast<uintptr_t>(ws) & 3u) || wsSize < mvx_warp_perspective_f32_workspace_size(count, dw, dh))
         return MVX_ERROR_INVALID_PARAMETERS;
     const F32Plane S{src, sw, sh, srcStride, srcBatch}, G{g, dw, dh, gStride, gBatch};
-    const dim3 grid = f32_grid(dw, dh, count);
     float *part = (float *)ws;
-    if (mode == 1)
-        hipLaunchKernelGGL(k_warp_f32_adjoint<1>, grid, dim3(WF_BX, WF_BY), 0, stream_of(stream), S, G, dw, dh, H, weight, gradSrc,
-                           gsStride, gsBatch, part);
-    else
-        hipLaunchKernelGGL(k_warp_f32_adjoint<0>, grid, dim3(WF_BX, WF_BY), 0, stream_of(stream), S, G, dw, dh, H, weight, gradSrc,
-                           gsStride, gsBatch, part);
+    const uint32_t tilesX = (dw + WF_BX - 1) / WF_BX;
+    const auto tiles_of = [&](uint32_t rows) { return (uint64_t)tilesX * ((dh + WF_BY * rows - 1) / (WF_BY * rows)); };
+    // rows per wave: setup and block sum cost about 100 instructions a wave, so eight rows where that leaves
+    // two rounds of waves or more for the 1024 SIMDs, else four (sixteen was no faster for 64 x 1024x1024)
+    const uint32_t rows = tiles_of(8) * count >= 2048 ? 8 : 4;
+    const uint64_t tiles = tiles_of(rows);
+    if (tiles > 0xffffffull || tiles * count > 0xffffffffull) return MVX_ERROR_INVALID_PARAMETERS;   // the launch's own limits
+    const auto run = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((uint32_t)tiles, count), dim3(WF_BX, WF_BY), 0, stream_of(stream), S, G, dw, dh, tilesX, H, weight,
+                           gradSrc, gsStride, gsBatch, part);
+    };
+    const auto pick = [&](auto m) {
+        constexpr int M = decltype(m)::value;
+        rows == 8 ? run(k_warp_f32_adjoint<M, 8>) : run(k_warp_f32_adjoint<M, 4>);
+    };
+    if (mode == 1) pick(std::integral_constant<int, 1>());
+    else pick(std::integral_constant<int, 0>());
     MVX_LAUNCH_CHECK();
     if (gradH || loss) {
-        hipLaunchKernelGGL(k_reduce_partials, dim3(count), dim3(256), 0, stream_of(stream), part, grid.x * grid.y, gradH, loss,
-                           accumulate);
+        hipLaunchKernelGGL(k_reduce_partials, dim3(count, WF_SLOTS), dim3(256), 0, stream_of(stream), part, (uint32_t)tiles, gradH,
+                           loss, accumulate);
         MVX_LAUNCH_CHECK();
     }
     return MVX_SUCCESS;

@@ -1,0 +1,80 @@
+"""The F32 warp's adjoint where its kernels change path: images narrower than a wave and heights off the
+row groups, sources of one row or column, samples that leave the source or lie behind the camera,
+homographies whose z leaves the range of the shared reciprocal, and scaled or rotated footprints whose
+contributions to dL/dsource do not line up from pixel to pixel.  Reference: float64 autograd.
+
+Tolerances: F32 positions carry about 1e-7 of their coordinate (below 140 here), so a bilinear weight is
+off by at most about 2e-5 and a sum of a few such terms by 1e-4 of the largest.  dL/dH is compared as a
+vector within 1e-4 plus what cell boundaries allow: the image slope jumps there, by at most 2 for values in
+[0, 1], so a sample within 4e-5 px of a boundary (twice the position error) may move its term of dL/dH by
+2 |g| / z times its coordinates."""
+import pytest
+import torch
+
+from mivisionx_amd import align
+from test_gpu_warp_adjoint import warp64
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [((1, 1), (1, 1)), ((5, 1), (3, 7)), ((1, 9), (70, 5)), ((2, 2), (63, 4)), ((64, 16), (64, 16)), ((65, 33), (65, 17)),
+         ((130, 37), (127, 35)), ((40, 50), (130, 66))]
+HOMS = {"near_identity": [1.013, 0.021, 0.37, -0.017, 0.991, -0.43, 1e-4, -2e-4, 1.0],
+        "shift_out": [1, 0, 31.3, 0, 1, -12.6, 0, 0, 1],
+        "shrink_rotate": [1.9, 0.83, -7.3, -0.77, 2.1, 5.2, 0, 0, 1],
+        "enlarge": [0.31, 0.013, 0.7, -0.02, 0.27, 0.4, 0, 0, 1],
+        "behind": [1.1, 0.1, 0.3, -0.2, 0.9, 0.6, 0.03, -0.04, 0.21],
+        "tiny_z": [1.013e-25, 0.021e-25, 0.37e-25, -0.017e-25, 0.991e-25, -0.43e-25, 0, 0, 1e-25],
+        "huge_z": [1.013e25, 0.021e25, 0.37e25, -0.017e25, 0.991e25, -0.43e25, 0, 0, 1e25]}
+
+
+def _boundary_allowance(H, g):
+    """the sum over samples near a cell boundary of 2 |g| / z |(x, y, 1)| |(u, v, 1)|, both images together"""
+    n, dh, dw = g.shape
+    ys, xs = torch.meshgrid(torch.arange(dh, dtype=torch.float64, device=g.device), torch.arange(dw, dtype=torch.float64, device=g.device),
+                            indexing="ij")
+    p = torch.stack([xs, ys, torch.ones_like(xs)], -1).reshape(-1, 3)
+    q = torch.einsum("nij,pj->npi", H.reshape(n, 3, 3), p)
+    z = q[..., 2]
+    ok = z > 0
+    uv = q[..., :2] / torch.where(ok, z, torch.ones_like(z))[..., None]
+    near = ok & ((uv - uv.round()).abs() < 4e-5).any(-1)
+    size = torch.linalg.norm(p, dim=-1)[None] * torch.sqrt(1 + (uv * uv).sum(-1))
+    return float((2 * g.double().abs().reshape(n, -1) / z * size)[near].sum())
+
+
+def _check_gH(got, want, H, g, what):
+    bound = 1e-4 * float(torch.linalg.norm(want)) + _boundary_allowance(H, g)
+    assert float(torch.linalg.norm(got - want)) <= bound, f"{what}: {got}\n{want}\nbound {bound}"
+
+
+@pytest.mark.parametrize("name", HOMS)
+@pytest.mark.parametrize("src_wh,dst_wh", SIZES)
+def test_adjoint_paths(gpu, src_wh, dst_wh, name):
+    print(f"adjoint {name}: source {src_wh}, destination {dst_wh}", flush=True)
+    (sw, sh), (dw, dh) = src_wh, dst_wh
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    src = torch.rand((2, sh, sw), generator=gen, device="cuda")
+    g = torch.rand((2, dh, dw), generator=gen, device="cuda") - 0.3
+    g[:, ::3, ::5] = 0.0
+    H = torch.tensor([HOMS[name], HOMS[name]], dtype=torch.float64, device="cuda")
+    H[1, 2] += 0.21 * H[1, 8]
+    s64, H64 = src.double().requires_grad_(True), H.clone().requires_grad_(True)
+    out = warp64(s64, H64.reshape(-1, 3, 3), (dh, dw))
+    ws, wH = torch.autograd.grad((out * g.double()).sum(), (s64, H64))
+    gs, gH = align.warp_adjoint(g, src, H)
+    assert float((gs.double() - ws).abs().max()) <= 1e-4 * max(1.0, float(ws.abs().max()))
+    _, gH_only = align.warp_adjoint(g, src, H, want_src=False)
+    _check_gH(gH, wH, H, g, "dL/dH beside dL/dsource")
+    _check_gH(gH_only, wH, H, g, "dL/dH alone")
+
+    # the fused loss: weight * sum (warp - target)^2 and its gradients, accumulated
+    l2 = align.L2Grad(src, g)
+    loss, gHl = torch.full((2,), 1.5, dtype=torch.float64, device="cuda"), torch.zeros((2, 9), dtype=torch.float64, device="cuda")
+    gsl = torch.zeros_like(src)
+    l2(H, 0.25, loss, gHl, accumulate=True, gsrc=gsl)
+    res = warp64(s64, H64.reshape(-1, 3, 3), (dh, dw)) - g.double()
+    want = 0.25 * (res ** 2).sum(dim=(1, 2))
+    ws, wH = torch.autograd.grad(want.sum(), (s64, H64))
+    assert float((loss - 1.5 - want).abs().max()) <= 1e-4 * max(1.0, float(want.abs().max()))
+    assert float((gsl.double() - ws).abs().max()) <= 1e-4 * max(1.0, float(ws.abs().max()))
+    _check_gH(gHl, wH, H, 0.5 * res.detach(), "dL/dH of the loss")
