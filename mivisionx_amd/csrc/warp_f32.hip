@@ -21,6 +21,7 @@
 //   dL/d map   (Remap) per pixel (g Iu, g Iv).
 // Images of one call share a size; `count` images lie at a fixed byte distance (batch stride).
 #include "mvx_common.hpp"
+#include <climits>
 #include <type_traits>
 
 namespace mvx {
@@ -194,6 +195,52 @@ MVX_DEV float div_by(float n, float z, float r)
 
 MVX_DEV bool wave_all(bool v) { return __builtin_amdgcn_ballot_w64(v) == __builtin_amdgcn_ballot_w64(true); }
 
+// dL/dsrc of one wave's samples, taken row by row.  Four atomics a pixel were the larger part of the
+// adjoint; neighbouring pixels add to the same source pixels, so they are merged in registers first: a lane
+// passes its right-hand column to the next lane when that lane's cell is the next one, and keeps its lower
+// row for the next image row's upper one.  Near unit scale that leaves about one atomic per pixel; samples
+// that do not line up (scaled, steeply rotated) add on their own as before.  An LDS image of the block's
+// footprint was measured too: its F32 LDS adds cost as much as the global atomics.
+MVX_DEV int dpp_prev(int old, int v) { return __builtin_amdgcn_update_dpp(old, v, 0x138, 0xf, 0xf, false); }
+MVX_DEV int dpp_next(int old, int v) { return __builtin_amdgcn_update_dpp(old, v, 0x130, 0xf, 0xf, false); }
+MVX_DEV float dpp_prev(float v) { return __int_as_float(dpp_prev(0, __float_as_int(v))); }
+
+struct SrcGrad {
+    static constexpr int NONE = INT_MIN / 2;
+    uint8_t *base;
+    uint32_t stride, w, h;
+    int bx = NONE, by = NONE;       // the pending lower row: pixels (bx, by) and (bx + 1, by)
+    float b0 = 0.f, b1 = 0.f;
+
+    MVX_DEV void add(int x, int y, float v)
+    {
+        if ((v != 0.f) & ((uint32_t)x < w) & ((uint32_t)y < h)) atomicAdd((float *)(base + (size_t)(uint32_t)y * stride) + x, v);
+    }
+    // one row, every lane of the wave active; lanes with `take` unset have nothing to add
+    MVX_DEV void row(bool take, const Sample &s, float g)
+    {
+        const int x0 = take ? s.x0 : NONE, y0 = take ? s.y0 : NONE;
+        const float gx = 1.f - s.fx, gy = 1.f - s.fy;
+        const float w00 = gx * gy, w01 = s.fx * gy, w10 = gx * s.fy, w11 = s.fx * s.fy;
+        float c00 = take && w00 != 0.f ? g * w00 : 0.f, c01 = take && w01 != 0.f ? g * w01 : 0.f;
+        float c10 = take && w10 != 0.f ? g * w10 : 0.f, c11 = take && w11 != 0.f ? g * w11 : 0.f;
+        const bool below = (x0 == bx) & (y0 == by);
+        if (!below) { add(bx, by, b0); add(bx + 1, by, b1); }
+        c00 += below ? b0 : 0.f;
+        c01 += below ? b1 : 0.f;
+        const int left = (dpp_prev(NONE - 1, x0) + 1 == x0) & (dpp_prev(NONE, y0) == y0) & (x0 != NONE);
+        const float l0 = dpp_prev(c01), l1 = dpp_prev(c11);
+        c00 += left ? l0 : 0.f;
+        c10 += left ? l1 : 0.f;
+        const bool given = dpp_next(0, left) != 0;
+        add(x0, y0, c00);
+        add(x0 + 1, y0, given ? 0.f : c01);
+        bx = x0; by = y0 + 1;
+        b0 = c10; b1 = given ? 0.f : c11;
+    }
+    MVX_DEV void finish() { add(bx, by, b0); add(bx + 1, by, b1); }
+};
+
 // MODE 0: g given per pixel (gradient of an arbitrary loss); MODE 1: L2 against `G`, g = 2 weight r.
 //
 // A wave owns a strip of 64 columns and ROWS consecutive rows, one row at a time.  Bound by VALU issue
@@ -207,9 +254,10 @@ MVX_DEV bool wave_all(bool v) { return __builtin_amdgcn_ballot_w64(v) == __built
 // more loads in flight per wave: with two and four rows at a time (58 to 96 and 115 to 155 registers) the
 // batch below took 236 and 286 us in all, with one row 232.
 // 64 pairs of 1024x1024 and their two smaller levels (L2, no source gradient), reductions included: 417 us
-// with four divisions, checked loads, ten sums a pixel and shuffle reductions; 232 us now.
-template <int MODE, int ROWS>
-__global__ void __launch_bounds__(WF_BX * WF_BY, 8)
+// with four divisions, checked loads, ten sums a pixel and shuffle reductions; 232 us now.  With dL/dsrc, 8
+// images of 509x387: 42.7 us with four atomics a pixel, 20.5 us now.
+template <int MODE, int ROWS, bool SCAT>
+__global__ void __launch_bounds__(WF_BX * WF_BY, SCAT ? 7 : 8)
 k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t tilesX, const double *Hs, float weight,
                    float *gsrc, uint32_t gsStride, size_t gsBatch, float *partials)
 {
@@ -230,6 +278,7 @@ k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t ti
     const bool small = max(max(dw, dh), max(S.w, S.h)) < (1u << 24) && S.stride < (1u << 24) && (uint64_t)S.h * S.stride < (1ull << 32);
     const float lox = small ? -X : INFINITY, hix = (float)((int)S.w - 2) - X, hiy = (float)((int)S.h - 2);
     float sa = 0.f, sb = 0.f, sc = 0.f, saY = 0.f, sbY = 0.f, scY = 0.f, loss = 0.f;
+    SrcGrad sg{(uint8_t *)gsrc + img * gsBatch, gsStride, S.w, S.h};
 #pragma unroll 1
     for (int y = yw; y < min(yw + ROWS, (int)dh); y++) {
         const float target = ((const float *)(gbase + (size_t)y * G.stride))[x];
@@ -264,7 +313,7 @@ k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t ti
                 sa += a; sb += b; sc += c;
                 saY = fmaf(a, Y, saY); sbY = fmaf(b, Y, sbY); scY = fmaf(c, Y, scY);
             }
-            if (gsrc && take && inx) scatter((float *)((uint8_t *)gsrc + img * gsBatch), gsStride, S.w, S.h, s, g);
+            if (SCAT) sg.row(take & inx, s, g);
         };
         if (wave_all(usual & (fu >= lox) & (fu <= hix) & (fv >= -Y) & (fv <= hiy - Y))) {
             const uint32_t off = __umul24((uint32_t)s.y0, S.stride) + 4u * (uint32_t)s.x0;
@@ -292,6 +341,7 @@ k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t ti
             accumulate(std::true_type());
         }
     }
+    if (SCAT) sg.finish();
     float acc[WF_SLOTS] = {sa * X, saY, sa, sb * X, sbY, sb, sc * X, scY, sc, loss};
     if (!inx)
 #pragma unroll
@@ -475,7 +525,8 @@ static int warp_adjoint_common(mvx_stream_t stream, int mode, uint32_t count, ui
     };
     const auto pick = [&](auto m) {
         constexpr int M = decltype(m)::value;
-        rows == 8 ? run(k_warp_f32_adjoint<M, 8>) : run(k_warp_f32_adjoint<M, 4>);
+        if (gradSrc) rows == 8 ? run(k_warp_f32_adjoint<M, 8, true>) : run(k_warp_f32_adjoint<M, 4, true>);
+        else rows == 8 ? run(k_warp_f32_adjoint<M, 8, false>) : run(k_warp_f32_adjoint<M, 4, false>);
     };
     if (mode == 1) pick(std::integral_constant<int, 1>());
     else pick(std::integral_constant<int, 0>());
