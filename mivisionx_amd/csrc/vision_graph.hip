@@ -35,6 +35,7 @@
 #include "rowmask.hpp"
 #include "pyramid.hpp"
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -76,6 +77,10 @@ struct GraphParams {
     uint32_t lower, upper;
     float k, thr, norm, dist;
     float normRcp;           // RN(1 / norm)
+    float hotMc;             // a score above thr needs mc > hotMc (and, k >= 0, gx2 * gy2 > hotProd)
+    float hotProd;
+    int upperBits, lowerBits;      // the Canny thresholds as float bits, magnitudes being float bits too
+    uint64_t upperAll, lowerAll;   // all ones where a threshold is negative as an int (every pixel above it)
     uint32_t capacity, candCap;
 };
 
@@ -100,26 +105,6 @@ MVX_DEV uint32_t yflat(const FrameDesc &F, const GraphParams &P, int r, int c)
     c = (int)(i - (long)r * P.yStride);
     if (c >= P.w) return 0;
     return luma(gmem(F.rgb) + (long)r * F.rgbStride + 3L * c);
-}
-
-// HafCpu_FastAtan2_Canny (ago_haf_cpu_arithmetic.cpp:9638-9656), statement order kept
-MVX_DEV uint32_t canny_sector_f(int gx, int gy)
-{
-    const uint32_t ax = (uint32_t)abs(gx) & 0xffffu, ay = (uint32_t)abs(gy) & 0xffffu;
-    const float d1 = (float)ax * 0.4142135623730950488016887242097f;
-    const float d2 = (float)ax * 2.4142135623730950488016887242097f;
-    uint32_t ret = (gx * gy) < 0 ? 3u : 1u;
-    if ((float)ay <= d1) ret = 0;
-    if ((float)ay >= d2) ret = 2;
-    return ret;
-}
-
-MVX_DEV uint16_t canny_pack_f(int gx, int gyn)
-{
-    int16_t t = (int16_t)(abs((int)(int16_t)gx) + abs((int)(int16_t)gyn));
-    t = (int16_t)(t << 2);
-    t = (int16_t)(t | (int16_t)(canny_sector_f((int16_t)gx, (int16_t)gyn) & 3u));
-    return (uint16_t)t;
 }
 
 // the value of lane + 1 of the wave (DPP wave_shl:1; lane 63 reads 0)
@@ -149,6 +134,12 @@ MVX_DEV void lunion(int *L, int a, int b)
 
 MVX_DEV float lane_next_f(float v) { return __int_as_float(lane_next(__float_as_int(v))); }
 
+// lane masks: one compare gives one (no VALU work beyond it), and masks combine, shift and wait in scalar
+// registers
+MVX_DEV uint64_t mask_of(bool v) { return __builtin_amdgcn_ballot_w64(v); }
+MVX_DEV bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+extern "C" __device__ int mvx_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+
 constexpr int FTW = 4;                                     // tiles (one wave each) per workgroup of k_front
 constexpr int RES_TILES = 4;                               // tiles per wave of k_resolve
 constexpr int CAND_MAX = ((TW + 1) / 2) * ((TH + 1) / 2);  // Harris NMS maxima of a tile are never 8-adjacent
@@ -157,11 +148,23 @@ constexpr int CAND_MAX = ((TW + 1) / 2) * ((TH + 1) / 2);  // Harris NMS maxima 
 // top to bottom, every later quantity from rolling register windows of the rows it needs, column
 // neighbours by DPP lane shifts.  At step k:
 //   luma row k -> pyramid level 0 (row k-3), the 2:1 scaled image and level 1 when their rows complete;
-//   gradient row g = k-2 (image row ty0-2+g, column tx0-2+lane) -> HG3 products and 3-column sums;
-//   Canny magnitude|sector row k-3 and Harris score row k-4 (image row ty0-1+m, column tx0-1+lane);
-//   NMS of tile row r = k-6 (image row ty0+r, column tx0+lane): Canny double threshold into 64-bit row
-//   masks (edge, strong; lane r holds row r), Harris maxima into the per-wave candidate buffer.
+//   gradient row (image row ty0+k-4, column tx0-2+lane) -> Canny magnitude and sector masks, HG3 products
+//   and 3-column sums;
+//   Canny NMS and double threshold of tile row k-5 into 64-bit row masks (edge, strong; lane r holds row r);
+//   Harris score row (image row ty0+k-5, column tx0-1+lane), Harris NMS of tile row k-6 into the per-wave
+//   candidate buffer.
 // Then the tile's hysteresis on the row masks and the settle pass.
+//
+// Bound by VALU issue, so the instructions of a row are what counts (16 frames of 3840x2160: @BEFORE@ us with
+// about 125 of them, @AFTER@ us with about @INSTR@):
+//   * luma, gradients, products and window sums are floats holding integers below 2^24 -- exact, like the
+//     integers the reference computes -- so the Canny sector test, the Harris score and |.| need no
+//     conversions; a 16-bit integer form exists for none of the float rules;
+//   * a pixel's Canny sector is never stored: its three compares leave lane masks in scalar registers, which
+//     wait there for the next row and select the NMS neighbours from there;
+//   * Harris scores above the threshold are rare, so a row first asks whether any lane can have one
+//     (gx2 * gy2 > thr * norm, then mc > thr * norm: scalar branches), and only then divides, compares
+//     and suppresses.
 template <bool INNER>
 MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P, int tx0, int ty0, int tile)
 {
@@ -185,187 +188,213 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
     // negative threshold negative scores occur, and the key flips their magnitude bits (an involution).
     // Scores are never -0 (mc is never -0), so equal keys are equal scores.
     const bool negKeys = P.thr < 0.0f;
-    const int U = (int)P.upper, Lo = (int)P.lower;
     // output columns of this lane: level 0 (luma lane), 2:1 scaled (lane 2X'+3), level 1 (lane 2X'+oxp+1)
     const int sp = lane - HY, lp1 = lane - oxp - 1;
     const bool scOut = sp >= 0 && !(sp & 1) && (sp >> 1) < TW / 2 && tx0 / 2 + (sp >> 1) < P.dw;
     const bool l1Out = lp1 >= 0 && !(lp1 & 1) && (lp1 >> 1) < TW / 2 && tx0 / 2 + (lp1 >> 1) < P.lvlW[1];
+    const bool allBody = tx0 / 2 + TW / 2 <= body;         // no column of the scaled image's scalar tail
     const bool scBody = tx0 / 2 + (sp >> 1) < body;
+    const uint64_t outCols = INNER ? (1ull << TW) - 1 : mask_of(lane < TW && ox >= 1 && ox <= w - 2);
 
-    uint32_t emLo = 0, emHi = 0, smLo = 0, smHi = 0;      // lane r: edge / strong mask of tile row r
+    int emLo = 0, emHi = 0, smLo = 0, smHi = 0;           // lane r: edge / strong mask of tile row r
     uint32_t nc = 0;                                      // candidates in the wave's buffer
-    uint32_t packedPrev = 0;                              // Canny magnitude|sector of gradient row k-3, its own column
+    uint64_t sec0 = 0, sec2 = 0, sec3 = 0;                // sector tests of the Canny centre row (see below)
+    int aPrev = 0;                                        // 2:1 scaled: rounded pair means of luma row k-1
+    float tPrev = 0.0f;                                   // luma pair sums of row k-1
     int Vb = 0;                                           // Harris score key row k-5
+    bool hotB = false;                                    // ... has a lane with a score
 
     // One step of the stream (luma row k).  Windows deeper than one row are passed in age order and
     // the step writes its new row over the oldest one, so the caller rotates the arguments instead of
     // the values (no register copies): yA..yD = luma rows k-4..k-1 (yA <- row k); dO, dN / sO, sN = rows
-    // k-2, k-1 (dO <- row k); xx0.. = HG3 sums of gradient rows g-2, g-1 (<- row g); MO, MN = Canny
-    // rows k-6, k-5 (MO <- row k-4); HO, HN = score key 3-column maxima rows k-6, k-5 (HO <- row k-4);
-    // pO, pN = RGB of rows k, k+1 (pO <- row k+2).
-    auto step = [&](const int k, uint32_t &pO, uint32_t &pN, int &yA, int &yB, int &yC, int &yD, int &dO, int &dN,
-                    int &sO, int &sN, int &xx0, int &xx1, int &xy0, int &xy1, int &yy0, int &yy1, uint32_t &MO,
-                    uint32_t &MN, int &HO, int &HN) {
+    // k-2, k-1 (dO <- row k); xx0.. = HG3 sums of the two gradient rows above (<- this row's); uO, uN / vO, vN =
+    // the two magnitude rows above at columns tx0-1+lane and tx0+lane (<- this row's); HO, HN = score key
+    // 3-column maxima rows k-6, k-5 (HO <- row k-4); pO, pN = RGB of rows k, k+1 (pO <- row k+2).
+    auto step = [&](const int k, uint32_t &pO, uint32_t &pN, float &yA, float &yB, float &yC, float &yD, float &dO,
+                    float &dN, float &sO, float &sN, float &xx0, float &xx1, float &xy0, float &xy1, float &yy0,
+                    float &yy1, int &uO, int &uN, int &vO, int &vN, int &HO, int &HN) {
         // ---- luma row k (ColorConvert Y of the RGB pixel, or the virtual plane's linear-address
         //      value); the float sum lies in [0, 256), so the truncation needs no clamp
-        int yk;
+        int yi;
         if (INNER) {
             const uint32_t cur = pO;
             if (k + 2 < YH) pO = fetch(k + 2);
             float f = (float)(cur & 0xffu) * 0.2126f;
             f = f + (float)((cur >> 8) & 0xffu) * 0.7152f;
             f = f + (float)((cur >> 16) & 0xffu) * 0.0722f;
-            yk = (int)f;
+            yi = (int)f;
         } else {
-            yk = (int)yflat(F, P, ty0 - HY + k, tx0 - HY + lane);
+            yi = (int)yflat(F, P, ty0 - HY + k, tx0 - HY + lane);
         }
+        const float yk = (float)yi;
         if (k >= HY && k < HY + th && lane >= HY && lane < HY + tw)
-            __builtin_amdgcn_raw_buffer_store_b8((uint8_t)yk, l0R, tx0 - HY + lane, (int)((uint32_t)(ty0 + k - HY) * F.lvlStride[0]), 0);
+            __builtin_amdgcn_raw_buffer_store_b8((uint8_t)yi, l0R, tx0 - HY + lane, (int)((uint32_t)(ty0 + k - HY) * F.lvlStride[0]), 0);
         // binomial column sums through one-lane shifts: t = Y[l]+Y[l+1], s = Y[l]+2Y[l+1]+Y[l+2], d = Y[l+2]-Y[l]
-        const int tk = yk + lane_next(yk);
-        const int sk = tk + lane_next(tk), dk = lane_next(tk) - tk;
+        const float tk = yk + lane_next_f(yk);
+        const float sk = tk + lane_next_f(tk), dk = lane_next_f(tk) - tk;
 
         // ---- ScaleImage 2:1 (ago_haf_cpu_geometric.cpp:2000-2045 with xscale = yscale = 2, offsets 0.5):
-        //      output row oy from luma rows 2oy+3 (k-1) and 2oy+4 (k); lane 2X'+3 holds output column X'
+        //      output row oy from luma rows 2oy+3 (k-1) and 2oy+4 (k); lane 2X'+3 holds output column X'.
+        //      The body rounds twice -- (128 a + 128 b + 0x80) >> 8 is the rounded mean of two bytes, one
+        //      v_lerp_u8 --, the scalar tail once: (128 * 128 sum + 0x8000) >> 16
+        const int ak = (int)__builtin_amdgcn_lerp((uint32_t)yi, (uint32_t)lane_next(yi), 1u);
         if (k >= 4 && !(k & 1) && k <= HY + TH - 1) {
             const int Yo = ty0 / 2 + ((k - 4) >> 1);
-            const int top = yD + lane_next(yD);                 // p00 + p01; p10 + p11 = tk
-            if (Yo < P.dh && scOut) {
-                const int v = scBody ? ((((top + 1) >> 1) + ((tk + 1) >> 1) + 1) >> 1)   // (128 a + 128 b + 0x80) >> 8, twice
-                                     : ((top + tk + 2) >> 2);                             // (128*128 sum + 0x8000) >> 16
+            int v = (int)__builtin_amdgcn_lerp((uint32_t)aPrev, (uint32_t)ak, 1u);
+            if (!allBody) v = scBody ? v : ((int)(tPrev + tk) + 2) >> 2;
+            if (Yo < P.dh && scOut)
                 __builtin_amdgcn_raw_buffer_store_b8((uint8_t)v, scR, tx0 / 2 + (sp >> 1), (int)((uint32_t)Yo * F.scaledStride), 0);
-            }
         }
+        aPrev = ak;
+        tPrev = tk;
         // ---- ScaleGaussianHalf_5x5 level 1 (ago_haf_cpu_pyramid.cpp:94-305): centre (2X+oxp, 2Y+oyp),
         //      luma rows k-4..k; the horizontal 1 4 6 4 1 is four "v + v[l+1]" steps, so lane 2X'+oxp+1
-        //      holds the sum over columns lane..lane+4 (centre lane+2)
+        //      holds the sum over columns lane..lane+4 (centre lane+2); at most 255 * 256
         if (P.levels > 1 && k >= 5 + oyp && !((k - 5 - oyp) & 1)) {
             const int oy = (k - 5 - oyp) >> 1, Yo = ty0 / 2 + oy;
             if (oy < TH / 2 && Yo >= 1 && Yo <= P.lvlH[1] - 2) {
-                int acc = (yA + yk) + 4 * (yB + yD) + 6 * yC;
-                acc = acc + lane_next(acc);
-                acc = acc + lane_next(acc);
-                acc = acc + lane_next(acc);
-                acc = acc + lane_next(acc);
+                float acc = fmaf(6.0f, yC, fmaf(4.0f, yB + yD, yA + yk));
+                acc = acc + lane_next_f(acc);
+                acc = acc + lane_next_f(acc);
+                acc = acc + lane_next_f(acc);
+                acc = acc + lane_next_f(acc);
                 if (l1Out)
-                    __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(((uint32_t)acc & 0xffffu) >> 8), l1R, tx0 / 2 + (lp1 >> 1),
+                    __builtin_amdgcn_raw_buffer_store_b8((uint8_t)((uint32_t)acc >> 8), l1R, tx0 / 2 + (lp1 >> 1),
                                                          (int)((uint32_t)Yo * F.lvlStride[1]), 0);
             }
         }
 
-        // ---- Sobel gradient row g = k-2 (linear-address luma; |gx|, |gy| <= 1020, so the reference's S16
-        //      values are these), HG3 products and 3-column sums.  HG3 rows 0 and h-1 are never written
-        //      (zero).  The products are integers whose 9-sums stay below 2^24, so int32 sums equal the
-        //      reference's float sums exactly.
-        const int g = k - 2;
-        const int gx = dO + 2 * dN + dk, gy = sk - sO;
-        int pxx = 0, pxy = 0, pyy = 0;
-        if (INNER || (ty0 - 2 + g >= 1 && ty0 - 2 + g <= h - 2)) { pxx = __mul24(gx, gx); pxy = __mul24(gx, gy); pyy = __mul24(gy, gy); }
-        asm("" : "+v"(pxx), "+v"(pxy), "+v"(pyy));   // keep the window sums as shifted adds (not mads)
-        const int hxx = pxx + lane_next(pxx + lane_next(pxx));
-        const int hxy = pxy + lane_next(pxy + lane_next(pxy));
-        const int hyy = pyy + lane_next(pyy + lane_next(pyy));
+        // ---- Sobel gradient row (linear-address luma; |gx|, |gy| <= 1020, so the reference's S16 values are
+        //      these), HG3 products and 3-column sums.  HG3 rows 0 and h-1 are never written (zero).  The
+        //      9-sums of products stay below 2^24, so every sum here is exact in any order.
+        const int yg = ty0 + k - 4;
+        const float gx = fmaf(2.0f, dN, dO) + dk, gy = sk - sO;
+        float pxx = gx * gx, pxy = gx * gy, pyy = gy * gy;
+        if (!INNER && (yg < 1 || yg > h - 2)) pxx = pxy = pyy = 0.0f;
+        const float hxx = pxx + lane_next_f(pxx + lane_next_f(pxx));
+        const float hxy = pxy + lane_next_f(pxy + lane_next_f(pxy));
+        const float hyy = pyy + lane_next_f(pyy + lane_next_f(pyy));
 
-        // ---- Harris score row k-4: Vc = mc / norm > T ? mc / norm : 0, the quotient exactly the IEEE one;
-        //      kept as its compare key, with the maximum of the key over columns lane..lane+2
-        int Vc = 0;
+        // ---- Harris score row k-4 (image row ty0+k-5): Vc = mc / norm > T ? mc / norm : 0, the quotient exactly
+        //      the IEEE one; kept as its compare key, with the maximum of the key over columns lane..lane+2
+        int Vc = 0, Hc = 0;
+        bool hot = false;
         {
-            const int yv = ty0 - 1 + (k - 4);
-            float v = 0.0f;
-            if (k >= 4 && (INNER || (x >= 1 && x <= w - 2 && yv >= 1 && yv <= h - 2))) {
-                const float gx2 = (float)(xx0 + xx1 + hxx);
-                const float gxy2 = (float)(xy0 + xy1 + hxy);
-                const float gy2 = (float)(yy0 + yy1 + hyy);
+            const int yv = ty0 + k - 5;
+            const float gx2 = (xx0 + xx1) + hxx, gy2 = (yy0 + yy1) + hyy;
+            const float prod = gx2 * gy2;
+            if (k >= 4 && mask_of(prod > P.hotProd)) {
+                const float gxy2 = (xy0 + xy1) + hxy;
                 const float tr = gx2 + gy2;
-                const float det = (gx2 * gy2) - (gxy2 * gxy2);
+                const float det = prod - (gxy2 * gxy2);
                 const float mc = det - (P.k * tr * tr);
-                const float q = div_by_const_rn(mc, P.norm, P.normRcp);
-                v = (q > P.thr) ? q : 0.0f;
-            }
-            Vc = __float_as_int(v);
-            if (negKeys) Vc ^= (Vc >> 31) & 0x7fffffff;
-        }
-        int Hc = max(Vc, lane_next(Vc));
-        Hc = max(Vc, lane_next(Hc));
-
-        // ---- Canny magnitude|sector row m = k-4 from gradient row k-3 (packed at its own column, moved
-        //      to the magnitude column: lane+1 -> lane)
-        uint32_t Mc = 0;
-        {
-            const int m = k - 4, y = ty0 - 1 + m;
-            const uint32_t shifted = (uint32_t)lane_next((int)packedPrev);
-            if (k >= 4 && (INNER || (y >= 1 && y <= h - 2 && x >= 1 && x < w))) {
-                Mc = shifted;
-            } else if (!INNER && k >= 4 && y >= 1 && y <= h - 2 && tx0 == 0) {
-                // CannySobel column 0 (ago_haf_cpu_canny.cpp:83-116 with the staged rows r0[-1] = 0 and
-                // r1[-1] = r0[ALIGN16(w)-1]); luma lanes 3, 4 are x = 0, 1 and rows k-3..k-1 are y-1..y+1
-                const int a3 = __builtin_amdgcn_readlane(yB, 3), a4 = __builtin_amdgcn_readlane(yB, 4);
-                const int b4 = __builtin_amdgcn_readlane(yC, 4);
-                const int c3 = __builtin_amdgcn_readlane(yD, 3), c4 = __builtin_amdgcn_readlane(yD, 4);
-                if (x == 0) {
-                    const int t0_1 = a4 + c4 + 2 * b4;
-                    const int t1_0 = c3 - a3, t1_1 = c4 - a4;
-                    const int t1_m1 = (w % 16 == 0) ? ((int)yflat(F, P, y - 1, w - 1) + (int)yflat(F, P, y + 1, w - 1) +
-                                                       2 * (int)yflat(F, P, y, w - 1)) : 0;
-                    Mc = canny_pack_f(t0_1, -(t1_m1 + 2 * t1_0 + t1_1));
+                if (mask_of(mc > P.hotMc)) {
+                    const float q = div_by_const_rn(mc, P.norm, P.normRcp);
+                    float v = (q > P.thr) ? q : 0.0f;
+                    if (!INNER && !(x >= 1 && x <= w - 2 && yv >= 1 && yv <= h - 2)) v = 0.0f;
+                    Vc = __float_as_int(v);
+                    if (negKeys) Vc ^= (Vc >> 31) & 0x7fffffff;
+                    Hc = max(Vc, lane_next(Vc));
+                    Hc = max(Vc, lane_next(Hc));
+                    hot = true;
                 }
             }
         }
-        packedPrev = canny_pack_f(gx, -gy);
 
-        // ---- NMS of tile row r = k-6 (image row ty0+r): magnitude rows r..r+2 = MO, MN, Mc and score
-        //      rows r..r+2 (maxima HO, raw Vb, maxima Hc), columns lane..lane+2, centre lane+1
-        if (k >= 6) {
+        // ---- Canny magnitude of this gradient row, as float bits (non-negative floats order like their
+        //      bits), zero outside rows 1..h-2 and columns 1..w-1, column 0 below; u, v = at columns tx0-1+lane
+        //      and tx0+lane
+        int mag = __float_as_int(fabsf(gx) + fabsf(gy));
+        if (!INNER) {
+            const int xg = tx0 - 2 + lane;
+            const bool rowOk = yg >= 1 && yg <= h - 2;
+            if (!(rowOk && xg >= 1 && xg < w)) mag = 0;
+            if (rowOk && tx0 == 0) {
+                // CannySobel column 0 (ago_haf_cpu_canny.cpp:83-116 with the staged rows r0[-1] = 0 and
+                // r1[-1] = r0[ALIGN16(w)-1]); luma lanes 3, 4 are x = 0, 1 and rows k-2..k are yg-1..yg+1.  It
+                // is never an NMS centre, so its sector does not matter.
+                const int a3 = __builtin_amdgcn_readlane((int)yC, 3), a4 = __builtin_amdgcn_readlane((int)yC, 4);
+                const int b4 = __builtin_amdgcn_readlane((int)yD, 4);
+                const int c3 = __builtin_amdgcn_readlane(yi, 3), c4 = __builtin_amdgcn_readlane(yi, 4);
+                if (xg == 0) {
+                    const int t0_1 = a4 + c4 + 2 * b4;
+                    const int t1_0 = c3 - a3, t1_1 = c4 - a4;
+                    const int t1_m1 = (w % 16 == 0) ? ((int)yflat(F, P, yg - 1, w - 1) + (int)yflat(F, P, yg + 1, w - 1) +
+                                                       2 * (int)yflat(F, P, yg, w - 1)) : 0;
+                    mag = __float_as_int((float)(abs(t0_1) + abs(t1_m1 + 2 * t1_0 + t1_1)));
+                }
+            }
+        }
+        const int uk = lane_next(mag), vk = lane_next(uk);
+
+        // ---- Canny NMS of tile row r = k-5 (image row ty0+r): rows uO/vO above, uN/vN the centre, uk/vk below; the
+        //      larger of the two neighbours along the centre's sector (HafCpu_FastAtan2_Canny,
+        //      ago_haf_cpu_arithmetic.cpp:9638-9656, on (gx, -gy): sector 1, or 3 where gx * -gy < 0; 0 where
+        //      |gy| <= tan(22.5) |gx|; 2 where |gy| >= tan(67.5) |gx|, the last test wins)
+        if (k >= 5 && k < TH + 5) {
+            const int r = k - 5, y = ty0 + r;
+            const int d0 = max(uN, lane_next(vN));      // left, right
+            const int d1 = max(uk, lane_next(vO));      // lower left, upper right
+            const int d2 = max(vO, vk);                 // above, below
+            const int d3 = max(uO, lane_next(vk));      // upper left, lower right
+            int nmax = in_mask(sec3 >> 2) ? d3 : d1;
+            nmax = in_mask(sec0 >> 2) ? d0 : nmax;
+            nmax = in_mask(sec2 >> 2) ? d2 : nmax;
+            const uint64_t peak = mask_of(vN > nmax), up = mask_of(vN > P.upperBits), lo = mask_of(vN > P.lowerBits);
+            const uint64_t valid = (INNER || (y >= 1 && y <= h - 2)) ? outCols : 0ull;
+            const uint64_t sb = valid & ((peak & up) | P.upperAll);
+            const uint64_t eb = valid & ((peak & (up | lo)) | P.upperAll | P.lowerAll);
+            emLo = mvx_writelane((int)(uint32_t)eb, r, emLo);
+            emHi = mvx_writelane((int)(uint32_t)(eb >> 32), r, emHi);
+            smLo = mvx_writelane((int)(uint32_t)sb, r, smLo);
+            smHi = mvx_writelane((int)(uint32_t)(sb >> 32), r, smHi);
+        }
+        {
+            const float ax = fabsf(gx), ay = fabsf(gy);
+            sec0 = mask_of(ay <= ax * 0.4142135623730950488016887242097f);
+            sec2 = mask_of(ay >= ax * 2.4142135623730950488016887242097f);
+            sec3 = mask_of((__float_as_int(gx) ^ __float_as_int(gy)) >= 0);   // (0 in either: sector 0 or 2)
+        }
+
+        // ---- Harris 3x3 NMS of tile row r = k-6: >= towards the upper-left half of the window, > towards the
+        //      lower-right; without a score in the centre row there is no maximum
+        if (k >= 6 && hotB) {
             const int r = k - 6, y = ty0 + r;
-            const bool valid = lane < TW && (INNER || (y >= 1 && y <= h - 2 && ox >= 1 && ox <= w - 2));
-            // Canny: the larger of the two neighbours along the sector's direction, packed values compared
-            // through (v | 3): mag > (n >> 2) <=> (centre | 3) > (n | 3)
-            const uint32_t a1 = (uint32_t)lane_next((int)MO), b1 = (uint32_t)lane_next((int)MN);
-            const uint32_t c1 = (uint32_t)lane_next((int)Mc);
-            const uint32_t sec = b1 & 3u;
-            const uint32_t d0 = max(MN, (uint32_t)lane_next((int)b1));     // (r+1, l), (r+1, l+2)
-            const uint32_t d1 = max(Mc, (uint32_t)lane_next((int)a1));     // (r, l+2), (r+2, l)
-            const uint32_t d2 = max(a1, c1);                               // (r, l+1), (r+2, l+1)
-            const uint32_t d3 = max(MO, (uint32_t)lane_next((int)c1));     // (r, l), (r+2, l+2)
-            const uint32_t nmax = sec == 0 ? d0 : sec == 1 ? d1 : sec == 2 ? d2 : d3;
-            const int edge = ((b1 | 3u) > (nmax | 3u)) ? (int)(b1 >> 2) : 0;
-            const bool strongPx = valid && edge > U, edgePx = valid && (edge > U || edge > Lo);
-            const uint64_t eb = __ballot(edgePx), sb = __ballot(strongPx);
-            if (lane == r) { emLo = (uint32_t)eb; emHi = (uint32_t)(eb >> 32); smLo = (uint32_t)sb; smHi = (uint32_t)(sb >> 32); }
-            // Harris 3x3 NMS: >= towards the upper-left half of the window, > towards the lower-right
             // the lane shifts run with every lane active: a DPP read of a lane that a short-circuited
             // && has switched off returns 0, not that lane's value
             const int c = lane_next(Vb), cRight = lane_next(c);
-            const bool isMax = valid & (c >= max(HO, Vb)) & (c > max(Hc, cRight));
-            const uint64_t cb = __ballot(isMax);
-            if (isMax) {
-                const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(cb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)cb, 0u));
-                const uint32_t bits = negKeys ? (uint32_t)(c ^ ((c >> 31) & 0x7fffffff)) : (uint32_t)c;
-                cand[nc + below] = (uint64_t)(uint16_t)ox | ((uint64_t)(uint16_t)y << 16) | ((uint64_t)bits << 32);
+            const uint64_t valid = (INNER || (y >= 1 && y <= h - 2)) ? outCols : 0ull;
+            const uint64_t cb = valid & mask_of(c >= max(HO, Vb)) & mask_of(c > max(Hc, cRight));
+            if (cb) {
+                if (in_mask(cb)) {
+                    const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(cb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)cb, 0u));
+                    const uint32_t bits = negKeys ? (uint32_t)(c ^ ((c >> 31) & 0x7fffffff)) : (uint32_t)c;
+                    cand[nc + below] = (uint64_t)(uint16_t)ox | ((uint64_t)(uint16_t)y << 16) | ((uint64_t)bits << 32);
+                }
+                nc += (uint32_t)__popcll(cb);
             }
-            nc += (uint32_t)__popcll(cb);
         }
         // the new rows over the oldest ones
         yA = yk; dO = dk; sO = sk;
         xx0 = hxx; xy0 = hxy; yy0 = hyy;
-        MO = Mc; HO = Hc; Vb = Vc;
+        uO = uk; vO = vk; HO = Hc; Vb = Vc; hotB = hot;
     };
 
     uint32_t pf0 = 0, pf1 = 0;
     if (INNER) { pf0 = fetch(0); pf1 = fetch(1); }
-    int y0 = 0, y1 = 0, y2 = 0, y3 = 0, dA = 0, dB = 0, sA = 0, sB = 0;
-    int xx0 = 0, xx1 = 0, xy0 = 0, xy1 = 0, yy0 = 0, yy1 = 0, Ha = 0, Hb = 0;
-    uint32_t Ma = 0, Mb = 0;
+    float y0 = 0, y1 = 0, y2 = 0, y3 = 0, dA = 0, dB = 0, sA = 0, sB = 0;
+    float xx0 = 0, xx1 = 0, xy0 = 0, xy1 = 0, yy0 = 0, yy1 = 0;
+    int ua = 0, ub = 0, va = 0, vb = 0, Ha = 0, Hb = 0;
     static_assert(YH % 4 == 2, "four steps per loop trip, two after it");
     int k = 0;
     for (; k + 4 <= YH; k += 4) {
-        step(k, pf0, pf1, y0, y1, y2, y3, dA, dB, sA, sB, xx0, xx1, xy0, xy1, yy0, yy1, Ma, Mb, Ha, Hb);
-        step(k + 1, pf1, pf0, y1, y2, y3, y0, dB, dA, sB, sA, xx1, xx0, xy1, xy0, yy1, yy0, Mb, Ma, Hb, Ha);
-        step(k + 2, pf0, pf1, y2, y3, y0, y1, dA, dB, sA, sB, xx0, xx1, xy0, xy1, yy0, yy1, Ma, Mb, Ha, Hb);
-        step(k + 3, pf1, pf0, y3, y0, y1, y2, dB, dA, sB, sA, xx1, xx0, xy1, xy0, yy1, yy0, Mb, Ma, Hb, Ha);
+        step(k, pf0, pf1, y0, y1, y2, y3, dA, dB, sA, sB, xx0, xx1, xy0, xy1, yy0, yy1, ua, ub, va, vb, Ha, Hb);
+        step(k + 1, pf1, pf0, y1, y2, y3, y0, dB, dA, sB, sA, xx1, xx0, xy1, xy0, yy1, yy0, ub, ua, vb, va, Hb, Ha);
+        step(k + 2, pf0, pf1, y2, y3, y0, y1, dA, dB, sA, sB, xx0, xx1, xy0, xy1, yy0, yy1, ua, ub, va, vb, Ha, Hb);
+        step(k + 3, pf1, pf0, y3, y0, y1, y2, dB, dA, sB, sA, xx1, xx0, xy1, xy0, yy1, yy0, ub, ua, vb, va, Hb, Ha);
     }
-    step(k, pf0, pf1, y0, y1, y2, y3, dA, dB, sA, sB, xx0, xx1, xy0, xy1, yy0, yy1, Ma, Mb, Ha, Hb);
-    step(k + 1, pf1, pf0, y1, y2, y3, y0, dB, dA, sB, sA, xx1, xx0, xy1, xy0, yy1, yy0, Mb, Ma, Hb, Ha);
+    step(k, pf0, pf1, y0, y1, y2, y3, dA, dB, sA, sB, xx0, xx1, xy0, xy1, yy0, yy1, ua, ub, va, vb, Ha, Hb);
+    step(k + 1, pf1, pf0, y1, y2, y3, y0, dB, dA, sB, sA, xx1, xx0, xy1, xy0, yy1, yy0, ub, ua, vb, va, Hb, Ha);
 
     // ---- Harris candidates: one global atomic per tile, then the buffer copied out
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -386,7 +415,7 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
     //      (-> 0); border-touching components without a strong pixel are undecided.
     static_assert(TH <= 32 && TW <= 63, "row masks: one lane per row in each half-wave");
     const int rr = lane & 31;
-    const uint64_t emine = ((uint64_t)emHi << 32) | emLo, smine = ((uint64_t)smHi << 32) | smLo;
+    const uint64_t emine = ((uint64_t)(uint32_t)emHi << 32) | (uint32_t)emLo, smine = ((uint64_t)(uint32_t)smHi << 32) | (uint32_t)smLo;
     const uint64_t e = __shfl(emine, rr);
     uint64_t seeds;
     if (lane < 32) seeds = __shfl(smine, rr);
@@ -627,6 +656,20 @@ inline GraphParams graph_params(const mvx_vision_params_t &p, const GraphLayout 
     float nf = 255.0f * (float)(1 << 2) * 3;
     P.norm = nf * nf * nf * nf;
     P.normRcp = recip_rn(P.norm);
+    // RN(mc / norm) > thr implies mc > thr * norm; the product is exact in double and rounds down here, and
+    // mc <= RN(gx2 * gy2) when k >= 0.  Negative (or NaN) thr and k: every row takes the full path.
+    P.hotMc = P.hotProd = -INFINITY;
+    if (P.thr >= 0.0f) {
+        const double m = (double)P.thr * (double)P.norm;
+        float f = (float)m;
+        if ((double)f > m) f = std::nextafter(f, 0.0f);
+        P.hotMc = f;
+        if (P.k >= 0.0f) P.hotProd = f;
+    }
+    const auto bits = [](uint32_t t) { const float f = (float)std::max((int)t, 0); int b; memcpy(&b, &f, 4); return b; };
+    P.upperBits = bits(P.upper); P.lowerBits = bits(P.lower);
+    P.upperAll = (int)P.upper < 0 ? ~0ull : 0ull;
+    P.lowerAll = (int)P.lower < 0 ? ~0ull : 0ull;
     P.capacity = p.cornerCapacity;
     P.candCap = L.candCap;
     return P;
