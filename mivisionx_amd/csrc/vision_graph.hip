@@ -155,8 +155,8 @@ constexpr int CAND_MAX = ((TW + 1) / 2) * ((TH + 1) / 2);  // Harris NMS maxima 
 //   candidate buffer.
 // Then the tile's hysteresis on the row masks and the settle pass.
 //
-// Bound by VALU issue, so the instructions of a row are what counts (16 frames of 3840x2160: @BEFORE@ us with
-// about 125 of them, @AFTER@ us with about @INSTR@):
+// Bound by VALU issue, so the instructions of a row are what counts (16 frames of 3840x2160: 690 us with
+// about 125 of them, 505 us with about 68):
 //   * luma, gradients, products and window sums are floats holding integers below 2^24 -- exact, like the
 //     integers the reference computes -- so the Canny sector test, the Harris score and |.| need no
 //     conversions; a 16-bit integer form exists for none of the float rules;
@@ -177,10 +177,11 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
     // inner tiles read a pixel's R, G, B (and the next pixel's R) with one dword load; the window's
     // last column is at most w-2, so the dword stays inside the row
     const __amdgpu_buffer_rsrc_t rgbR = plane_rsrc(F.rgb), l0R = plane_rsrc(F.lvl[0]), scR = plane_rsrc(F.scaled);
-    const __amdgpu_buffer_rsrc_t l1R = plane_rsrc(F.lvl[1]), edR = plane_rsrc(F.edges);
+    const __amdgpu_buffer_rsrc_t l1R = plane_rsrc(F.lvl[1]);
+    const uint32_t rgbStride = F.rgbStride, l0Stride = F.lvlStride[0], l1Stride = F.lvlStride[1], scStride = F.scaledStride;
     const int rgbCol = 3 * (tx0 - HY + lane);
     auto fetch = [&](int k) -> uint32_t {
-        return __builtin_amdgcn_raw_buffer_load_b32(rgbR, rgbCol, (int)((uint32_t)(ty0 - HY + k) * F.rgbStride), 0);
+        return __builtin_amdgcn_raw_buffer_load_b32(rgbR, rgbCol, (int)((uint32_t)(ty0 - HY + k) * rgbStride), 0);
     };
     const int body = P.dw & ~7;
     const int oxp = (w & 1) ? 0 : 1, oyp = (h & 1) ? 0 : 1;
@@ -228,7 +229,7 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
         }
         const float yk = (float)yi;
         if (k >= HY && k < HY + th && lane >= HY && lane < HY + tw)
-            __builtin_amdgcn_raw_buffer_store_b8((uint8_t)yi, l0R, tx0 - HY + lane, (int)((uint32_t)(ty0 + k - HY) * F.lvlStride[0]), 0);
+            __builtin_amdgcn_raw_buffer_store_b8((uint8_t)yi, l0R, tx0 - HY + lane, (int)((uint32_t)(ty0 + k - HY) * l0Stride), 0);
         // binomial column sums through one-lane shifts: t = Y[l]+Y[l+1], s = Y[l]+2Y[l+1]+Y[l+2], d = Y[l+2]-Y[l]
         const float tk = yk + lane_next_f(yk);
         const float sk = tk + lane_next_f(tk), dk = lane_next_f(tk) - tk;
@@ -243,7 +244,7 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
             int v = (int)__builtin_amdgcn_lerp((uint32_t)aPrev, (uint32_t)ak, 1u);
             if (!allBody) v = scBody ? v : ((int)(tPrev + tk) + 2) >> 2;
             if (Yo < P.dh && scOut)
-                __builtin_amdgcn_raw_buffer_store_b8((uint8_t)v, scR, tx0 / 2 + (sp >> 1), (int)((uint32_t)Yo * F.scaledStride), 0);
+                __builtin_amdgcn_raw_buffer_store_b8((uint8_t)v, scR, tx0 / 2 + (sp >> 1), (int)((uint32_t)Yo * scStride), 0);
         }
         aPrev = ak;
         tPrev = tk;
@@ -260,7 +261,7 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
                 acc = acc + lane_next_f(acc);
                 if (l1Out)
                     __builtin_amdgcn_raw_buffer_store_b8((uint8_t)((uint32_t)acc >> 8), l1R, tx0 / 2 + (lp1 >> 1),
-                                                         (int)((uint32_t)Yo * F.lvlStride[1]), 0);
+                                                         (int)((uint32_t)Yo * l1Stride), 0);
             }
         }
 
@@ -396,6 +397,9 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
     step(k, pf0, pf1, y0, y1, y2, y3, dA, dB, sA, sB, xx0, xx1, xy0, xy1, yy0, yy1, ua, ub, va, vb, Ha, Hb);
     step(k + 1, pf1, pf0, y1, y2, y3, y0, dB, dA, sB, sA, xx1, xx0, xy1, xy0, yy1, yy0, ub, ua, vb, va, Hb, Ha);
 
+    const __amdgpu_buffer_rsrc_t edR = plane_rsrc(F.edges);
+    const uint32_t edStride = F.edgesStride;
+
     // ---- Harris candidates: one global atomic per tile, then the buffer copied out
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -429,9 +433,9 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
     for (int r = 0; r < th; r++) {
         const uint64_t R = readlane64(rm, r), B = readlane64(bmAll, r);
         const int y = ty0 + r;
-        if (lane < TW && (INNER || (y >= 1 && y <= h - 2 && ox >= 1 && ox <= w - 2)))
-            __builtin_amdgcn_raw_buffer_store_b8(((R >> lane) & 1ull) ? 255 : (((B >> lane) & 1ull) ? 127 : 0), edR, ox,
-                                                 (int)((uint32_t)y * F.edgesStride), 0);
+        const int v = in_mask(R) ? 255 : in_mask(B) ? 127 : 0;
+        if (in_mask(outCols) && (INNER || (y >= 1 && y <= h - 2)))
+            __builtin_amdgcn_raw_buffer_store_b8((uint8_t)v, edR, ox, (int)((uint32_t)y * edStride), 0);
     }
 
     //  (c) the undecided components, one at a time: the first set bit in row-major order is the
@@ -443,8 +447,8 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
     int32_t topv = -1, botv = -1, leftv = -1, rightv = -1;
     {
         const uint64_t R0 = readlane64(rm, 0), Rb = readlane64(rm, th - 1);
-        if (lane < tw && ((R0 >> lane) & 1ull)) topv = 0;
-        if (lane < tw && ((Rb >> lane) & 1ull)) botv = 0;
+        topv = in_mask(R0) ? 0 : topv;     // the masks hold no column past the tile's width
+        botv = in_mask(Rb) ? 0 : botv;
         if (lane < th && (rm & 1ull)) leftv = 0;
         if (lane < th && ((rm >> (tw - 1)) & 1ull)) rightv = 0;
     }
@@ -460,8 +464,8 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
         const uint64_t c = grow_rows(lane == r0 ? (1ull << c0) : 0ull, bm, lane);
         if (lane == 0) gmem(F.parent)[gid] = gid;
         const uint64_t C0 = readlane64(c, 0), Cb = readlane64(c, th - 1);
-        if (lane < tw && ((C0 >> lane) & 1ull)) topv = (int32_t)gid;
-        if (lane < tw && ((Cb >> lane) & 1ull)) botv = (int32_t)gid;
+        topv = in_mask(C0) ? (int32_t)gid : topv;
+        botv = in_mask(Cb) ? (int32_t)gid : botv;
         if (lane < th && (c & 1ull)) leftv = (int32_t)gid;
         if (lane < th && ((c >> (tw - 1)) & 1ull)) rightv = (int32_t)gid;
         // list the component's pixels for k_resolve: p | k << 16
@@ -470,7 +474,7 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
             const int r = __builtin_ctzll(crow);
             crow &= crow - 1;
             const uint64_t m = readlane64(c, r);
-            if ((m >> lane) & 1ull) {
+            if (in_mask(m)) {
                 const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
                 ulist[nU + below] = (uint32_t)(r * TP + lane) | (nComp << 16);
             }
@@ -489,13 +493,13 @@ __global__ void __launch_bounds__(64 * FTW)
 k_front(const FrameDesc *__restrict__ frames, GraphParams P)
 {
     __shared__ uint64_t candLds[FTW][CAND_MAX];
-    const FrameDesc F = frames[blockIdx.z];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int tX = (int)blockIdx.x * FTW + wave, tY = (int)blockIdx.y;
     if (tX >= P.tilesX) return;
     const int tile = tY * P.tilesX + tX;
     const int tx0 = tX * TW, ty0 = tY * TH;
     const bool inner = tx0 >= 4 && tx0 + TW + 4 <= P.w && ty0 >= 4 && ty0 + TH + 4 <= P.h;
+    const FrameDesc &F = frames[blockIdx.z];   // fields are read where they are used: the stream needs the scalar registers
     if (inner) front_tile<true>(candLds[wave], F, P, tx0, ty0, tile);
     else front_tile<false>(candLds[wave], F, P, tx0, ty0, tile);
 }
