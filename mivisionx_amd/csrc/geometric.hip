@@ -335,14 +335,13 @@ k_scale_area2(uint32_t dw8, uint32_t dh, uint8_t *__restrict__ dst, uint32_t dst
 }
 
 // ------------------------------------------------------------------ ScaleGaussianHalf 5x5 ------
-// one thread: 8 outputs x PYR_ROWS rows (pyramid.hpp)
+// one wave: one output row of 62 chunks of 8 columns (pyramid.hpp)
 __global__ void __launch_bounds__(256)
 k_gaussian_half_5x5(uint32_t dw, uint32_t dh, uint8_t *__restrict__ dst, uint32_t dstStride, uint32_t sw, uint32_t sh,
                     const uint8_t *__restrict__ src, uint32_t srcStride)
 {
-    const uint32_t x0 = (blockIdx.x * 64 + threadIdx.x) * 8;
-    const int y0 = 1 + (int)(blockIdx.y * 4 + threadIdx.y) * PYR_ROWS;
-    half_strip(dw, dh, dst, dstStride, sw, sh, src, srcStride, x0, y0);
+    for (int y = 1 + (int)(blockIdx.y * 4) + __builtin_amdgcn_readfirstlane((int)threadIdx.y); y <= (int)dh - 2; y += (int)gridDim.y * 4)
+        half_row(dw, dst, dstStride, sw, sh, src, srcStride, blockIdx.x * PYR_CHUNKS, y);
 }
 
 // ------------------------------------------------------------------ ScaleGaussianHalf 3x3 ------
@@ -654,10 +653,7 @@ extern "C" int mvx_ScaleGaussianHalf_U8_U8_5x5(mvx_stream_t stream, uint32_t dw,
     if (sw < 5 || sh < 5 || dw < 3 || dh < 3) return -15;
     if (!plane_ok_g(dst, dw, dstStride, 1) || !plane_ok_g(src, sw, srcStride, 1) || (dstStride & 7u))
         return MVX_ERROR_INVALID_PARAMETERS;
-    const uint32_t chunks = (dw + 7) / 8;
-    const uint32_t strips = (dh - 2 + PYR_ROWS - 1) / PYR_ROWS;
-    dim3 grid((chunks + 63) / 64, (strips + 3) / 4);
-    hipLaunchKernelGGL(k_gaussian_half_5x5, grid, dim3(64, 4), 0, stream_of(stream), dw, dh, dst, dstStride, sw, sh,
+    hipLaunchKernelGGL(k_gaussian_half_5x5, half_grid(dw, dh, 1), dim3(64, 4), 0, stream_of(stream), dw, dh, dst, dstStride, sw, sh,
                        src, srcStride);
     MVX_LAUNCH_CHECK();
     return MVX_SUCCESS;

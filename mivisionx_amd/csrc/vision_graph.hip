@@ -580,10 +580,10 @@ __global__ void __launch_bounds__(256)
 k_half_batched(const FrameDesc *__restrict__ frames, GraphParams P, int lvl)
 {
     const FrameDesc &F = frames[blockIdx.z];
-    const uint32_t x0 = (blockIdx.x * 64 + threadIdx.x) * 8;
-    const int y0 = 1 + (int)(blockIdx.y * 4 + threadIdx.y) * PYR_ROWS;
-    half_strip((uint32_t)P.lvlW[lvl], (uint32_t)P.lvlH[lvl], F.lvl[lvl], F.lvlStride[lvl], (uint32_t)P.lvlW[lvl - 1],
-               (uint32_t)P.lvlH[lvl - 1], F.lvl[lvl - 1], F.lvlStride[lvl - 1], x0, y0);
+    const int y = 1 + (int)(blockIdx.y * 4) + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    if (y <= P.lvlH[lvl] - 2)
+        half_row((uint32_t)P.lvlW[lvl], F.lvl[lvl], F.lvlStride[lvl], (uint32_t)P.lvlW[lvl - 1], (uint32_t)P.lvlH[lvl - 1],
+                 F.lvl[lvl - 1], F.lvlStride[lvl - 1], blockIdx.x * PYR_CHUNKS, y);
 }
 
 // Harris sort and pick, one workgroup per frame; clears the candidate count for the next batch
@@ -763,12 +763,8 @@ static void launch_stage(hipStream_t s, const GraphParams &P, const FrameDesc *D
                            s, D, P);
         break;
     case 3:
-        for (int l = 2; l < P.levels; l++) {
-            const uint32_t chunks = ((uint32_t)P.lvlW[l] + 7) / 8;
-            const uint32_t strips = ((uint32_t)P.lvlH[l] - 2 + PYR_ROWS - 1) / PYR_ROWS;
-            hipLaunchKernelGGL(k_half_batched, dim3((chunks + 63) / 64, (strips + 3) / 4, nframes), dim3(64, 4), 0, s, D,
-                               P, l);
-        }
+        for (int l = 2; l < P.levels; l++)
+            hipLaunchKernelGGL(k_half_batched, half_grid((uint32_t)P.lvlW[l], (uint32_t)P.lvlH[l], nframes), dim3(64, 4), 0, s, D, P, l);
         break;
     case 4:
         hipLaunchKernelGGL(k_pick_batched, dim3(nframes), dim3(PICK_THREADS), 0, s, D, P);

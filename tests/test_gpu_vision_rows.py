@@ -1,0 +1,76 @@
+"""The fused tile pass where its rows change path -- Harris rows with and without a score, scores at and
+around zero, negative thresholds and sensitivities, Canny thresholds from 0 to above every magnitude, the
+scaled image's scalar tail, tiles cut at every edge -- and the half-size pyramid step at the edges of its
+62-chunk waves.  The per-node kernels are the reference for the graph (each has its own oracle tests), the
+oracle for the pyramid step; every byte has to be the same."""
+import numpy as np
+import pytest
+import torch
+
+from mivisionx_amd import synth
+from mivisionx_amd.device import Plane, call
+from mivisionx_amd.pipelines import FusedVisionGraph, VisionGraph4K
+from util import assert_same
+
+pytestmark = pytest.mark.gpu
+
+
+def _rgb(kind, w, h):
+    if kind == "noise":       # scores everywhere
+        return synth.u32(11, 3, w * h * 3).astype(np.uint8).reshape(h, w, 3)
+    if kind == "flat":        # no gradient at all
+        return np.full((h, w, 3), 77, np.uint8)
+    img = np.zeros((h, w, 3), np.uint8)      # sparse corners: most rows have no score
+    img[h // 3:h // 3 + 9, w // 4:w // 2] = 200
+    img[2 * h // 3:, 5:9] = (10, 250, 60)
+    return img
+
+
+@pytest.mark.parametrize("k,thr", [(0.04, 0.0005), (0.04, 0.0), (0.04, 1e-9), (0.04, 1e30), (0.04, -1.0), (-0.04, 0.0005), (0.0, 0.0)])
+@pytest.mark.parametrize("kind", ["noise", "sparse", "flat"])
+def test_harris_rows(gpu, kind, k, thr):
+    print(f"fused graph: {kind}, sensitivity {k}, threshold {thr}", flush=True)
+    _compare(_rgb(kind, 244, 106), 80, 100, k, thr)
+
+
+@pytest.mark.parametrize("lower,upper", [(0, 0), (1, 2), (80, 100), (100, 80), (2040, 2041), (4000, 5000)])
+@pytest.mark.parametrize("w,h", [(16, 16), (60, 34), (116, 64), (128, 66), (180, 98)])
+def test_canny_thresholds_and_sizes(gpu, w, h, lower, upper):
+    print(f"fused graph: {w}x{h}, Canny {lower}/{upper}", flush=True)
+    _compare(_rgb("noise", w, h), lower, upper, 0.04, 0.0005)
+
+
+def _compare(rgb, lower, upper, k, thr):
+    h, w = rgb.shape[:2]
+    levels = 3 if min(w, h) >= 20 else 1
+    args = dict(levels=levels, lower=lower, upper=upper, k=k, thr=thr, dist=5.0, capacity=4096)
+    fused = FusedVisionGraph(w, h, w // 2, h // 2, frames=2, **args)
+    for f in fused.frames:
+        f.rgb.upload(rgb)
+    nodes = VisionGraph4K(w, h, w // 2, h // 2, **args)
+    nodes.rgb.upload(rgb)
+    for _ in range(2):
+        fused.run()
+    nodes.run()
+    torch.cuda.synchronize()
+    want = nodes.results()
+    for i, f in enumerate(fused.frames):
+        got = f.results()
+        assert_same(got["edges"], want["edges"], f"frame {i} edges")
+        assert_same(got["scaled"], want["scaled"], f"frame {i} scaled")
+        for l in range(levels):
+            assert_same(got["pyramid"][l], want["pyramid"][l], f"frame {i} level {l}")
+        assert got["count"] == want["count"]
+        assert got["corners"].tobytes() == want["corners"].tobytes(), f"frame {i} corners"
+
+
+@pytest.mark.parametrize("w,h", [(5, 5), (6, 5), (15, 6), (17, 7), (990, 9), (991, 11), (992, 12), (993, 13), (994, 7), (1008, 6), (1985, 10)])
+def test_half_step_wave_edges(gpu, orc, w, h):
+    print(f"half step {w}x{h}", flush=True)
+    src = synth.uniform_u8(w, h, 3)
+    dw, dh = (w + 1) // 2, (h + 1) // 2
+    s, d = Plane.from_array(src), Plane(dw, dh)
+    call("ScaleGaussianHalf_U8_U8_5x5", dw, dh, d, d.stride, w, h, s, s.stride)
+    torch.cuda.synchronize()
+    assert_same(d.download(), orc.gaussian_half(src, dw, dh), f"half {w}x{h}")
+    assert not d.t[:, dw:].any(), "padding bytes stay zero"
