@@ -15,12 +15,13 @@ MVX_DEV uint32_t gfind(gptr_t<const uint32_t> par, uint32_t p)
     return p;
 }
 
+// The larger id hangs under the smaller at once, without finding the roots first: when it was a root (most
+// ids are) that is the whole union, one trip to memory instead of three.  When it was not, its old parent
+// still has to join b's set, and the loop goes on with those two; ids only fall, so it ends.  An id may so
+// hang under one that is no root: chains are as correct as stars for gfind.
 MVX_DEV void gunion(gptr_t<uint32_t> par, uint32_t a, uint32_t b)
 {
-    while (true) {
-        a = gfind(par, a);
-        b = gfind(par, b);
-        if (a == b) return;
+    while (a != b) {
         if (a < b) { uint32_t t = a; a = b; b = t; }
         const uint32_t old = __hip_atomic_fetch_min(par + a, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (old == a) return;

@@ -520,30 +520,19 @@ k_border(const FrameDesc *__restrict__ frames, GraphParams P)
     gptr_t<const int32_t> tables = gmem((const int32_t *)F.border);
     gptr_t<const int32_t> bt = tables + (long)tile * 2 * (TW + TH);
     gptr_t<uint32_t> par = gmem(F.parent);
-    // right neighbour: my right column (rows 0..th-1) against its left column, |dr| <= 1
-    if (tX + 1 < P.tilesX) {
-        gptr_t<const int32_t> nb = tables + (long)(tile + 1) * 2 * (TW + TH);
-        border_unions(par, lane < th ? bt[2 * TW + TH + lane] : -1, lane < th ? nb[2 * TW + lane] : -1, lane);
-    }
-    // lower neighbour: my bottom row against its top row, |dc| <= 1 (the tile below has the same width)
-    if (tYi + 1 < P.tilesY) {
-        gptr_t<const int32_t> nb = tables + (long)(tile + P.tilesX) * 2 * (TW + TH);
-        border_unions(par, lane < tw ? bt[TW + lane] : -1, lane < tw ? nb[lane] : -1, lane);
-        if (lane == 0) {
-            // diagonals: bottom-right corner <-> lower-right tile's top-left,
-            // bottom-left corner <-> lower-left tile's top-right (a full-width tile)
-            if (tX + 1 < P.tilesX) {
-                const int32_t a = bt[TW + tw - 1];
-                gptr_t<const int32_t> nd = tables + (long)(tile + P.tilesX + 1) * 2 * (TW + TH);
-                if (a >= 0 && nd[0] >= 0 && nd[0] != a) gunion(par, (uint32_t)a, (uint32_t)nd[0]);
-            }
-            if (tX > 0) {
-                const int32_t a = bt[TW + 0];
-                gptr_t<const int32_t> nd = tables + (long)(tile + P.tilesX - 1) * 2 * (TW + TH);
-                if (a >= 0 && nd[TW - 1] >= 0 && nd[TW - 1] != a) gunion(par, (uint32_t)a, (uint32_t)nd[TW - 1]);
-            }
-        }
-    }
+    // all table reads first, so that the wave waits for memory once: my right column (rows 0..th-1) and its
+    // right neighbour's left column, |dr| <= 1; my bottom row and the top row below it (the tile below has the
+    // same width), |dc| <= 1; the corners of the lower right and lower left tiles (the latter of full width)
+    const bool right = tX + 1 < P.tilesX, down = tYi + 1 < P.tilesY;
+    gptr_t<const int32_t> nr = tables + (long)(tile + 1) * 2 * (TW + TH), nd = tables + (long)(tile + P.tilesX) * 2 * (TW + TH);
+    const int32_t ra = right && lane < th ? bt[2 * TW + TH + lane] : -1, rb = right && lane < th ? nr[2 * TW + lane] : -1;
+    const int32_t da = down && lane < tw ? bt[TW + lane] : -1, db = down && lane < tw ? nd[lane] : -1;
+    const int32_t cr = down && right ? (nd + 2 * (TW + TH))[0] : -1, cl = down && tX > 0 ? (nd - 2 * (TW + TH))[TW - 1] : -1;
+    const int32_t ar = __builtin_amdgcn_readlane(da, tw - 1), al = __builtin_amdgcn_readlane(da, 0);
+    border_unions(par, ra, rb, lane);
+    border_unions(par, da, db, lane);
+    if (lane == 0 && ar >= 0 && cr >= 0) gunion(par, (uint32_t)ar, (uint32_t)cr);
+    if (lane == 0 && al >= 0 && cl >= 0) gunion(par, (uint32_t)al, (uint32_t)cl);
 }
 
 // the undecided pixels k_front listed take the state of their component's global root (strong iff
@@ -556,21 +545,46 @@ k_resolve(const FrameDesc *__restrict__ frames, GraphParams P)
     const int w0 = ((int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * RES_TILES;
     const int tiles = P.tilesX * P.tilesY;
     if (w0 >= tiles) return;
-    // most tiles list nothing: the wave reads its tiles' counts at once and visits only the busy ones
+    // the wave's tiles side by side: their counts, the first 64 entries of their lists (whatever the list
+    // holds past its count is not used) and then the roots of all of them, so that a wave waits for memory
+    // about three times however many of its tiles list pixels
     const uint32_t cnt = (lane < RES_TILES && w0 + lane < tiles) ? gmem(F.ucount)[w0 + lane] : 0u;
-    uint64_t busy = __ballot(cnt != 0u);
-    while (busy) {
-        const int j = __builtin_ctzll(busy);
-        busy &= busy - 1;
-        const int tile = w0 + j;
-        const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)cnt, j);
-        const int tx0 = (tile % P.tilesX) * TW, ty0 = (tile / P.tilesX) * TH;
-        gptr_t<const uint32_t> list = gmem((const uint32_t *)F.ulist) + (size_t)tile * TS;
-        for (uint32_t i = (uint32_t)lane; i < n; i += 64) {
-            const uint32_t e = list[i];
-            const uint32_t p = e & 0xffffu, comp = e >> 16;
-            const uint32_t g = gfind(gmem(F.parent), 1u + (uint32_t)tile * TNB + comp);
-            gmem(F.edges)[(long)(ty0 + (int)(p / TP)) * F.edgesStride + tx0 + (int)(p % TP)] = (g == 0) ? 255 : 0;
+    uint32_t e[RES_TILES];
+#pragma unroll
+    for (int j = 0; j < RES_TILES; j++) e[j] = w0 + j < tiles ? gmem((const uint32_t *)F.ulist)[(size_t)(w0 + j) * TS + lane] : 0u;
+    if (!__any(cnt != 0u)) return;
+    gptr_t<const uint32_t> par = gmem((const uint32_t *)F.parent);
+    gptr_t<uint8_t> edges = gmem(F.edges);
+    const auto put = [&](int tile, uint32_t entry, uint32_t root) {
+        const uint32_t p = entry & 0xffffu;
+        edges[(long)((tile / P.tilesX) * TH + (int)(p / TP)) * F.edgesStride + (tile % P.tilesX) * TW + (int)(p % TP)] = (root == 0) ? 255 : 0;
+    };
+    uint32_t g[RES_TILES], up[RES_TILES];
+    bool has[RES_TILES];
+#pragma unroll
+    for (int j = 0; j < RES_TILES; j++) {
+        has[j] = lane < __builtin_amdgcn_readlane((int)cnt, j);
+        g[j] = has[j] ? 1u + (uint32_t)(w0 + j) * TNB + (e[j] >> 16) : 0u;
+        up[j] = has[j] ? par[g[j]] : 0u;
+    }
+    while (true) {
+        bool more = false;
+#pragma unroll
+        for (int j = 0; j < RES_TILES; j++) {
+            if (up[j] != g[j]) {
+                g[j] = up[j];
+                up[j] = par[g[j]];
+                more = true;
+            }
+        }
+        if (!__any(more)) break;
+    }
+#pragma unroll
+    for (int j = 0; j < RES_TILES; j++) {
+        if (has[j]) put(w0 + j, e[j], g[j]);
+        for (uint32_t i = 64u + (uint32_t)lane; i < (uint32_t)__builtin_amdgcn_readlane((int)cnt, j); i += 64) {
+            const uint32_t entry = gmem((const uint32_t *)F.ulist)[(size_t)(w0 + j) * TS + i];
+            put(w0 + j, entry, gfind(par, 1u + (uint32_t)(w0 + j) * TNB + (entry >> 16)));
         }
     }
 }
@@ -877,8 +891,8 @@ extern "C" int mvx_VisionGraph_lane_destroy(mvx_vision_lane_t *lane)
 
 // The frames go through in chunks of framesPerChunk: the fused tile pass of each chunk on the caller's
 // stream, then -- once it has finished, while the caller's stream goes on with the next chunk's tile
-// pass -- that chunk's hysteresis stages on one lane stream (the last chunk's on the caller's stream)
-// and its pyramid levels and Harris pick on the other.  At the end the caller's stream waits for both
+// pass -- that chunk's hysteresis stages on one lane stream and its pyramid levels and Harris pick on the
+// other (the last chunk's hysteresis on the caller's stream and its pick on the first).  At the end the caller's stream waits for both
 // lane streams, so the call orders like a single-stream sequence.  Fork and join are event waits, which a hipGraph capture of the caller's
 // stream records as dependencies.  Once forked, the joins are recorded and waited for on every path,
 // errors included, so a captured caller stream is never left forked.
@@ -910,11 +924,12 @@ extern "C" int mvx_VisionGraph_run_pipelined(mvx_stream_t stream, mvx_vision_lan
             break;
         }
         forked = true;
-        launch_stage(lane->stream, P, D + f0, n, 3);
-        launch_stage(lane->stream, P, D + f0, n, 4);
         // the last chunk's hysteresis follows its tile pass on the caller's stream: no stream hop on
-        // the critical path
-        hipStream_t hs = f0 + n < nframes ? lane->hyst : main;
+        // the critical path; its Harris pick then has the other lane stream to itself
+        const bool last = f0 + n >= nframes;
+        hipStream_t hs = last ? main : lane->hyst;
+        launch_stage(last ? lane->hyst : lane->stream, P, D + f0, n, 4);
+        launch_stage(lane->stream, P, D + f0, n, 3);
         launch_stage(hs, P, D + f0, n, 1);
         launch_stage(hs, P, D + f0, n, 2);
         if (hipGetLastError() != hipSuccess) rc = MVX_ERROR_LAUNCH;
