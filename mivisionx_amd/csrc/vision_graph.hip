@@ -180,8 +180,31 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
     const __amdgpu_buffer_rsrc_t l1R = plane_rsrc(F.lvl[1]);
     const uint32_t rgbStride = F.rgbStride, l0Stride = F.lvlStride[0], l1Stride = F.lvlStride[1], scStride = F.scaledStride;
     const int rgbCol = 3 * (tx0 - HY + lane);
+    // other tiles read the virtual luma plane at linear addresses: a column before 0 or past the stride lies in
+    // the row above or below (edgeRow), one of the padding or outside the plane is 0.  The same dword loads,
+    // two rows ahead, from a row clamped into the image; the last column's dword starts one byte early.
+    // Images narrower than a tile's window may wrap more than once: they go through yflat.
+    const bool wide = w >= 64;
+    int edgeRow = 0, edgeCol = tx0 - HY + lane;
+    if (edgeCol < 0) { edgeRow = -1; edgeCol += P.yStride; }
+    else if (edgeCol >= P.yStride) { edgeRow = 1; edgeCol -= P.yStride; }
+    const bool edgeColOk = edgeCol < w;
+    const uint32_t edgeOff = edgeColOk ? 3u * (uint32_t)edgeCol - (edgeCol == w - 1 ? 1u : 0u) : 0u, edgeShift = edgeCol == w - 1 ? 8u : 0u;
     auto fetch = [&](int k) -> uint32_t {
-        return __builtin_amdgcn_raw_buffer_load_b32(rgbR, rgbCol, (int)((uint32_t)(ty0 - HY + k) * rgbStride), 0);
+        if (INNER) return __builtin_amdgcn_raw_buffer_load_b32(rgbR, rgbCol, (int)((uint32_t)(ty0 - HY + k) * rgbStride), 0);
+        const uint32_t r = (uint32_t)min(max(ty0 - HY + k + edgeRow, 0), h - 1);
+        return __builtin_amdgcn_raw_buffer_load_b32(rgbR, (int)(__umul24(r, rgbStride) + edgeOff), 0, 0);
+    };
+    // luma row k from its fetched dwords
+    auto luma_of = [&](int k, uint32_t p) -> int {
+        if (!INNER) p >>= edgeShift;
+        float f = (float)(p & 0xffu) * 0.2126f;
+        f = f + (float)((p >> 8) & 0xffu) * 0.7152f;
+        f = f + (float)((p >> 16) & 0xffu) * 0.0722f;
+        const int v = (int)f;
+        if (INNER) return v;
+        const int r = ty0 - HY + k + edgeRow;
+        return edgeColOk && r >= 0 && r < h ? v : 0;
     };
     const int body = P.dw & ~7;
     const int oxp = (w & 1) ? 0 : 1, oyp = (h & 1) ? 0 : 1;
@@ -217,13 +240,10 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
         // ---- luma row k (ColorConvert Y of the RGB pixel, or the virtual plane's linear-address
         //      value); the float sum lies in [0, 256), so the truncation needs no clamp
         int yi;
-        if (INNER) {
+        if (INNER || wide) {
             const uint32_t cur = pO;
             if (k + 2 < YH) pO = fetch(k + 2);
-            float f = (float)(cur & 0xffu) * 0.2126f;
-            f = f + (float)((cur >> 8) & 0xffu) * 0.7152f;
-            f = f + (float)((cur >> 16) & 0xffu) * 0.0722f;
-            yi = (int)f;
+            yi = luma_of(k, cur);
         } else {
             yi = (int)yflat(F, P, ty0 - HY + k, tx0 - HY + lane);
         }
@@ -317,11 +337,20 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
                 const int a3 = __builtin_amdgcn_readlane((int)yC, 3), a4 = __builtin_amdgcn_readlane((int)yC, 4);
                 const int b4 = __builtin_amdgcn_readlane((int)yD, 4);
                 const int c3 = __builtin_amdgcn_readlane(yi, 3), c4 = __builtin_amdgcn_readlane(yi, 4);
+                int t1_m1 = 0;
+                if (w % 16 == 0) {
+                    // column w-1 of a row is lane 2 (x = -1) of the row below it: rows k-1, k, and k+1, whose pixels
+                    // are in pN
+                    if (wide) {
+                        t1_m1 = __builtin_amdgcn_readlane((int)yD, 2) + 2 * __builtin_amdgcn_readlane(yi, 2) +
+                                __builtin_amdgcn_readlane(luma_of(k + 1, pN), 2);
+                    } else {
+                        t1_m1 = (int)yflat(F, P, yg - 1, w - 1) + (int)yflat(F, P, yg + 1, w - 1) + 2 * (int)yflat(F, P, yg, w - 1);
+                    }
+                }
                 if (xg == 0) {
                     const int t0_1 = a4 + c4 + 2 * b4;
                     const int t1_0 = c3 - a3, t1_1 = c4 - a4;
-                    const int t1_m1 = (w % 16 == 0) ? ((int)yflat(F, P, yg - 1, w - 1) + (int)yflat(F, P, yg + 1, w - 1) +
-                                                       2 * (int)yflat(F, P, yg, w - 1)) : 0;
                     mag = __float_as_int((float)(abs(t0_1) + abs(t1_m1 + 2 * t1_0 + t1_1)));
                 }
             }
@@ -382,7 +411,7 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
     };
 
     uint32_t pf0 = 0, pf1 = 0;
-    if (INNER) { pf0 = fetch(0); pf1 = fetch(1); }
+    if (INNER || wide) { pf0 = fetch(0); pf1 = fetch(1); }
     float y0 = 0, y1 = 0, y2 = 0, y3 = 0, dA = 0, dB = 0, sA = 0, sB = 0;
     float xx0 = 0, xx1 = 0, xy0 = 0, xy1 = 0, yy0 = 0, yy1 = 0;
     int ua = 0, ub = 0, va = 0, vb = 0, Ha = 0, Hb = 0;
