@@ -531,7 +531,9 @@ typedef struct mvx_image_level {
  * iterations; the reference loops without bound).  windowDimension 3..15.
  * The workspace (mvx_OpticalFlowPyrLK_workspace_size(level-0 width, height, capacity) bytes, device,
  * 16-byte aligned) must be zero-filled before the first call and then kept: like the reference
- * node's local data it carries state from call to call that the reference's results depend on. */
+ * node's local data it carries state from call to call that the reference's results depend on.  Its
+ * tail holds the derivative images of the levels above level 0, which lets one launch take the points
+ * through all levels; where they do not fit (levels larger than halves) there is a launch per level. */
 size_t mvx_OpticalFlowPyrLK_workspace_size(uint32_t width0, uint32_t height0, uint32_t capacity);
 int mvx_OpticalFlowPyrLK_XY_XY(mvx_stream_t stream, void *pNewKeypoints, uint32_t *pNewCount,
                                const mvx_image_level_t *oldPyramid, const mvx_image_level_t *newPyramid, uint32_t levels,

@@ -1,0 +1,58 @@
+"""All pyramid levels in one tracking launch against one launch per level (which a workspace without room
+for a derivative image per level still takes): the same keypoints, call after call, at level widths with
+and without whole 8-column chunks -- the cells no level writes keep the last call's values in both -- and
+windows on both sides of the small-window kernel.  The per-level form is the oracle-tested one."""
+import pytest
+import torch
+
+from mivisionx_amd import synth
+from mivisionx_amd.device import Plane, call
+from mivisionx_amd.pipelines import PyrLKTracker, pyramid_dims
+
+pytestmark = pytest.mark.gpu
+
+
+def _pyramid(img, levels):
+    h, w = img.shape
+    dims = pyramid_dims(w, h, levels)
+    out = [Plane.from_array(img)]
+    for (a, b), (pa, pb) in zip(dims[1:], dims[:-1]):
+        p = Plane(a, b)
+        call("ScaleGaussianHalf_U8_U8_5x5", a, b, p, p.stride, pa, pb, out[-1], out[-1].stride)
+        out.append(p)
+    return out
+
+
+def _align256(n):
+    return (n + 255) // 256 * 256
+
+
+@pytest.mark.parametrize("w,h,levels", [(96, 64, 2), (157, 101, 3), (203, 90, 3), (334, 250, 4), (640, 480, 4)])
+@pytest.mark.parametrize("win", [3, 5, 8, 9, 11, 12, 15])
+def test_together_equals_level_at_a_time(gpu, w, h, levels, win):
+    print(f"LK {w}x{h}, {levels} levels, window {win}", flush=True)
+    n = 200
+    trackers = []
+    frames = [synth.scene_u8(w, h, s) for s in (1, 2)]
+    frames.append(synth.shift_image(frames[1], 1.7, -2.3))
+    pyrs = [_pyramid(f, levels) for f in frames]
+    kp = synth.lk_keypoints(w, h, n, 5, margin=4)
+    kp["tracking_status"][::17] = 0
+    for together in (True, False):
+        results = []
+        t = PyrLKTracker(pyrs[0], pyrs[1], n)
+        if not together:     # row scratch + one derivative image + positions
+            t.ws_size = _align256(_align256(_align256((2 * w + 64) * 2) + w * h * 4) + 8 * n)
+        t.set_points(kp)
+        for old, new in ((0, 1), (1, 2), (2, 1), (1, 2)):     # successive calls on one workspace
+            for lv in range(levels):
+                t.lo[lv].ptr, t.ln[lv].ptr = pyrs[old][lv].t.data_ptr(), pyrs[new][lv].t.data_ptr()
+            t.run(0xF002, 0.01, 20, False, win)
+            torch.cuda.synchronize()
+            results.append(t.result().tobytes())
+        t.run(0xF002, 0.01, 20, True, win)                    # with initial estimates
+        torch.cuda.synchronize()
+        results.append(t.result().tobytes())
+        trackers.append(results)
+    for i, (a, b) in enumerate(zip(*trackers)):
+        assert a == b, f"call {i}"
