@@ -97,4 +97,38 @@ MVX_DEV uint32_t phase_px(int32_t gx, int32_t gy)
     return ((uint32_t)t + (v - t >= 0.5f ? 1u : 0u)) & 0xffu;
 }
 
+// The same rules for gradients of a 3x3 Sobel, given as floats: |fx|, |fy| <= 1020, integers, never -0.
+// Checked for every such pair on the GPU by the test suite.
+
+// sqrt(gx^2 + gy^2) rounded to an integer -- mag_body's and mag_tail's value alike, since the root is never
+// within half an ulp of k + 1/2 -- as a float in [2^23, 2^23 + 1443]: its low 16 bits are the integer.
+// sqrt(s) rounds up from s = k^2 + k + 1 on; the root of s - 1/4 is k + 1/2 at the middle of that gap and at
+// least 1.4 ulps from it at every integer s, more than the hardware root's 1-ulp error (s - 1/4 is exact).
+MVX_DEV uint32_t mag_sobel(float fx, float fy)
+{
+    const float s = fmaxf(fmaf(fx, fx, fmaf(fy, fy, -0.25f)), 0.f);
+    return __float_as_uint(__builtin_amdgcn_sqrtf(s) + 8388608.f);
+}
+
+// floor(sqrt(gx^2 + gy^2)), mag_trunc's value: the root of s + 1/2 is 1.4 ulps and more from every integer
+MVX_DEV uint32_t mag_sobel_trunc(float fx, float fy)
+{
+    return (uint32_t)__builtin_amdgcn_sqrtf(fmaf(fx, fx, fmaf(fy, fy, 0.5f)));
+}
+
+// phase_px; the low 8 bits are the phase (256 stands for 0).  floor(v + 1/2) as one float add and a
+// truncation: v is never the one float below 1/2 whose sum rounds up to 1.
+MVX_DEV uint32_t phase_sobel(float fx, float fy)
+{
+    const float eps = (float)2.2204460492503131e-16;   // (float)DBL_EPSILON, which only matters for (0, 0)
+    const float ax = fabsf(fx), ay = fabsf(fy);
+    const float c = div_small_rn(fminf(ax, ay), fmaxf(fmaxf(ax, ay), eps));
+    const float c2 = c * c;
+    const float p = (((ATAN_P7 * c2 + ATAN_P5) * c2 + ATAN_P3) * c2 + ATAN_P1) * c;
+    float a = ax >= ay ? p : 90.f - p;
+    if (fx < 0.f) a = 180.f - a;
+    if (fy < 0.f) a = 360.f - a;
+    return (uint32_t)(a * (128.f / 180.f) + 0.5f);
+}
+
 }  // namespace mvx

@@ -54,19 +54,49 @@ template <int TW, int TH> struct ChainTile {
     static_assert(TW % 16 == 0 && TH % 2 == 0, "tile width is a multiple of 16, height even");
 };
 
-MVX_DEV void unpack8(uint2 v, uint32_t *o)
+// The 3-row vertical sums of an 8-pixel chunk and the pixel on either side of it, from byte rows in LDS:
+// r0 + 2 r1 + r2 and r2 - r0 as column pairs.  E[0..1], O[0..1] are the chunk's two dwords; Ol.hi is the column
+// left of it, Er.lo the one right of it.
+struct ChunkSums {
+    u16x2 E[2], O[2], Ol, Er;
+};
+
+struct ChunkRows {
+    uint32_t w[3][4];   // rows, dwords: the one left of the chunk, its two, the one right of it
+};
+
+// p: the chunk's first byte in the first of three rows `pitch` apart, 8-byte aligned
+MVX_DEV ChunkRows chunk_rows(const uint8_t *p, int pitch)
 {
+    ChunkRows c;
 #pragma unroll
-    for (int i = 0; i < 4; i++) { o[i] = (v.x >> (8 * i)) & 0xffu; o[4 + i] = (v.y >> (8 * i)) & 0xffu; }
+    for (int j = 0; j < 3; j++) {
+        const uint8_t *q = p + j * pitch;
+        const uint2 m = *reinterpret_cast<const uint2 *>(q);
+        c.w[j][0] = *reinterpret_cast<const uint32_t *>(q - 4);
+        c.w[j][1] = m.x;
+        c.w[j][2] = m.y;
+        c.w[j][3] = *reinterpret_cast<const uint32_t *>(q + 8);
+    }
+    return c;
 }
 
-MVX_DEV void row24(const uint8_t *p, uint32_t (&b)[24])  // 24 bytes at an 8-byte aligned LDS address
+template <class Op> MVX_DEV ChunkSums chunk_sums(const ChunkRows &c, Op op)
 {
-    const uint2 *q = reinterpret_cast<const uint2 *>(p);
-    unpack8(q[0], b);
-    unpack8(q[1], b + 8);
-    unpack8(q[2], b + 16);
+    ChunkSums s;
+#pragma unroll
+    for (int d = 0; d < 2; d++) {
+        s.E[d] = op(even_bytes(c.w[0][d + 1]), even_bytes(c.w[1][d + 1]), even_bytes(c.w[2][d + 1]));
+        s.O[d] = op(odd_bytes(c.w[0][d + 1]), odd_bytes(c.w[1][d + 1]), odd_bytes(c.w[2][d + 1]));
+    }
+    s.Ol = op(odd_bytes(c.w[0][0]), odd_bytes(c.w[1][0]), odd_bytes(c.w[2][0]));
+    s.Er = op(even_bytes(c.w[0][3]), even_bytes(c.w[1][3]), even_bytes(c.w[2][3]));
+    return s;
 }
+
+// left and right neighbours of the even and odd columns of dword d
+MVX_DEV u16x2 even_left(const ChunkSums &s, int d) { return pair_shift(d ? s.O[0] : s.Ol, s.O[d]); }
+MVX_DEV u16x2 odd_right(const ChunkSums &s, int d) { return pair_shift(s.E[d], d ? s.Er : s.E[1]); }
 
 // blurred pixel validity at extended coordinate (r, c): the Gaussian node writes rows 1..h-2,
 // columns 0..w-1; every other byte of the virtual plane is zero.
@@ -147,34 +177,27 @@ k_chain_batch(const ChainRow *__restrict__ plan, uint32_t count, uint32_t numTil
         if (t + perXcd < tEnd) fetch(t + perXcd);
 
         // 2. blurred tile, 8 pixels per chunk: (h(r-1) + 2 h(r) + h(r+1)) >> 4 with
-        //    h = p(c-1) + 2 p(c) + p(c+1), as the Gaussian node computes it.
+        //    h = p(c-1) + 2 p(c) + p(c+1), as the Gaussian node computes it (vertical sums first: integers).
+        //    inside: every blurred byte of the tile is one the node writes.
+        const bool inside = x0 >= 8 && x0 + TW + 8 <= w && y0 >= 2 && y0 + TH <= h - 2;
         for (int i = threadIdx.x; i < T::RB * T::CB; i += T::NT) {
             const int rb = i / T::CB, cb = i - rb * T::CB;
-            uint32_t hs[8], b[24];
-            row24(sIn + rb * T::PIN + 8 * cb, b);
+            const ChunkRows rows = chunk_rows(sIn + rb * T::PIN + 8 + 8 * cb, T::PIN);
+            const ChunkSums v = chunk_sums(rows, [](u16x2 a, u16x2 b, u16x2 c) { return a + b * (unsigned short)2 + c; });
+            uint32_t o[2];
 #pragma unroll
-            for (int j = 0; j < 8; j++) hs[j] = b[7 + j] + 2 * b[8 + j] + b[9 + j];
-            row24(sIn + (rb + 1) * T::PIN + 8 * cb, b);
-#pragma unroll
-            for (int j = 0; j < 8; j++) hs[j] += 2 * (b[7 + j] + 2 * b[8 + j] + b[9 + j]);
-            row24(sIn + (rb + 2) * T::PIN + 8 * cb, b);
-#pragma unroll
-            for (int j = 0; j < 8; j++) hs[j] = (hs[j] + b[7 + j] + 2 * b[8 + j] + b[9 + j]) >> 4;
-            const int r = y0 - 1 + rb, c0 = x0 - 8 + 8 * cb;
-            if (c0 >= 0 && c0 + 8 <= stride) {
-                const bool rowOk = r >= 1 && r <= h - 2;
-#pragma unroll
-                for (int j = 0; j < 8; j++)
-                    if (!rowOk || c0 + j >= w) hs[j] = 0;
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; j++)
-                    if (!blur_valid(r, c0 + j, stride, w, h)) hs[j] = 0;
+            for (int d = 0; d < 2; d++) {
+                const u16x2 e = (even_left(v, d) + v.O[d] + v.E[d] * (unsigned short)2) >> (unsigned short)4;
+                const u16x2 f = (v.E[d] + odd_right(v, d) + v.O[d] * (unsigned short)2) >> (unsigned short)4;
+                o[d] = bits_of(e) | (bits_of(f) << 8);
             }
-            uint2 o;
-            o.x = hs[0] | (hs[1] << 8) | (hs[2] << 16) | (hs[3] << 24);
-            o.y = hs[4] | (hs[5] << 8) | (hs[6] << 16) | (hs[7] << 24);
-            *reinterpret_cast<uint2 *>(sBlur + rb * T::PB + 8 * cb) = o;
+            if (!inside) {   // bytes the Gaussian node does not write are zero
+                const int r = y0 - 1 + rb, c0 = x0 - 8 + 8 * cb;
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    if (!blur_valid(r, c0 + j, stride, w, h)) o[j >> 2] &= ~(0xffu << (8 * (j & 3)));
+            }
+            *reinterpret_cast<uint2 *>(sBlur + rb * T::PB + 8 * cb) = make_uint2(o[0], o[1]);
         }
         __syncthreads();
 
@@ -182,7 +205,7 @@ k_chain_batch(const ChainRow *__restrict__ plan, uint32_t count, uint32_t numTil
         //    NULL) the image takes the merged SobelMagnitudePhase kernel instead: no gradient stores, rows
         //    1..h-2 only, and magnitude columns from w & ~15 on truncate (ago_haf_cpu_filter.cpp:3972-4202).
         const bool merged = d.gx == nullptr;
-        const int magBody = merged ? (w & ~15) : (w & ~7);
+        const int magBody = w & ~15;
         for (int i = threadIdx.x; i < TH * (TW / 8); i += T::NT) {
             const int ro = i / (TW / 8), co = i - ro * (TW / 8);
             const int y = y0 + ro, x = x0 + 8 * co;
@@ -193,52 +216,56 @@ k_chain_batch(const ChainRow *__restrict__ plan, uint32_t count, uint32_t numTil
             int16_t *pgy = (int16_t *)((uint8_t *)d.gy + (long)y * d.gyStride) + x;
             int16_t *pmg = (int16_t *)((uint8_t *)d.mag + (long)y * d.magStride) + x;
             uint8_t *pph = d.phase + (long)y * d.phaseStride + x;
-            // gx | gy << 16 per pixel (both in [-1020, 1020]); zero on rows the Sobel node skips
-            uint32_t g[8];
+            // column pairs of gx and gy (16-bit, in [-1020, 1020]); zero on rows the Sobel node skips
+            uint32_t gxw[4] = {0, 0, 0, 0}, gyw[4] = {0, 0, 0, 0};
             if (rowOk) {
-                uint32_t b0[24], b1[24], b2[24];
-                row24(sBlur + ro * T::PB + 8 * co, b0);
-                row24(sBlur + (ro + 1) * T::PB + 8 * co, b1);
-                row24(sBlur + (ro + 2) * T::PB + 8 * co, b2);
+                const ChunkRows rows = chunk_rows(sBlur + ro * T::PB + 8 + 8 * co, T::PB);
+                const ChunkSums sm = chunk_sums(rows, [](u16x2 a, u16x2 b, u16x2 c) { return a + b * (unsigned short)2 + c; });
+                const ChunkSums df = chunk_sums(rows, [](u16x2 a, u16x2, u16x2 c) { return c - a; });
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int gx = ((int)b0[9 + j] - (int)b0[7 + j]) + 2 * ((int)b1[9 + j] - (int)b1[7 + j]) +
-                                   ((int)b2[9 + j] - (int)b2[7 + j]);
-                    const int gy = (int)(b2[7 + j] + 2 * b2[8 + j] + b2[9 + j]) - (int)(b0[7 + j] + 2 * b0[8 + j] + b0[9 + j]);
-                    g[j] = ((uint32_t)gx & 0xffffu) | ((uint32_t)gy << 16);
+                for (int d = 0; d < 2; d++) {
+                    const uint32_t xe = bits_of(sm.O[d] - even_left(sm, d)), xo = bits_of(odd_right(sm, d) - sm.E[d]);
+                    const uint32_t ye = bits_of(even_left(df, d) + df.O[d] + df.E[d] * (unsigned short)2);
+                    const uint32_t yo = bits_of(df.E[d] + odd_right(df, d) + df.O[d] * (unsigned short)2);
+                    gxw[2 * d] = __builtin_amdgcn_perm(xo, xe, 0x05040100u);       // columns 4d, 4d+1
+                    gxw[2 * d + 1] = __builtin_amdgcn_perm(xo, xe, 0x07060302u);   // columns 4d+2, 4d+3
+                    gyw[2 * d] = __builtin_amdgcn_perm(yo, ye, 0x05040100u);
+                    gyw[2 * d + 1] = __builtin_amdgcn_perm(yo, ye, 0x07060302u);
                 }
                 if (merged) {
                 } else if (full) {
-                    uint4 vx, vy;
-                    vx.x = (g[0] & 0xffffu) | (g[1] << 16);
-                    vx.y = (g[2] & 0xffffu) | (g[3] << 16);
-                    vx.z = (g[4] & 0xffffu) | (g[5] << 16);
-                    vx.w = (g[6] & 0xffffu) | (g[7] << 16);
-                    vy.x = (g[0] >> 16) | (g[1] & 0xffff0000u);
-                    vy.y = (g[2] >> 16) | (g[3] & 0xffff0000u);
-                    vy.z = (g[4] >> 16) | (g[5] & 0xffff0000u);
-                    vy.w = (g[6] >> 16) | (g[7] & 0xffff0000u);
-                    *reinterpret_cast<uint4 *>(pgx) = vx;
-                    *reinterpret_cast<uint4 *>(pgy) = vy;
+                    *reinterpret_cast<uint4 *>(pgx) = make_uint4(gxw[0], gxw[1], gxw[2], gxw[3]);
+                    *reinterpret_cast<uint4 *>(pgy) = make_uint4(gyw[0], gyw[1], gyw[2], gyw[3]);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 8; j++)
-                        if (x + j < w) { pgx[j] = (int16_t)(g[j] & 0xffffu); pgy[j] = (int16_t)(g[j] >> 16); }
+                        if (x + j < w) { pgx[j] = (int16_t)(gxw[j >> 1] >> (16 * (j & 1))); pgy[j] = (int16_t)(gyw[j >> 1] >> (16 * (j & 1))); }
                 }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; j++) g[j] = 0;
             }
-            // Magnitude and Phase, packed as they are produced
-            uint32_t mw[4] = {0, 0, 0, 0}, pw[2] = {0, 0};
-            const bool body = x + 8 <= magBody;
+            // Magnitude and Phase, packed as they are produced; the chain's gradients need no distinction of
+            // Magnitude's body and tail columns, only the merged kernel's tail truncates
+            uint32_t mw[4], pw[2];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int32_t gx = (int16_t)(g[j] & 0xffffu), gy = (int32_t)g[j] >> 16;
-                const int32_t m = (body || x + j < magBody) ? mag_body(gx, gy) : merged ? mag_trunc(gx, gy) : mag_tail(gx, gy);
-                mw[j >> 1] |= ((uint32_t)m & 0xffffu) << (16 * (j & 1));
-                pw[j >> 2] |= phase_px(gx, gy) << (8 * (j & 3));
+            for (int q = 0; q < 2; q++) {
+                uint32_t ph[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t a = gxw[2 * q + (j >> 1)], b = gyw[2 * q + (j >> 1)];
+                    const float fx = (float)((j & 1) ? (int32_t)a >> 16 : (int32_t)(int16_t)a), fy = (float)((j & 1) ? (int32_t)b >> 16 : (int32_t)(int16_t)b);
+                    const uint32_t m = mag_sobel(fx, fy);
+                    if (j & 1) mw[2 * q + (j >> 1)] = __builtin_amdgcn_perm(m, mw[2 * q + (j >> 1)], 0x05040100u);
+                    else mw[2 * q + (j >> 1)] = m;
+                    ph[j] = phase_sobel(fx, fy);
+                }
+                pw[q] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(ph[3], ph[2], 0x0c0c0400u), __builtin_amdgcn_perm(ph[1], ph[0], 0x0c0c0400u), 0x05040100u);
             }
+            if (merged && x + 8 > magBody)
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    if (x + j >= magBody) {
+                        const uint32_t m = mag_sobel_trunc((float)((int32_t)(gxw[j >> 1] << (16 * (~j & 1))) >> 16), (float)((int32_t)(gyw[j >> 1] << (16 * (~j & 1))) >> 16));
+                        mw[j >> 1] = (j & 1) ? (mw[j >> 1] & 0xffffu) | (m << 16) : (mw[j >> 1] & 0xffff0000u) | m;
+                    }
             if (full) {
                 *reinterpret_cast<uint4 *>(pmg) = make_uint4(mw[0], mw[1], mw[2], mw[3]);
                 *reinterpret_cast<uint2 *>(pph) = make_uint2(pw[0], pw[1]);
@@ -265,27 +292,26 @@ k_chain_batch(const ChainRow *__restrict__ plan, uint32_t count, uint32_t numTil
                 if (yh >= dh || xh >= dw) continue;
                 const uint4 r0 = *reinterpret_cast<const uint4 *>(sIn + (2 * rh + 2) * T::PIN + 16 + 16 * k);
                 const uint4 r1 = *reinterpret_cast<const uint4 *>(sIn + (2 * rh + 3) * T::PIN + 16 + 16 * k);
-                uint32_t a[16], c[16], o[8];
+                uint32_t o[8];
+                if (xh + 8 <= halfBody) {
+                    // rounded byte means: of each pair (bytes 0 and 2 of a dword), then of the two rows
+                    const uint32_t a[4] = {r0.x, r0.y, r0.z, r0.w}, c[4] = {r1.x, r1.y, r1.z, r1.w};
+                    uint32_t m[4];
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        m[j] = __builtin_amdgcn_lerp(__builtin_amdgcn_lerp(a[j], a[j] >> 8, 0x01010101u),
+                                                     __builtin_amdgcn_lerp(c[j], c[j] >> 8, 0x01010101u), 0x01010101u);
+                    *reinterpret_cast<uint2 *>(d.half + (long)yh * d.halfStride + xh) =
+                        make_uint2(__builtin_amdgcn_perm(m[1], m[0], 0x06040200u), __builtin_amdgcn_perm(m[3], m[2], 0x06040200u));
+                    continue;
+                }
+                uint32_t a[16], c[16];
                 unpack16(r0, a);
                 unpack16(r1, c);
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    if (xh + j < halfBody) {
-                        const uint32_t t0 = (a[2 * j] + a[2 * j + 1] + 1) >> 1, t1 = (c[2 * j] + c[2 * j + 1] + 1) >> 1;
-                        o[j] = (t0 + t1 + 1) >> 1;
-                    } else {
-                        o[j] = (a[2 * j] + a[2 * j + 1] + c[2 * j] + c[2 * j + 1] + 2) >> 2;
-                    }
-                }
+                for (int j = 0; j < 8; j++) o[j] = (a[2 * j] + a[2 * j + 1] + c[2 * j] + c[2 * j + 1] + 2) >> 2;
                 uint8_t *ph = d.half + (long)yh * d.halfStride + xh;
-                if (xh + 8 <= dw) {
-                    uint2 v;
-                    v.x = o[0] | (o[1] << 8) | (o[2] << 16) | (o[3] << 24);
-                    v.y = o[4] | (o[5] << 8) | (o[6] << 16) | (o[7] << 24);
-                    *reinterpret_cast<uint2 *>(ph) = v;
-                } else {
-                    for (int j = 0; xh + j < dw; j++) ph[j] = (uint8_t)o[j];
-                }
+                for (int j = 0; j < 8 && xh + j < dw; j++) ph[j] = (uint8_t)o[j];
             }
         }
         __syncthreads();  // the next tile overwrites both LDS tiles

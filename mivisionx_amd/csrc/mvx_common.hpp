@@ -77,6 +77,17 @@ MVX_DEV void st16_partial(uint8_t *p, const uint32_t (&o)[16], int n)
     }
 }
 
+// Two 16-bit values a register (packed integer arithmetic).  A row of bytes splits into pairs of even and odd
+// columns: dword d of the row gives (4d, 4d+2) and (4d+1, 4d+3).
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+MVX_DEV u16x2 pair_of(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
+MVX_DEV uint32_t bits_of(u16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+MVX_DEV u16x2 even_bytes(uint32_t v) { return pair_of(v & 0x00ff00ffu); }
+MVX_DEV u16x2 odd_bytes(uint32_t v) { return pair_of((v >> 8) & 0x00ff00ffu); }
+// (a.hi, b.lo): the pair one step on from a, b the pair that follows it
+MVX_DEV u16x2 pair_shift(u16x2 a, u16x2 b) { return pair_of(__builtin_amdgcn_alignbit(bits_of(b), bits_of(a), 16)); }
+
 // a / b for a divisor b fixed per launch, given y = RN(1/b) from recip_rn(b): the product a*y, its
 // exact remainder r = a - b*(a*y) by FMA, and one FMA correction (Markstein's correction step).
 // Where it replaces an IEEE division the replacement is checked exhaustively over every float a

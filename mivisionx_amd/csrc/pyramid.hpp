@@ -20,16 +20,10 @@ namespace mvx {
 // independent 16-byte loads and about 140 instructions make it 3 us for the small ones (3840x2160 to 1920x1080: 10.4 -> 6.2 us).
 constexpr int PYR_CHUNKS = 62;
 
-typedef unsigned short pyr_u16x2 __attribute__((ext_vector_type(2)));
-
-MVX_DEV pyr_u16x2 pyr_pair(uint32_t v) { return __builtin_bit_cast(pyr_u16x2, v); }
-MVX_DEV uint32_t pyr_bits(pyr_u16x2 v) { return __builtin_bit_cast(uint32_t, v); }
-// (a.hi, b.lo): the pair one column on from a, b the pair that follows it
-MVX_DEV pyr_u16x2 pyr_shift(pyr_u16x2 a, pyr_u16x2 b) { return pyr_pair(__builtin_amdgcn_alignbit(pyr_bits(b), pyr_bits(a), 16)); }
-MVX_DEV pyr_u16x2 pyr_from_prev(pyr_u16x2 v) { return pyr_pair((uint32_t)__builtin_amdgcn_update_dpp(0, (int)pyr_bits(v), 0x138, 0xf, 0xf, true)); }
-MVX_DEV pyr_u16x2 pyr_from_next(pyr_u16x2 v) { return pyr_pair((uint32_t)__builtin_amdgcn_update_dpp(0, (int)pyr_bits(v), 0x130, 0xf, 0xf, true)); }
+MVX_DEV u16x2 pyr_from_prev(u16x2 v) { return pair_of((uint32_t)__builtin_amdgcn_update_dpp(0, (int)bits_of(v), 0x138, 0xf, 0xf, true)); }
+MVX_DEV u16x2 pyr_from_next(u16x2 v) { return pair_of((uint32_t)__builtin_amdgcn_update_dpp(0, (int)bits_of(v), 0x130, 0xf, 0xf, true)); }
 // 1 4 6 4 1
-MVX_DEV pyr_u16x2 pyr_taps(pyr_u16x2 a, pyr_u16x2 b, pyr_u16x2 c, pyr_u16x2 d, pyr_u16x2 e)
+MVX_DEV u16x2 pyr_taps(u16x2 a, u16x2 b, u16x2 c, u16x2 d, u16x2 e)
 {
     return (a + e) + (b + d) * (unsigned short)4 + c * (unsigned short)6;
 }
@@ -50,35 +44,35 @@ MVX_DEV void half_row(uint32_t dw, uint8_t *dst, uint32_t dstStride, uint32_t sw
         const long off = row0 + (long)j * srcStride + 16 * chunk;   // linear addresses, zeros outside the plane
         p[j] = (off < 0 || off >= n) ? make_uint4(0, 0, 0, 0) : *reinterpret_cast<const uint4 *>(src + off);
     }
-    pyr_u16x2 E[6], O[6];   // vertical sums of columns 4d, 4d+2 and 4d+1, 4d+3 of dword d at [d + 1]
+    u16x2 E[6], O[6];   // vertical sums of columns 4d, 4d+2 and 4d+1, 4d+3 of dword d at [d + 1]
 #pragma unroll
     for (int d = 0; d < 4; d++) {
-        pyr_u16x2 e[5], o[5];
+        u16x2 e[5], o[5];
 #pragma unroll
         for (int j = 0; j < 5; j++) {
             const uint32_t v = d == 0 ? p[j].x : d == 1 ? p[j].y : d == 2 ? p[j].z : p[j].w;
-            e[j] = pyr_pair(v & 0x00ff00ffu);
-            o[j] = pyr_pair((v >> 8) & 0x00ff00ffu);
+            e[j] = even_bytes(v);
+            o[j] = odd_bytes(v);
         }
         E[d + 1] = pyr_taps(e[0], e[1], e[2], e[3], e[4]);
         O[d + 1] = pyr_taps(o[0], o[1], o[2], o[3], o[4]);
     }
-    pyr_u16x2 r[4];
+    u16x2 r[4];
     if (sw & 1) {   // centres 2x
         E[0] = pyr_from_prev(E[4]); O[0] = pyr_from_prev(O[4]);
         E[5] = pyr_from_next(E[1]);
 #pragma unroll
         for (int d = 1; d <= 4; d++)
-            r[d - 1] = pyr_taps(pyr_shift(E[d - 1], E[d]), pyr_shift(O[d - 1], O[d]), E[d], O[d], pyr_shift(E[d], E[d + 1]));
+            r[d - 1] = pyr_taps(pair_shift(E[d - 1], E[d]), pair_shift(O[d - 1], O[d]), E[d], O[d], pair_shift(E[d], E[d + 1]));
     } else {        // centres 2x + 1
         O[0] = pyr_from_prev(O[4]);
         E[5] = pyr_from_next(E[1]); O[5] = pyr_from_next(O[1]);
 #pragma unroll
         for (int d = 1; d <= 4; d++)
-            r[d - 1] = pyr_taps(pyr_shift(O[d - 1], O[d]), E[d], O[d], pyr_shift(E[d], E[d + 1]), pyr_shift(O[d], O[d + 1]));
+            r[d - 1] = pyr_taps(pair_shift(O[d - 1], O[d]), E[d], O[d], pair_shift(E[d], E[d + 1]), pair_shift(O[d], O[d + 1]));
     }
-    const uint2 v = make_uint2(__builtin_amdgcn_perm(pyr_bits(r[1]), pyr_bits(r[0]), 0x07050301u),
-                               __builtin_amdgcn_perm(pyr_bits(r[3]), pyr_bits(r[2]), 0x07050301u));
+    const uint2 v = make_uint2(__builtin_amdgcn_perm(bits_of(r[1]), bits_of(r[0]), 0x07050301u),
+                               __builtin_amdgcn_perm(bits_of(r[3]), bits_of(r[2]), 0x07050301u));
     const long x0 = 8 * chunk;
     if (lane == 0 || lane == 63 || x0 >= (long)dw) return;
     uint8_t *out = dst + (long)y * dstStride + x0;

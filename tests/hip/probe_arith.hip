@@ -9,6 +9,8 @@
 //   * div_by_const_rn(a, b, RN(1/b)) vs IEEE single division for every finite float a, for a given b;
 //   * l2_pack_simd(f) vs the Canny L2 SSE rule, cvtps_epi32(sqrt_ps(f)) packed to 16 bits, for every
 //     integer-valued float below 2^32;
+//   * mag_sobel, mag_sobel_trunc and phase_sobel vs mag_body and mag_tail, mag_trunc and phase_px, for every
+//     pair of 3x3 Sobel gradients (-1020..1020 each);
 //   * the lane mapping of the DPP wave_shl:1 control.
 #include "../../mivisionx_amd/csrc/arith.hpp"
 
@@ -39,6 +41,20 @@ __global__ void k_mag(uint32_t maxA, uint32_t *out)
         if (m != want) {
             atomicAdd(out, 1u);
             atomicCAS(out + 1, 0u, (gx << 16) | gy);
+        }
+    }
+}
+
+__global__ void k_sobel_px(uint32_t maxG, uint32_t *out)
+{
+    const int32_t gx = (int32_t)blockIdx.x - (int32_t)maxG;
+    for (int32_t gy = (int32_t)threadIdx.x - (int32_t)maxG; gy <= (int32_t)maxG; gy += (int32_t)blockDim.x) {
+        const float fx = (float)gx, fy = (float)gy;
+        const int32_t m = (int32_t)(mag_sobel(fx, fy) & 0xffffu);
+        if (m != mag_body(gx, gy) || m != mag_tail(gx, gy) || (int32_t)mag_sobel_trunc(fx, fy) != mag_trunc(gx, gy) ||
+            (phase_sobel(fx, fy) & 0xffu) != phase_px(gx, gy)) {
+            atomicAdd(out, 1u);
+            atomicCAS(out + 1, 0u, ((uint32_t)(gx + (int32_t)maxG) << 16) | (uint32_t)(gy + (int32_t)maxG));
         }
     }
 }
@@ -99,6 +115,7 @@ __global__ void k_dpp(int32_t *out)
 
 // result[0] = mismatches, result[1] = first mismatch packed as (b << 16) | a (b, a <= 32768)
 extern "C" int probe_div_small(uint32_t maxB, uint32_t *result) { return run(k_div, maxB, maxB, result); }
+extern "C" int probe_sobel_px(uint32_t maxG, uint32_t *result) { return run(k_sobel_px, 2 * maxG + 1, maxG, result); }
 extern "C" int probe_mag_body(uint32_t maxA, uint32_t *result) { return run(k_mag, maxA + 1, maxA, result); }
 
 // result[0] = mismatches, result[1] = bits of the first mismatching dividend

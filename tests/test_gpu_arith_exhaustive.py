@@ -38,6 +38,12 @@ def test_magnitude_rounding_all_pairs(probe):
     assert bad == 0, f"{bad} magnitudes differ; first (gx, gy) = {first}"
 
 
+def test_sobel_magnitude_and_phase_all_pairs(probe):
+    """the short forms for 3x3 Sobel gradients against the full-range ones, every pair of gradients"""
+    bad, first = _run(probe.probe_sobel_px, 1020)
+    assert bad == 0, f"{bad} pixels differ; first (gx + 1020, gy + 1020) = {first}"
+
+
 @pytest.mark.parametrize("gradient", [3])
 def test_harris_norm_division_all_floats(probe, gradient):
     """the Harris score divides by the fixed norm (255 * 2^(g-1) * 3)^4; the reciprocal-and-FMA
