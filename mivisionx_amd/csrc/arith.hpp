@@ -116,19 +116,19 @@ MVX_DEV uint32_t mag_sobel_trunc(float fx, float fy)
     return (uint32_t)__builtin_amdgcn_sqrtf(fmaf(fx, fx, fmaf(fy, fy, 0.5f)));
 }
 
-// phase_px; the low 8 bits are the phase (256 stands for 0).  floor(v + 1/2) as one float add and a
-// truncation: v is never the one float below 1/2 whose sum rounds up to 1.
+// phase_px; the low 8 bits are the phase (256 stands for 0).  The polynomial, the scale and the half of
+// floor(v + 1/2) fused: no pair's quantised phase depends on the roundings that leaves out.
 MVX_DEV uint32_t phase_sobel(float fx, float fy)
 {
     const float eps = (float)2.2204460492503131e-16;   // (float)DBL_EPSILON, which only matters for (0, 0)
     const float ax = fabsf(fx), ay = fabsf(fy);
     const float c = div_small_rn(fminf(ax, ay), fmaxf(fmaxf(ax, ay), eps));
     const float c2 = c * c;
-    const float p = (((ATAN_P7 * c2 + ATAN_P5) * c2 + ATAN_P3) * c2 + ATAN_P1) * c;
+    const float p = fmaf(fmaf(fmaf(ATAN_P7, c2, ATAN_P5), c2, ATAN_P3), c2, ATAN_P1) * c;
     float a = ax >= ay ? p : 90.f - p;
     if (fx < 0.f) a = 180.f - a;
     if (fy < 0.f) a = 360.f - a;
-    return (uint32_t)(a * (128.f / 180.f) + 0.5f);
+    return (uint32_t)fmaf(a, 128.f / 180.f, 0.5f);
 }
 
 }  // namespace mvx

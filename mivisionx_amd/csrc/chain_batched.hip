@@ -5,25 +5,32 @@
 // (HafCpu_Gaussian_U8_U8_3x3 ago_haf_cpu_filter.cpp:1681-1861 into a virtual image,
 // HafCpu_Sobel_S16S16_U8_3x3_GXY :2237, HafCpu_Magnitude_S16_S16S16 ago_haf_cpu_arithmetic.cpp:4989,
 // HafCpu_Phase_U8_S16S16 :9592, HafCpu_ScaleImage_U8_U8_Bilinear ago_haf_cpu_geometric.cpp:1977 on
-// the input), but the blurred image never leaves LDS.
+// the input), but the blurred image never leaves registers.
 //
-// Tiles.  An output tile is TW x TH pixels of one image.  Its workgroup stages the input rows
-// y0-2 .. y0+TH+1 over columns x0-16 .. x0+TW+15 in LDS, each cell holding the byte at LINEAR
-// index r*stride + c of the plane (0 outside [0, h*stride)): the reference reads 3x3 neighbours by
-// linear address, so the left neighbour of column 0 is the previous row's last byte and the right
-// neighbour of column w-1 is padding or the next row's first byte, and this "extended coordinate"
-// tile reproduces all of that without a special case.  The blurred tile (rows y0-1 .. y0+TH,
-// columns x0-8 .. x0+TW+7) is then computed from it with the Gaussian node's row rule -- a
-// blurred pixel is nonzero only on rows 1..h-2 and columns < w, because the node writes nothing
-// else and the plane starts zeroed -- and Sobel, Magnitude and Phase run from the blurred tile.
-// Rows 0 and h-1 of gx/gy are not written (the Sobel node leaves them); Magnitude and Phase of
-// those rows are computed from zero gradients, which is what the nodes compute from the zeroed
-// rows.  The half-size image is computed from the same input tile.
+// Lanes and tiles.  A lane owns 8 columns and streams down its rows, everything in registers: the input
+// rows' vertical sums, the blurred rows and the gradients are pairs of 16-bit columns, and the one or two
+// columns it needs on either side come with its own loads (16 bytes from 4 left of its columns), so no
+// lane waits for another and there is no LDS and no barrier.  Every byte is the one at LINEAR index
+// r*stride + c of the plane (0 outside [0, h*stride)): the reference reads 3x3 neighbours by linear address,
+// so the left neighbour of column 0 is the previous row's last byte and the right neighbour of column w-1
+// is padding or the next row's first byte.  A blurred pixel is nonzero only on rows 1..h-2 and columns < w,
+// because the Gaussian node writes nothing else and the plane starts zeroed.  Rows 0 and h-1 of gx/gy are
+// not written (the Sobel node leaves them); Magnitude and Phase of those rows are computed from zero
+// gradients, which is what the nodes compute from the zeroed rows.  The half-size image comes from the same
+// input rows.
+// An output tile is TW x TH pixels of one image, TW / 8 lanes; a wave takes tiles that follow each other, and an
+// image's tiles are counted up to whole waves, so a wave's lanes share one image.  Where all tiles together
+// leave SIMDs idle, a tile's rows are split among several waves (the two rows above and below a lane's rows
+// are read and blurred again: small batches have the room).
 //
-// Schedule.  Tiles of all images form one sequence (image after image, row-major inside an
+// Bound by memory and VALU issue alike: 8.25 bytes and 53 lane operations a pixel.  48 uneven images of
+// 118 Mpixel: 349 us with tiles in LDS (73 operations a pixel, a third of them blurring halos and unpacking
+// bytes twice), 283 us now.
+//
+// Schedule.  The waves' units of all images form one sequence (image after image, row-major inside an
 // image).  The grid is persistent: it is a multiple of 8 workgroups, workgroup b runs on XCD b%8
 // (MI355X dispatches workgroups round-robin over its 8 XCDs), the sequence is cut into 8 equal
-// contiguous ranges, one per XCD, and the workgroups of an XCD stride through its range, so tiles
+// contiguous ranges, one per XCD, and the waves of an XCD stride through its range, so tiles
 // that share halo rows are processed at the same time on the same L2.  No atomics: the schedule is
 // static, so a captured hipGraph replays without any reset.
 #include "arith.hpp"
@@ -44,70 +51,7 @@ struct ChainRow {  // device plan: one 128-byte row per image
 };
 static_assert(sizeof(ChainRow) == 128, "plan row is 128 bytes");
 
-template <int TW, int TH> struct ChainTile {
-    static constexpr int PIN = TW + 32;               // input tile pitch (columns x0-16 .. x0+TW+15)
-    static constexpr int RIN = TH + 4;                // input tile rows (y0-2 .. y0+TH+1)
-    static constexpr int PB = TW + 16;                // blurred tile pitch (columns x0-8 .. x0+TW+7)
-    static constexpr int RB = TH + 2;                 // blurred tile rows (y0-1 .. y0+TH)
-    static constexpr int CB = TW / 8 + 2;             // 8-pixel chunks per blurred row
-    static constexpr int NT = (TW * TH / 8 < 64) ? 64 : TW * TH / 8;   // threads: one 8-pixel chunk each
-    static_assert(TW % 16 == 0 && TH % 2 == 0, "tile width is a multiple of 16, height even");
-};
-
-// The 3-row vertical sums of an 8-pixel chunk and the pixel on either side of it, from byte rows in LDS:
-// r0 + 2 r1 + r2 and r2 - r0 as column pairs.  E[0..1], O[0..1] are the chunk's two dwords; Ol.hi is the column
-// left of it, Er.lo the one right of it.
-struct ChunkSums {
-    u16x2 E[2], O[2], Ol, Er;
-};
-
-struct ChunkRows {
-    uint32_t w[3][4];   // rows, dwords: the one left of the chunk, its two, the one right of it
-};
-
-// p: the chunk's first byte in the first of three rows `pitch` apart, 8-byte aligned
-MVX_DEV ChunkRows chunk_rows(const uint8_t *p, int pitch)
-{
-    ChunkRows c;
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-        const uint8_t *q = p + j * pitch;
-        const uint2 m = *reinterpret_cast<const uint2 *>(q);
-        c.w[j][0] = *reinterpret_cast<const uint32_t *>(q - 4);
-        c.w[j][1] = m.x;
-        c.w[j][2] = m.y;
-        c.w[j][3] = *reinterpret_cast<const uint32_t *>(q + 8);
-    }
-    return c;
-}
-
-template <class Op> MVX_DEV ChunkSums chunk_sums(const ChunkRows &c, Op op)
-{
-    ChunkSums s;
-#pragma unroll
-    for (int d = 0; d < 2; d++) {
-        s.E[d] = op(even_bytes(c.w[0][d + 1]), even_bytes(c.w[1][d + 1]), even_bytes(c.w[2][d + 1]));
-        s.O[d] = op(odd_bytes(c.w[0][d + 1]), odd_bytes(c.w[1][d + 1]), odd_bytes(c.w[2][d + 1]));
-    }
-    s.Ol = op(odd_bytes(c.w[0][0]), odd_bytes(c.w[1][0]), odd_bytes(c.w[2][0]));
-    s.Er = op(even_bytes(c.w[0][3]), even_bytes(c.w[1][3]), even_bytes(c.w[2][3]));
-    return s;
-}
-
-// left and right neighbours of the even and odd columns of dword d
-MVX_DEV u16x2 even_left(const ChunkSums &s, int d) { return pair_shift(d ? s.O[0] : s.Ol, s.O[d]); }
-MVX_DEV u16x2 odd_right(const ChunkSums &s, int d) { return pair_shift(s.E[d], d ? s.Er : s.E[1]); }
-
-// blurred pixel validity at extended coordinate (r, c): the Gaussian node writes rows 1..h-2,
-// columns 0..w-1; every other byte of the virtual plane is zero.
-MVX_DEV bool blur_valid(int r, int c, int stride, int w, int h)
-{
-    if (c < 0) { r -= 1; c += stride; }
-    else if (c >= stride) { const int q = c / stride; r += q; c -= q * stride; }
-    return r >= 1 && r <= h - 2 && c < w;
-}
-
-// image of tile t: the last plan row with tileBegin <= t (uniform across the workgroup)
+// image of tile t: the last plan row with tileBegin <= t (uniform across the wave)
 MVX_DEV uint32_t find_image(const ChainRow *__restrict__ plan, uint32_t count, uint32_t t)
 {
     uint32_t lo = 0, hi = count - 1;
@@ -118,203 +62,261 @@ MVX_DEV uint32_t find_image(const ChainRow *__restrict__ plan, uint32_t count, u
     return lo;
 }
 
-template <int TW, int TH>
-__global__ void __launch_bounds__((ChainTile<TW, TH>::NT))
-k_chain_batch(const ChainRow *__restrict__ plan, uint32_t count, uint32_t numTiles)
-{
-    using T = ChainTile<TW, TH>;
-    __shared__ __align__(16) uint8_t sIn[T::RIN * T::PIN];
-    __shared__ __align__(16) uint8_t sBlur[T::RB * T::PB];
+constexpr int CHAIN_THREADS = 256;
 
-    const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3, perXcd = gridDim.x >> 3;
-    const uint32_t span = (numTiles + 7u) / 8u;
-    const uint32_t tBegin = xcd * span, tEnd = min(numTiles, tBegin + span);
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x4 u32x4_dword __attribute__((aligned(4)));   // at a 4-byte aligned address
 
-    // Loads of the next tile's input are issued into registers before the current tile is
-    // computed, so their latency hides behind the blur / gradient work of this tile.
-    constexpr int CHUNKS = T::RIN * (T::PIN / 16), LOADS = (CHUNKS + T::NT - 1) / T::NT;
-    uint4 pre[LOADS];
-    auto fetch = [&](uint32_t t) {
-        const uint32_t img = find_image(plan, count, t);
-        const ChainRow &d = plan[img];
-        const int stride = (int)d.srcStride;
-        const uint32_t local = t - d.tileBegin;
-        const int ty = (int)(local / d.tilesX), tx = (int)(local - (uint32_t)ty * d.tilesX);
-        const long n = (long)d.h * stride;
+// the plane pointers come out of the plan: as global memory (flat accesses take the LDS counter along)
+template <class T> MVX_DEV gptr_t<T> at(const void *base, long offset) { return (gptr_t<T>)(gmem((const uint8_t *)base) + offset); }
+
+// one input row of a lane: dwords c-4, c, c+4, c+8 as column pairs
+struct InRow {
+    u16x2 E[4], O[4];
+};
+// one blurred row: columns c-1 (Ol.hi), c..c+7, c+8 (Er.lo)
+struct BlurRow {
+    u16x2 Ol, E[2], O[2], Er;
+};
+// the raw input bytes c..c+7 of a row, for the half-size image
+struct RawRow {
+    uint32_t w[2];
+};
+
+// One lane's rows of one image (its tile column x, rows y0 .. y0+rows-1 below h).
+struct ChainLane {
+    const ChainRow &d;
+    int w, h, stride, n, x;
+    bool merged, edge;                // edge: some blurred byte it sees may be one the Gaussian node does not write
+    uint32_t colE[2], colO[2];        // columns below w
+    bool wrapL, wrapR, rightOk;       // column c-1 / c+8 lies in the row above / below; column c+8 is below w
+    u16x2 two;                        // {2, 2} the compiler does not see through: multiply-adds instead of shifts and adds
+
+    MVX_DEV u32x4 load(int r) const
+    {
+        const uint32_t off = (uint32_t)r * (uint32_t)stride + (uint32_t)x - 4u;   // outside the plane: past n, or wrapped far past it
+        u32x4 v;
+        if (off <= (uint32_t)(n - 16)) {
+            v = *at<const u32x4_dword>(d.src, off);
+        } else {
+            v = u32x4{0, 0, 0, 0};
 #pragma unroll
-        for (int k = 0; k < LOADS; k++) {
-            const int i = threadIdx.x + k * T::NT;
-            pre[k] = make_uint4(0, 0, 0, 0);
-            if (i < CHUNKS) {
-                // 16-byte chunks at linear index (y0-2+row)*stride + x0-16+16c; stride and x0 are
-                // multiples of 16, so a chunk lies wholly inside or wholly outside [0, n)
-                const int row = i / (T::PIN / 16), c = i - row * (T::PIN / 16);
-                const long L = (long)(ty * TH - 2 + row) * stride + (tx * TW - 16 + 16 * c);
-                if (L >= 0 && L < n) pre[k] = ld16(d.src + L);
-            }
+            for (int k = 0; k < 4; k++)
+                if (off + 4u * k <= (uint32_t)(n - 4)) v[k] = *at<const uint32_t>(d.src, off + 4u * k);
         }
-    };
+        return v;
+    }
 
-    uint32_t t = tBegin + slot;
-    if (t < tEnd) fetch(t);
-    for (; t < tEnd; t += perXcd) {
-        const ChainRow &d = plan[find_image(plan, count, t)];
-        const int w = (int)d.w, h = (int)d.h, stride = (int)d.srcStride;
-        const uint32_t local = t - d.tileBegin;
-        const int ty = (int)(local / d.tilesX), tx = (int)(local - (uint32_t)ty * d.tilesX);
-        const int x0 = tx * TW, y0 = ty * TH;
+    MVX_DEV uint32_t row_mask(int r) const { return (uint32_t)(r - 1) < (uint32_t)(h - 2) ? ~0u : 0u; }
 
-        // 1. input tile (rows y0-2 .. y0+TH+1, columns x0-16 .. x0+TW+15) from the prefetched chunks
+    // blurred row r from input rows r-1, r, r+1: (h(r-1) + 2 h(r) + h(r+1)) >> 4 with h = p(c-1) + 2 p(c) + p(c+1),
+    // as the Gaussian node computes it (vertical sums first: integers)
+    MVX_DEV BlurRow blur(int r, const InRow &a, const InRow &b, const InRow &c) const
+    {
+        InRow v;
 #pragma unroll
-        for (int k = 0; k < LOADS; k++) {
-            const int i = threadIdx.x + k * T::NT;
-            if (i < CHUNKS) {
-                const int row = i / (T::PIN / 16), c = i - row * (T::PIN / 16);
-                *reinterpret_cast<uint4 *>(sIn + row * T::PIN + 16 * c) = pre[k];
-            }
+        for (int k = 0; k < 4; k++) {
+            v.E[k] = a.E[k] + b.E[k] * two + c.E[k];
+            v.O[k] = a.O[k] + b.O[k] * two + c.O[k];
         }
-        __syncthreads();
-        if (t + perXcd < tEnd) fetch(t + perXcd);
-
-        // 2. blurred tile, 8 pixels per chunk: (h(r-1) + 2 h(r) + h(r+1)) >> 4 with
-        //    h = p(c-1) + 2 p(c) + p(c+1), as the Gaussian node computes it (vertical sums first: integers).
-        //    inside: every blurred byte of the tile is one the node writes.
-        const bool inside = x0 >= 8 && x0 + TW + 8 <= w && y0 >= 2 && y0 + TH <= h - 2;
-        for (int i = threadIdx.x; i < T::RB * T::CB; i += T::NT) {
-            const int rb = i / T::CB, cb = i - rb * T::CB;
-            const ChunkRows rows = chunk_rows(sIn + rb * T::PIN + 8 + 8 * cb, T::PIN);
-            const ChunkSums v = chunk_sums(rows, [](u16x2 a, u16x2 b, u16x2 c) { return a + b * (unsigned short)2 + c; });
-            uint32_t o[2];
+        const auto even = [&](int k) { return (pair_shift(v.O[k - 1], v.O[k]) + v.O[k] + v.E[k] * two) >> (unsigned short)4; };
+        const auto odd = [&](int k) { return (v.E[k] + pair_shift(v.E[k], v.E[k + 1]) + v.O[k] * two) >> (unsigned short)4; };
+        BlurRow o{odd(0), {even(1), even(2)}, {odd(1), odd(2)}, even(3)};
+        if (edge) {
+            const uint32_t m = row_mask(r);
 #pragma unroll
-            for (int d = 0; d < 2; d++) {
-                const u16x2 e = (even_left(v, d) + v.O[d] + v.E[d] * (unsigned short)2) >> (unsigned short)4;
-                const u16x2 f = (v.E[d] + odd_right(v, d) + v.O[d] * (unsigned short)2) >> (unsigned short)4;
-                o[d] = bits_of(e) | (bits_of(f) << 8);
+            for (int k = 0; k < 2; k++) {
+                o.E[k] = pair_of(bits_of(o.E[k]) & colE[k] & m);
+                o.O[k] = pair_of(bits_of(o.O[k]) & colO[k] & m);
             }
-            if (!inside) {   // bytes the Gaussian node does not write are zero
-                const int r = y0 - 1 + rb, c0 = x0 - 8 + 8 * cb;
-#pragma unroll
-                for (int j = 0; j < 8; j++)
-                    if (!blur_valid(r, c0 + j, stride, w, h)) o[j >> 2] &= ~(0xffu << (8 * (j & 3)));
-            }
-            *reinterpret_cast<uint2 *>(sBlur + rb * T::PB + 8 * cb) = make_uint2(o[0], o[1]);
+            o.Ol = pair_of(bits_of(o.Ol) & (x > 0 ? m : wrapL ? row_mask(r - 1) : 0u));
+            o.Er = pair_of(bits_of(o.Er) & (rightOk ? m : wrapR ? row_mask(r + 1) : 0u));
         }
-        __syncthreads();
+        return o;
+    }
 
-        // 3. Sobel, Magnitude, Phase: 8 pixels of one row per chunk.  With virtual gradients (gx == gy ==
-        //    NULL) the image takes the merged SobelMagnitudePhase kernel instead: no gradient stores, rows
-        //    1..h-2 only, and magnitude columns from w & ~15 on truncate (ago_haf_cpu_filter.cpp:3972-4202).
-        const bool merged = d.gx == nullptr;
-        const int magBody = w & ~15;
-        for (int i = threadIdx.x; i < TH * (TW / 8); i += T::NT) {
-            const int ro = i / (TW / 8), co = i - ro * (TW / 8);
-            const int y = y0 + ro, x = x0 + 8 * co;
-            if (y >= h || x >= w) continue;
-            const bool rowOk = y >= 1 && y <= h - 2, full = x + 8 <= w;
-            if (merged && !rowOk) continue;
-            int16_t *pgx = (int16_t *)((uint8_t *)d.gx + (long)y * d.gxStride) + x;
-            int16_t *pgy = (int16_t *)((uint8_t *)d.gy + (long)y * d.gyStride) + x;
-            int16_t *pmg = (int16_t *)((uint8_t *)d.mag + (long)y * d.magStride) + x;
-            uint8_t *pph = d.phase + (long)y * d.phaseStride + x;
-            // column pairs of gx and gy (16-bit, in [-1020, 1020]); zero on rows the Sobel node skips
-            uint32_t gxw[4] = {0, 0, 0, 0}, gyw[4] = {0, 0, 0, 0};
-            if (rowOk) {
-                const ChunkRows rows = chunk_rows(sBlur + ro * T::PB + 8 + 8 * co, T::PB);
-                const ChunkSums sm = chunk_sums(rows, [](u16x2 a, u16x2 b, u16x2 c) { return a + b * (unsigned short)2 + c; });
-                const ChunkSums df = chunk_sums(rows, [](u16x2 a, u16x2, u16x2 c) { return c - a; });
+    MVX_DEV void put_magphase(int y, bool full, u32x4 m, u32x2 p) const
+    {
+        const long pm = (long)y * d.magStride + 2 * x, pp = (long)y * d.phaseStride + x;
+        if (full) {
+            *at<u32x4>(d.mag, pm) = m;
+            *at<u32x2>(d.phase, pp) = p;
+            return;
+        }
 #pragma unroll
-                for (int d = 0; d < 2; d++) {
-                    const uint32_t xe = bits_of(sm.O[d] - even_left(sm, d)), xo = bits_of(odd_right(sm, d) - sm.E[d]);
-                    const uint32_t ye = bits_of(even_left(df, d) + df.O[d] + df.E[d] * (unsigned short)2);
-                    const uint32_t yo = bits_of(df.E[d] + odd_right(df, d) + df.O[d] * (unsigned short)2);
-                    gxw[2 * d] = __builtin_amdgcn_perm(xo, xe, 0x05040100u);       // columns 4d, 4d+1
-                    gxw[2 * d + 1] = __builtin_amdgcn_perm(xo, xe, 0x07060302u);   // columns 4d+2, 4d+3
-                    gyw[2 * d] = __builtin_amdgcn_perm(yo, ye, 0x05040100u);
-                    gyw[2 * d + 1] = __builtin_amdgcn_perm(yo, ye, 0x07060302u);
-                }
-                if (merged) {
-                } else if (full) {
-                    *reinterpret_cast<uint4 *>(pgx) = make_uint4(gxw[0], gxw[1], gxw[2], gxw[3]);
-                    *reinterpret_cast<uint4 *>(pgy) = make_uint4(gyw[0], gyw[1], gyw[2], gyw[3]);
+        for (int j = 0; j < 4; j++)   // widths are even
+            if (x + 2 * j < w) {
+                *at<uint32_t>(d.mag, pm + 4 * j) = m[j];
+                *at<uint16_t>(d.phase, pp + 2 * j) = (uint16_t)(p[j >> 1] >> (16 * (j & 1)));
+            }
+    }
+
+    // Sobel, Magnitude, Phase of row y from blurred rows y-1, y, y+1.  With virtual gradients (gx == gy == NULL)
+    // the image takes the merged SobelMagnitudePhase kernel instead: no gradient stores, rows 1..h-2 only,
+    // and magnitude columns from w & ~15 on truncate (ago_haf_cpu_filter.cpp:3972-4202).
+    MVX_DEV void gradients(int y, const BlurRow &a, const BlurRow &b, const BlurRow &c) const
+    {
+        const bool full = x + 8 <= w;
+        if (row_mask(y) == 0) {   // the Sobel node skips the row; the other nodes see zero gradients
+            if (merged) return;
+            put_magphase(y, full, u32x4{0, 0, 0, 0}, u32x2{0, 0});
+            return;
+        }
+        uint32_t gxw[4], gyw[4];   // columns of gx and gy in order (16-bit, in [-1020, 1020])
+        {
+            const auto sum = [this](u16x2 p, u16x2 q, u16x2 r) { return p + q * two + r; };
+            const BlurRow s{sum(a.Ol, b.Ol, c.Ol), {sum(a.E[0], b.E[0], c.E[0]), sum(a.E[1], b.E[1], c.E[1])},
+                            {sum(a.O[0], b.O[0], c.O[0]), sum(a.O[1], b.O[1], c.O[1])}, sum(a.Er, b.Er, c.Er)};
+            const BlurRow f{c.Ol - a.Ol, {c.E[0] - a.E[0], c.E[1] - a.E[1]}, {c.O[0] - a.O[0], c.O[1] - a.O[1]}, c.Er - a.Er};
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const uint32_t xe = bits_of(s.O[k] - pair_shift(k ? s.O[0] : s.Ol, s.O[k])), xo = bits_of(pair_shift(s.E[k], k ? s.Er : s.E[1]) - s.E[k]);
+                const uint32_t ye = bits_of(sum(pair_shift(k ? f.O[0] : f.Ol, f.O[k]), f.E[k], f.O[k]));
+                const uint32_t yo = bits_of(sum(f.E[k], f.O[k], pair_shift(f.E[k], k ? f.Er : f.E[1])));
+                gxw[2 * k] = __builtin_amdgcn_perm(xo, xe, 0x05040100u);       // columns 4k, 4k+1
+                gxw[2 * k + 1] = __builtin_amdgcn_perm(xo, xe, 0x07060302u);   // columns 4k+2, 4k+3
+                gyw[2 * k] = __builtin_amdgcn_perm(yo, ye, 0x05040100u);
+                gyw[2 * k + 1] = __builtin_amdgcn_perm(yo, ye, 0x07060302u);
+            }
+            if (!merged) {
+                const long px = (long)y * d.gxStride + 2 * x, py = (long)y * d.gyStride + 2 * x;
+                if (full) {
+                    *at<u32x4>(d.gx, px) = u32x4{gxw[0], gxw[1], gxw[2], gxw[3]};
+                    *at<u32x4>(d.gy, py) = u32x4{gyw[0], gyw[1], gyw[2], gyw[3]};
                 } else {
 #pragma unroll
-                    for (int j = 0; j < 8; j++)
-                        if (x + j < w) { pgx[j] = (int16_t)(gxw[j >> 1] >> (16 * (j & 1))); pgy[j] = (int16_t)(gyw[j >> 1] >> (16 * (j & 1))); }
-                }
-            }
-            // Magnitude and Phase, packed as they are produced; the chain's gradients need no distinction of
-            // Magnitude's body and tail columns, only the merged kernel's tail truncates
-            uint32_t mw[4], pw[2];
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                uint32_t ph[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const uint32_t a = gxw[2 * q + (j >> 1)], b = gyw[2 * q + (j >> 1)];
-                    const float fx = (float)((j & 1) ? (int32_t)a >> 16 : (int32_t)(int16_t)a), fy = (float)((j & 1) ? (int32_t)b >> 16 : (int32_t)(int16_t)b);
-                    const uint32_t m = mag_sobel(fx, fy);
-                    if (j & 1) mw[2 * q + (j >> 1)] = __builtin_amdgcn_perm(m, mw[2 * q + (j >> 1)], 0x05040100u);
-                    else mw[2 * q + (j >> 1)] = m;
-                    ph[j] = phase_sobel(fx, fy);
-                }
-                pw[q] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(ph[3], ph[2], 0x0c0c0400u), __builtin_amdgcn_perm(ph[1], ph[0], 0x0c0c0400u), 0x05040100u);
-            }
-            if (merged && x + 8 > magBody)
-#pragma unroll
-                for (int j = 0; j < 8; j++)
-                    if (x + j >= magBody) {
-                        const uint32_t m = mag_sobel_trunc((float)((int32_t)(gxw[j >> 1] << (16 * (~j & 1))) >> 16), (float)((int32_t)(gyw[j >> 1] << (16 * (~j & 1))) >> 16));
-                        mw[j >> 1] = (j & 1) ? (mw[j >> 1] & 0xffffu) | (m << 16) : (mw[j >> 1] & 0xffff0000u) | m;
-                    }
-            if (full) {
-                *reinterpret_cast<uint4 *>(pmg) = make_uint4(mw[0], mw[1], mw[2], mw[3]);
-                *reinterpret_cast<uint2 *>(pph) = make_uint2(pw[0], pw[1]);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; j++)
-                    if (x + j < w) {
-                        pmg[j] = (int16_t)(mw[j >> 1] >> (16 * (j & 1)));
-                        pph[j] = (uint8_t)(pw[j >> 2] >> (8 * (j & 3)));
-                    }
-            }
-        }
-
-        // 4. ScaleImage to (w/2, h/2).  With xscale = yscale = 2 the reference's fixed-point setup
-        //    (xinc = 2^19, xoffs = 2^17) gives source column 2x and row 2y with weight 128 on both
-        //    pixels, so the two-stage SIMD rule is ((p00+p01+1)>>1 + (p10+p11+1)>>1 + 1) >> 1 and
-        //    the single-rounding tail (columns >= (w/2) & ~7) is (p00+p01+p10+p11+2) >> 2; the row
-        //    and column clamps never engage.
-        if (d.half) {
-            const int dw = w >> 1, dh = h >> 1, halfBody = dw & ~7;
-            for (int i = threadIdx.x; i < (TH / 2) * (TW / 16); i += T::NT) {
-                const int rh = i / (TW / 16), k = i - rh * (TW / 16);
-                const int yh = (y0 >> 1) + rh, xh = (x0 >> 1) + 8 * k;
-                if (yh >= dh || xh >= dw) continue;
-                const uint4 r0 = *reinterpret_cast<const uint4 *>(sIn + (2 * rh + 2) * T::PIN + 16 + 16 * k);
-                const uint4 r1 = *reinterpret_cast<const uint4 *>(sIn + (2 * rh + 3) * T::PIN + 16 + 16 * k);
-                uint32_t o[8];
-                if (xh + 8 <= halfBody) {
-                    // rounded byte means: of each pair (bytes 0 and 2 of a dword), then of the two rows
-                    const uint32_t a[4] = {r0.x, r0.y, r0.z, r0.w}, c[4] = {r1.x, r1.y, r1.z, r1.w};
-                    uint32_t m[4];
-#pragma unroll
                     for (int j = 0; j < 4; j++)
-                        m[j] = __builtin_amdgcn_lerp(__builtin_amdgcn_lerp(a[j], a[j] >> 8, 0x01010101u),
-                                                     __builtin_amdgcn_lerp(c[j], c[j] >> 8, 0x01010101u), 0x01010101u);
-                    *reinterpret_cast<uint2 *>(d.half + (long)yh * d.halfStride + xh) =
-                        make_uint2(__builtin_amdgcn_perm(m[1], m[0], 0x06040200u), __builtin_amdgcn_perm(m[3], m[2], 0x06040200u));
-                    continue;
+                        if (x + 2 * j < w) {
+                            *at<uint32_t>(d.gx, px + 4 * j) = gxw[j];
+                            *at<uint32_t>(d.gy, py + 4 * j) = gyw[j];
+                        }
                 }
-                uint32_t a[16], c[16];
-                unpack16(r0, a);
-                unpack16(r1, c);
-#pragma unroll
-                for (int j = 0; j < 8; j++) o[j] = (a[2 * j] + a[2 * j + 1] + c[2 * j] + c[2 * j + 1] + 2) >> 2;
-                uint8_t *ph = d.half + (long)yh * d.halfStride + xh;
-                for (int j = 0; j < 8 && xh + j < dw; j++) ph[j] = (uint8_t)o[j];
             }
         }
-        __syncthreads();  // the next tile overwrites both LDS tiles
+        // the chain's gradients need no distinction of Magnitude's body and tail columns, only the merged
+        // kernel's tail truncates
+        uint32_t mw[4], pw[2];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            uint32_t ph[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t gx = gxw[2 * q + (j >> 1)], gy = gyw[2 * q + (j >> 1)];
+                const float fx = (float)((j & 1) ? (int32_t)gx >> 16 : (int32_t)(int16_t)gx), fy = (float)((j & 1) ? (int32_t)gy >> 16 : (int32_t)(int16_t)gy);
+                const uint32_t m = mag_sobel(fx, fy);
+                if (j & 1) mw[2 * q + (j >> 1)] = __builtin_amdgcn_perm(m, mw[2 * q + (j >> 1)], 0x05040100u);
+                else mw[2 * q + (j >> 1)] = m;
+                ph[j] = phase_sobel(fx, fy);
+            }
+            pw[q] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(ph[3], ph[2], 0x0c0c0400u), __builtin_amdgcn_perm(ph[1], ph[0], 0x0c0c0400u), 0x05040100u);
+        }
+        const int body = w & ~15;
+        if (merged && x + 8 > body)
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (x + j >= body) {
+                    const uint32_t gx = gxw[j >> 1], gy = gyw[j >> 1];
+                    const uint32_t m = mag_sobel_trunc((float)((j & 1) ? (int32_t)gx >> 16 : (int32_t)(int16_t)gx),
+                                                       (float)((j & 1) ? (int32_t)gy >> 16 : (int32_t)(int16_t)gy));
+                    mw[j >> 1] = (j & 1) ? (mw[j >> 1] & 0xffffu) | (m << 16) : (mw[j >> 1] & 0xffff0000u) | m;
+                }
+        put_magphase(y, full, u32x4{mw[0], mw[1], mw[2], mw[3]}, u32x2{pw[0], pw[1]});
+    }
+
+    // ScaleImage to (w/2, h/2), rows y and y+1 (y even).  With xscale = yscale = 2 the reference's fixed-point
+    // setup (xinc = 2^19, xoffs = 2^17) gives source column 2x and row 2y with weight 128 on both pixels, so the
+    // two-stage SIMD rule is ((p00+p01+1)>>1 + (p10+p11+1)>>1 + 1) >> 1 -- rounded byte means, v_lerp_u8 -- and the
+    // single-rounding tail (columns >= (w/2) & ~7) is (p00+p01+p10+p11+2) >> 2; the row and column clamps never
+    // engage.
+    MVX_DEV void half(int y, const RawRow &a, const RawRow &b) const
+    {
+        const int dw = w >> 1, xh = x >> 1;
+        const long ph = (long)(y >> 1) * d.halfStride + xh;
+        if (xh + 4 <= (dw & ~7)) {
+            uint32_t m[2];
+#pragma unroll
+            for (int k = 0; k < 2; k++)   // bytes 0 and 2
+                m[k] = __builtin_amdgcn_lerp(__builtin_amdgcn_lerp(a.w[k], a.w[k] >> 8, 0x01010101u),
+                                             __builtin_amdgcn_lerp(b.w[k], b.w[k] >> 8, 0x01010101u), 0x01010101u);
+            *at<uint32_t>(d.half, ph) = __builtin_amdgcn_perm(m[1], m[0], 0x06040200u);
+            return;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int sh = 16 * (j & 1);
+            const uint32_t p = a.w[j >> 1] >> sh, q = b.w[j >> 1] >> sh;
+            if (xh + j < dw) *at<uint8_t>(d.half, ph + j) = (uint8_t)(((p & 0xffu) + ((p >> 8) & 0xffu) + (q & 0xffu) + ((q >> 8) & 0xffu) + 2) >> 2);
+        }
+    }
+};
+
+// `rows` per lane (even, a divisor of TH); `units` waves' worth of work, TH / rows of them per wave of tiles
+template <int TW, int TH>
+__global__ void __launch_bounds__(CHAIN_THREADS)
+k_chain_batch(const ChainRow *__restrict__ plan, uint32_t count, uint32_t units, uint32_t rows)
+{
+    constexpr uint32_t LPT = TW / 8, TPW = 64 / LPT;   // lanes per tile, tiles per wave
+    const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3, step = (gridDim.x >> 3) * (CHAIN_THREADS / 64);
+    const uint32_t span = (units + 7u) / 8u;
+    const uint32_t uBegin = xcd * span, uEnd = min(units, uBegin + span);
+    const uint32_t parts = TH / rows;
+    for (uint32_t u = uBegin + slot * (CHAIN_THREADS / 64) + wave; u < uEnd; u += step) {
+        const uint32_t group = u / parts, part = u - group * parts;
+        const ChainRow &d = plan[find_image(plan, count, group * TPW)];
+        const uint32_t tile = group * TPW - d.tileBegin + lane / LPT, ty = tile / d.tilesX, tx = tile - ty * d.tilesX;
+        const int x = (int)(tx * TW + 8 * (lane % LPT)), y0 = (int)(ty * TH + part * rows);
+        const int w = (int)d.w, h = (int)d.h, stride = (int)d.srcStride;
+        if (x >= w || y0 >= h) continue;
+        ChainLane L{d, w, h, stride, h * stride, x};
+        uint32_t two = 0x00020002u;
+        asm("" : "+s"(two));
+        L.two = pair_of(two);
+        L.merged = d.gx == nullptr;
+        L.wrapL = stride == w;
+        L.rightOk = x + 8 < w;
+        L.wrapR = x + 8 == stride;
+        L.edge = x == 0 || !L.rightOk || y0 < 2 || y0 + (int)rows > h - 2;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {   // (widths are even: a pair's columns c, c+2 end at w - c > 0, > 2)
+            const int e = x + 4 * k, o = e + 1;
+            L.colE[k] = (e < w ? 0xffffu : 0u) | (e + 2 < w ? 0xffff0000u : 0u);
+            L.colO[k] = (o < w ? 0xffffu : 0u) | (o + 2 < w ? 0xffff0000u : 0u);
+        }
+        const bool wantHalf = d.half != nullptr;
+        const auto split = [](const u32x4 &v) {
+            InRow r;
+#pragma unroll
+            for (int k = 0; k < 4; k++) { r.E[k] = even_bytes(v[k]); r.O[k] = odd_bytes(v[k]); }
+            return r;
+        };
+        // Step k takes input row y0+k (next), which completes blurred row y0+k-1 and, from k = 2 on, output row
+        // y0+k-2.  Two rows of each kind are kept and the new one goes over the older, so the caller swaps the
+        // arguments instead of the values.
+        InRow ia = split(L.load(y0 - 2)), ib = split(L.load(y0 - 1));
+        u32x4 next = L.load(y0);
+        BlurRow ba{}, bb{};
+        RawRow ra{}, rb{};
+        const auto row = [&](int k, InRow &iO, InRow &iN, BlurRow &bO, BlurRow &bN, RawRow &rO, RawRow &rN) {
+            const u32x4 cur = next;
+            next = L.load(y0 + k + 1);
+            const InRow in = split(cur);
+            const BlurRow b = L.blur(y0 + k - 1, iO, iN, in);
+            if (k >= 2 && y0 + k - 2 < h) {
+                L.gradients(y0 + k - 2, bO, bN, b);
+                if (wantHalf && !(k & 1)) L.half(y0 + k - 2, rO, rN);
+            }
+            iO = in;
+            bO = b;
+            rO.w[0] = cur[1];
+            rO.w[1] = cur[2];
+        };
+#pragma unroll 1
+        for (int k = 0; k < (int)rows + 2; k += 2) {
+            row(k, ia, ib, ba, bb, ra, rb);
+            row(k + 1, ib, ia, bb, ba, rb, ra);
+        }
     }
 }
 
@@ -322,11 +324,22 @@ k_chain_batch(const ChainRow *__restrict__ plan, uint32_t count, uint32_t numTil
 struct TileShape { int tw, th; };
 constexpr TileShape kShapes[MVX_CHAIN_TILE_COUNT] = {{16, 16}, {32, 16}, {32, 32}, {64, 16}, {64, 32}};
 
-typedef void (*ChainKernel)(const ChainRow *, uint32_t, uint32_t);
+typedef void (*ChainKernel)(const ChainRow *, uint32_t, uint32_t, uint32_t);
 constexpr ChainKernel kKernels[MVX_CHAIN_TILE_COUNT] = {k_chain_batch<16, 16>, k_chain_batch<32, 16>, k_chain_batch<32, 32>,
                                                         k_chain_batch<64, 16>, k_chain_batch<64, 32>};
-constexpr int kThreads[MVX_CHAIN_TILE_COUNT] = {ChainTile<16, 16>::NT, ChainTile<32, 16>::NT, ChainTile<32, 32>::NT,
-                                                ChainTile<64, 16>::NT, ChainTile<64, 32>::NT};
+// tiles one wave takes side by side
+constexpr uint32_t tiles_per_wave(uint32_t tile) { return 64u / ((uint32_t)kShapes[tile].tw / 8u); }
+
+// Rows a lane streams: the tile's, halved down to 4 while the whole batch is fewer than 8192 waves (eight for each of
+// the 1024 SIMDs, of which about four run at a time, so that no SIMD ends long after the others: 48 uneven images with
+// 64x32 tiles took 294 us at 2048, 283 at 8192); a lane's rows cost one more load and blur above and below them each.
+inline uint32_t rows_per_lane(uint32_t numTiles, uint32_t tile)
+{
+    uint32_t rows = (uint32_t)kShapes[tile].th;
+    uint64_t waves = numTiles / tiles_per_wave(tile);
+    while (rows > 4 && waves < 8192) { rows /= 2; waves *= 2; }
+    return rows;
+}
 
 inline bool plane_ok_cb(const void *p, uint32_t w, uint32_t stride, uint32_t bpp)
 {
@@ -414,19 +427,22 @@ extern "C" int mvx_ChainBatch_prepare(const mvx_chain_image_t *images, uint32_t 
         r.magStride = im.magStride; r.phaseStride = im.phaseStride; r.halfStride = im.halfStride;
         r.tilesX = (im.width + s.tw - 1) / s.tw;
         r.tileBegin = (uint32_t)tiles;
-        tiles += (uint64_t)r.tilesX * ((im.height + s.th - 1) / s.th);
+        const uint64_t own = (uint64_t)r.tilesX * ((im.height + s.th - 1) / s.th), per = tiles_per_wave(tile);
+        tiles += (own + per - 1) / per * per;   // whole waves: a wave's lanes share one image
         if (tiles >= (1ull << 31)) return MVX_ERROR_INVALID_PARAMETERS;
     }
     int occ = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void *>(kKernels[tile]), kThreads[tile], 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void *>(kKernels[tile]), CHAIN_THREADS, 0) !=
             hipSuccess || occ <= 0)
         return MVX_FAILURE;
     const int cus = device_cus();
     if (cus <= 0) return MVX_FAILURE;
     const uint32_t perCu = workgroupsPerCU == 0 ? (uint32_t)occ : std::min<uint32_t>(workgroupsPerCU, (uint32_t)occ);
     uint32_t wgs = (uint32_t)cus * perCu;
-    // no more workgroups than tiles (rounded to a multiple of the 8 XCDs)
-    wgs = std::min<uint32_t>(wgs, (uint32_t)((tiles + 7) / 8 * 8));
+    // no more workgroups than there are waves' units for (rounded to a multiple of the 8 XCDs)
+    const uint64_t units = tiles / tiles_per_wave(tile) * ((uint32_t)s.th / rows_per_lane((uint32_t)tiles, tile));
+    const uint64_t perXcd = ((units + 7) / 8 + CHAIN_THREADS / 64 - 1) / (CHAIN_THREADS / 64);
+    wgs = (uint32_t)std::min<uint64_t>(wgs, perXcd * 8);
     wgs = std::max<uint32_t>(8u, wgs & ~7u);
     if (hipMemcpy(workspace, rows.data(), rows.size() * sizeof(ChainRow), hipMemcpyHostToDevice) != hipSuccess)
         return MVX_FAILURE;
@@ -446,8 +462,11 @@ extern "C" int mvx_ChainBatch_run(mvx_stream_t stream, const mvx_chain_plan_t *p
         (plan->workgroups & 7u))
         return MVX_ERROR_INVALID_PARAMETERS;
     if (plan->numTiles == 0) return MVX_SUCCESS;
-    hipLaunchKernelGGL(kKernels[plan->tile], dim3(plan->workgroups), dim3(kThreads[plan->tile]), 0, stream_of(stream),
-                       (const ChainRow *)plan->table, plan->count, plan->numTiles);
+    const uint32_t rows = rows_per_lane(plan->numTiles, plan->tile);
+    const uint64_t units = (uint64_t)(plan->numTiles / tiles_per_wave(plan->tile)) * ((uint32_t)kShapes[plan->tile].th / rows);
+    if (units > UINT32_MAX) return MVX_ERROR_INVALID_PARAMETERS;   // not a plan of mvx_ChainBatch_prepare
+    hipLaunchKernelGGL(kKernels[plan->tile], dim3(plan->workgroups), dim3(CHAIN_THREADS), 0, stream_of(stream),
+                       (const ChainRow *)plan->table, plan->count, (uint32_t)units, rows);
     MVX_LAUNCH_CHECK();
     return MVX_SUCCESS;
 }
