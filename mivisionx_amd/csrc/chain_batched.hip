@@ -330,14 +330,16 @@ constexpr ChainKernel kKernels[MVX_CHAIN_TILE_COUNT] = {k_chain_batch<16, 16>, k
 // tiles one wave takes side by side
 constexpr uint32_t tiles_per_wave(uint32_t tile) { return 64u / ((uint32_t)kShapes[tile].tw / 8u); }
 
-// Rows a lane streams: the tile's, halved down to 4 while the whole batch is fewer than 8192 waves (eight for each of
+// Rows a lane streams: the tile's, halved down to 2 while the whole batch is fewer than 8192 waves (eight for each of
 // the 1024 SIMDs, of which about four run at a time, so that no SIMD ends long after the others: 48 uneven images with
 // 64x32 tiles took 294 us at 2048, 283 at 8192); a lane's rows cost one more load and blur above and below them each.
+// A small batch is bound by the chain of a lane's rows, each a wait for memory: one 320x240 image 9.8 us with no fewer
+// than 4 rows, 6.7 with 2, 4096x2160 10.6 and 9.0.
 inline uint32_t rows_per_lane(uint32_t numTiles, uint32_t tile)
 {
     uint32_t rows = (uint32_t)kShapes[tile].th;
     uint64_t waves = numTiles / tiles_per_wave(tile);
-    while (rows > 4 && waves < 8192) { rows /= 2; waves *= 2; }
+    while (rows > 2 && waves < 8192) { rows /= 2; waves *= 2; }
     return rows;
 }
 
