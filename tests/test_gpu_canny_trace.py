@@ -73,3 +73,26 @@ def test_trace_stack_alignment(gpu, orc):
     rc = kernels().mvx_CannyEdgeTrace_U8_U8XY(None, w, h, p.ptr, p.stride,
                                               ctypes.c_void_p(base.data_ptr() + 2), w * h)
     assert rc == -10
+
+
+@pytest.mark.parametrize("w,h", [(63, 40), (64, 48), (65, 47), (79, 33), (250, 31), (257, 49), (400, 64)])
+def test_trace_leaves_other_bytes(gpu, orc, w, h):
+    """four tiles a wave, 16 bytes a load: bytes that are neither 127 nor 255 keep their value, and so does
+    whatever lies beside the image in the rows' padding (here 127 and 255, as a wider image would hold)"""
+    m = _random_map(w, h, 0.4, 0.01, w + h)
+    rng = np.random.default_rng(w)
+    other = (m == 0) & (rng.random((h, w)) < 0.3)
+    other[0, :] = other[-1, :] = other[:, 0] = other[:, -1] = False
+    junk = m.copy()
+    junk[other] = rng.choice([1, 126, 128, 254], int(other.sum()))
+    want = orc.canny_trace(m)
+    want[other] = junk[other]
+    p = Plane(w, h)
+    full = rng.choice([127, 255], (h, p.stride)).astype(np.uint8)
+    full[:, :w] = junk
+    p.t.copy_(torch.from_numpy(full))
+    stack = torch.zeros(w * h * 4, dtype=torch.uint8, device="cuda")
+    call("CannyEdgeTrace_U8_U8XY", w, h, p, p.stride, ctypes.c_void_p(stack.data_ptr()), w * h)
+    got = p.t.cpu().numpy()
+    assert_same(got[:, :w].copy(), want, f"trace with other bytes {w}x{h}")
+    assert_same(got[:, w:].copy(), full[:, w:].copy(), f"padding {w}x{h}")
