@@ -27,14 +27,18 @@ MVX_DEV int32_t mag_body(int32_t gx, int32_t gy)
 
 // Canny L2 magnitude of the reference's SSE loops (ago_haf_cpu_canny.cpp:646-1056): _mm_sqrt_ps of the
 // float sum, _mm_cvtps_epi32 (round half to even) and the unsigned 16-bit pack.  f >= 0 is an
-// integer-valued float below 2^32; sqrtf is the correctly rounded square root under this build's
-// -fhip-fp32-correctly-rounded-divide-sqrt, and rint the nearest-even conversion: the same operations
-// (checked for every such float by an exhaustive GPU probe).
-MVX_DEV int l2_pack_simd(float f)
+// integer-valued float below 2^32.  The square root is f times the hardware's reciprocal root with one
+// FMA correction from the exact remainder (Markstein's step), the rounding the one of adding 2^23: the same
+// integers as the correctly rounded sequence (checked for every such float by an exhaustive GPU probe).
+// The integer is the low 23 bits, at most 65536.
+MVX_DEV uint32_t l2_round(float f)
 {
-    const int k = __float2int_rn(sqrtf(f));
-    return k > 65535 ? 65535 : k;
+    const float g = fmaxf(f, 9.5367431640625e-7f);   // zero: a root of 2^-10 rounds to zero too
+    const float y = __builtin_amdgcn_rsqf(g), s = g * y;
+    return __float_as_uint(fmaf(fmaf(-s, s, g), 0.5f * y, s) + 8388608.f) & 0x7fffffu;
 }
+
+MVX_DEV int l2_pack_simd(float f) { return (int)min(l2_round(f), 65535u); }
 
 // Magnitude postfix rule (columns w & ~7 .. w-1), ago_haf_cpu_arithmetic.cpp:5087-5091:
 // (vx_int16)round(sqrtf((float)(gx*gx) + (float)(gy*gy))), float adds and sqrt correctly rounded.

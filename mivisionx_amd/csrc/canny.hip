@@ -11,6 +11,10 @@
 
 namespace mvx {
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_dword __attribute__((aligned(4)));   // at a 4-byte aligned address
+typedef uint32_t u32x2_dword __attribute__((ext_vector_type(2), aligned(4)));
+
 inline bool plane_ok_c(const void *p, uint32_t w, uint32_t stride, uint32_t bpp)
 {
     return p && aligned16(p) && (stride % 16u) == 0 && stride >= ((w * bpp + 15u) & ~15u);
@@ -28,81 +32,7 @@ MVX_DEV uint32_t canny_sector(int gx, int gy)
     return ret;
 }
 
-MVX_DEV uint16_t canny_pack(int gx, int gyn)
-{
-    int16_t t = (int16_t)(abs((int)(int16_t)gx) + abs((int)(int16_t)gyn));
-    t = (int16_t)(t << 2);
-    t = (int16_t)(t | (int16_t)(canny_sector((int16_t)gx, (int16_t)gyn) & 3u));
-    return (uint16_t)t;
-}
-
-// linear-address Sobel at (x, y) -> packed U16 (the reference's scalar loop, ago_haf_cpu_canny.cpp:120-131)
-MVX_DEV uint16_t canny_flat(const uint8_t *src, long n, long stride, int x, int y)
-{
-    const long c0 = (long)(y - 1) * stride + x, c1 = (long)y * stride + x, c2 = (long)(y + 1) * stride + x;
-    const int gx = ((int)ld_u8(src, n, c0 + 1) - (int)ld_u8(src, n, c0 - 1)) + ((int)ld_u8(src, n, c2 + 1) - (int)ld_u8(src, n, c2 - 1))
-                 + 2 * ((int)ld_u8(src, n, c1 + 1) - (int)ld_u8(src, n, c1 - 1));
-    const int gy = (int)ld_u8(src, n, c2 - 1) + (int)ld_u8(src, n, c2 + 1) - (int)ld_u8(src, n, c0 - 1) - (int)ld_u8(src, n, c0 + 1)
-                 + 2 * ((int)ld_u8(src, n, c2) - (int)ld_u8(src, n, c0));
-    return canny_pack((int16_t)gx, (int16_t)(-(int16_t)gy));
-}
-
-// CannySobel_U16_U8_3x3_L1NORM (ago_haf_cpu_canny.cpp:44-136), rows 1..h-2, widths >= 16.
-// Column 0 takes the SSE path's staged values: r0[-1] = 0 and r1[-1] = r0[ALIGN16(w)-1], i.e. this
-// row's vertical sum t0(w-1) when w is a multiple of 16, else 0.  Every other column equals the
-// linear-address Sobel (interior SSE columns read only in-row neighbours; the scalar loop redoes
-// columns aligned-1 .. w-1 with linear reads).
-__global__ void __launch_bounds__(256)
-k_canny_sobel(uint32_t w, uint32_t h, uint16_t *__restrict__ dst, uint32_t dstStride, const uint8_t *__restrict__ src,
-              uint32_t srcStride)
-{
-    const uint32_t x0 = (blockIdx.x * 256 + threadIdx.x) * 8;
-    const int y = 1 + (int)blockIdx.y;
-    if (x0 >= w || y >= (int)h - 1) return;
-    const long n = (long)h * srcStride;
-    uint16_t o[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int x = (int)x0 + i;
-        if (x >= (int)w) { o[i] = 0; continue; }
-        if (x == 0) {
-            const long bm = (long)(y - 1) * srcStride, b0 = (long)y * srcStride, bp = (long)(y + 1) * srcStride;
-            const int t0_1 = (int)src[bm + 1] + (int)src[bp + 1] + 2 * (int)src[b0 + 1];
-            const int t1_0 = (int)src[bp] - (int)src[bm];
-            const int t1_1 = (int)src[bp + 1] - (int)src[bm + 1];
-            const int t1_m1 = (w % 16 == 0) ? ((int)src[bm + w - 1] + (int)src[bp + w - 1] + 2 * (int)src[b0 + w - 1]) : 0;
-            o[i] = canny_pack(t0_1, -(t1_m1 + 2 * t1_0 + t1_1));
-        } else {
-            o[i] = canny_flat(src, n, srcStride, x, y);
-        }
-    }
-    uint16_t *d = (uint16_t *)((uint8_t *)dst + (long)y * dstStride) + x0;
-    if (x0 + 8 <= w) {
-        uint4 v;
-        v.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
-        v.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
-        v.z = (uint32_t)o[4] | ((uint32_t)o[5] << 16);
-        v.w = (uint32_t)o[6] | ((uint32_t)o[7] << 16);
-        *reinterpret_cast<uint4 *>(d) = v;
-    } else {
-        for (uint32_t i = 0; x0 + i < w; i++) d[i] = o[i];
-    }
-}
-
-// Widths below 16: the reference runs only its scalar loop, from x = -1 (it writes the U16 slot just
-// before each row, i.e. the last slot of the previous row's stride), rows in order.  One thread
-// replays that order exactly; these planes are at most 15 pixels wide.
-__global__ void k_canny_sobel_narrow(uint32_t w, uint32_t h, uint16_t *dst, uint32_t dstStride, const uint8_t *src,
-                                     uint32_t srcStride)
-{
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    const long n = (long)h * srcStride;
-    for (int y = 1; y < (int)h - 1; y++)
-        for (int x = -1; x < (int)w; x++)
-            *(uint16_t *)((uint8_t *)dst + (long)y * dstStride + 2L * x) = canny_flat(src, n, srcStride, x, y);
-}
-
-// ---- gradient 5 / 7 and L2 Sobel planes (ago_haf_cpu_canny.cpp:145-427, 646-1056) -------------------
+// ---- Sobel planes, gradients 3, 5, 7, norms L1 and L2 (ago_haf_cpu_canny.cpp:44-427, 646-1056) -------------------
 // 16-bit lane arithmetic of the reference's SSE code
 MVX_DEV int w16(int v) { return (int16_t)(uint16_t)(uint32_t)v; }
 MVX_DEV int s16(int v) { return min(max(v, -32768), 32767); }
@@ -152,7 +82,7 @@ template <int G, bool L2> MVX_DEV uint16_t canny_scalar(const uint8_t *src, long
     }
     const int gx = w16(gxs);
     int gy = w16(gys);
-    if (G == 5 && !L2) gy = w16(-gy);
+    if (G <= 5 && !L2) gy = w16(-gy);
     const int mag = L2 ? l2_scalar(gx, gy) : w16(abs(gx) + abs(gy));
     return canny_out(mag, canny_sector(gx, gy));
 }
@@ -165,11 +95,9 @@ template <int G, bool L2> MVX_DEV uint16_t canny_scalar(const uint8_t *src, long
 // registers (all of the strip's rows are loaded first); its two vertical sums reach the neighbouring lanes by DPP
 // lane shifts, so no LDS and no barrier is involved.  Lanes R .. 63-R finish one column each; columns
 // aligned-1 .. w-1 take the scalar loop's value.
-// Short waves: a wave's rows are one chain of loads and dependent arithmetic, and many short waves keep
-// more of the image in flight than a few long ones (3840x2160, gradient 5, L2: 2 rows per wave 28 us,
-// 4 rows 29 us, 8 rows 35 us, 16 rows 50 us; 8 strips per workgroup 28 us, 4 strips 36 us).
-constexpr int CSW_ROWS = 2;    // output rows per wave
-constexpr int CSW_WAVES = 8;   // strips (waves) per workgroup
+// Only columns 0 .. 7 and those from aligned - 8 on need that (k_canny_sobel_g's edge waves); between them a
+// window's slots are all in the row, and lanes own 8 columns (canny_columns).
+constexpr int CSW_ROWS = 1;    // output rows per edge wave
 
 // which scratch value a slot holds: kind 1 = (r0, r1) of source column sc, 2 = r0 <- r1 of sc (the slot
 // lies past the end of r0), 3 = r1 <- r0 of sc (before the start of r1), 0 = zeros
@@ -244,22 +172,22 @@ template <int G, bool L2> MVX_DEV uint16_t canny_simd_px(const int (&a0)[G], con
     return canny_out(mag, canny_sector(gx, gy));
 }
 
-// one strip: EDGE strips hold slots outside [0, aligned) or columns from aligned - 1 on
-template <int G, bool L2, bool EDGE>
+// one strip: output columns xs .. xe - 1 (at most 64 - 2R), rows yb .. ye - 1
+template <int G, bool L2>
 MVX_DEV void canny_strip(uint32_t w, uint32_t h, uint16_t *dst, uint32_t dstStride, const uint8_t *src, uint32_t srcStride,
-                         int xs, int yb, int ye)
+                         int xs, int xe, int yb, int ye)
 {
     constexpr int R = G / 2;
     const int lane = (int)threadIdx.x & 63;
     const int aligned = (int)(w & ~15u), a16 = (int)((w + 15u) & ~15u);
     const int col = xs - R + lane;
     int sc = col;
-    const int kind = EDGE ? canny_slot(col, aligned, a16, sc) : 1;
+    const int kind = canny_slot(col, aligned, a16, sc);
     const __amdgpu_buffer_rsrc_t sR = plane_rsrc(src), dR = plane_rsrc(dst);
     // a zero slot still loads an in-plane byte (column 0) and drops it, so the loads stay unconditional
     auto load = [&](int r) -> int {
         const int v = (int)__builtin_amdgcn_raw_buffer_load_b8(sR, sc, (int)((uint32_t)r * srcStride), 0);
-        return (EDGE && kind == 0) ? 0 : v;
+        return kind == 0 ? 0 : v;
     };
     // every source row of the strip is loaded before the first is used: the loads are all in flight
     // together, and row i waits only for its own G rows
@@ -268,7 +196,7 @@ MVX_DEV void canny_strip(uint32_t w, uint32_t h, uint16_t *dst, uint32_t dstStri
 #pragma unroll
     for (int j = 0; j < NR; j++) rw[j] = (yb - R + j < ye + R) ? load(yb - R + j) : 0;
     const int x = col;   // output column of lanes R .. 63 - R
-    const bool outLane = lane >= R && lane < 64 - R && x < (int)w;
+    const bool outLane = lane >= R && lane < 64 - R && x < xe;
 #pragma unroll
     for (int i = 0; i < CSW_ROWS; i++) {
         const int y = yb + i;
@@ -279,12 +207,8 @@ MVX_DEV void canny_strip(uint32_t w, uint32_t h, uint16_t *dst, uint32_t dstStri
         int t0, t1;
         canny_vsum<G>(win, t0, t1);
         int a0[G], a1[G];
-        a0[R] = t0;
-        a1[R] = t1;
-        if (EDGE) {
-            a0[R] = kind == 1 ? t0 : kind == 2 ? t1 : 0;
-            a1[R] = kind == 1 ? t1 : kind == 3 ? t0 : 0;
-        }
+        a0[R] = kind == 1 ? t0 : kind == 2 ? t1 : 0;
+        a1[R] = kind == 1 ? t1 : kind == 3 ? t0 : 0;
         // the lane shifts run with every lane active
 #pragma unroll
         for (int d = 1; d <= R; d++) {
@@ -295,26 +219,186 @@ MVX_DEV void canny_strip(uint32_t w, uint32_t h, uint16_t *dst, uint32_t dstStri
         }
         uint16_t out = canny_simd_px<G, L2>(a0, a1);
         if (outLane) {
-            if (EDGE && x >= aligned - 1) out = canny_scalar<G, L2>(src, (long)h * srcStride, srcStride, x, y);
+            if (x >= aligned - 1) out = canny_scalar<G, L2>(src, (long)h * srcStride, srcStride, x, y);
             __builtin_amdgcn_raw_buffer_store_b16(out, dR, 2 * x, (int)((uint32_t)y * dstStride), 0);
         }
     }
 }
 
-template <int G, bool L2>
-__global__ void __launch_bounds__(64 * CSW_WAVES)
-k_canny_sobel_g(uint32_t w, uint32_t h, uint16_t *__restrict__ dst, uint32_t dstStride, const uint8_t *__restrict__ src,
-                uint32_t srcStride, uint32_t strips)
+// Eight columns of a lane: x0 .. x0+7 with 8 <= x0 and x0 + 16 <= aligned, CSC_ROWS rows down.  A lane loads the
+// 16 bytes from x0 - 4 on of each row, so that no lane waits for another; sums are pairs of 16-bit columns, the
+// even ones of four columns k and the odd ones (E_k, O_k), and the pairs one or two columns on are shifts by half
+// a register.  Every sum but the gradient-7 ones' last is exact in 16 bits, that one saturates as the SSE code's
+// does; the rest of a pixel is a few float operations.
+typedef short i16x2 __attribute__((ext_vector_type(2)));
+
+MVX_DEV i16x2 i16_pair(uint32_t v) { return __builtin_bit_cast(i16x2, v); }
+MVX_DEV uint32_t bits_of(i16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+MVX_DEV i16x2 pair_shift(i16x2 a, i16x2 b) { return i16_pair(__builtin_amdgcn_alignbit(bits_of(b), bits_of(a), 16)); }
+MVX_DEV i16x2 pair_abs(i16x2 v) { return __builtin_elementwise_max(v, (i16x2)(0 - v)); }
+
+// pairs of 2 and of 4 that the compiler cannot see through: it would split a multiply-add by them into a shift
+// and an add, two instructions for one
+struct CannyMul { i16x2 two, four; };
+MVX_DEV CannyMul canny_mul()
 {
-    constexpr int R = G / 2, CW = 64 - 2 * R;
-    const int strip = (int)blockIdx.x * CSW_WAVES + ((int)threadIdx.x >> 6);
-    if (strip >= (int)strips) return;   // the whole wave
-    const int yb = R + (int)blockIdx.y * CSW_ROWS, ye = min(yb + CSW_ROWS, (int)h - R);
-    const int xs = strip * CW, aligned = (int)(w & ~15u);
-    if (xs - R < 0 || xs - R + 63 >= aligned)
-        canny_strip<G, L2, true>(w, h, dst, dstStride, src, srcStride, xs, yb, ye);
-    else
-        canny_strip<G, L2, false>(w, h, dst, dstStride, src, srcStride, xs, yb, ye);
+    uint32_t two = 0x00020002u, four = 0x00040004u;
+    asm("" : "+s"(two), "+s"(four));
+    return {i16_pair(two), i16_pair(four)};
+}
+
+// canny_vsum for two columns
+template <int G> MVX_DEV void canny_vsum2(const i16x2 (&s)[G], const CannyMul &k, i16x2 &t0, i16x2 &t1)
+{
+    if constexpr (G == 3) {
+        t0 = s[1] * k.two + (s[0] + s[2]);
+        t1 = s[2] - s[0];
+    } else if constexpr (G == 5) {
+        t0 = s[2] * (short)6 + ((s[1] + s[3]) * k.four + (s[0] + s[4]));
+        t1 = (s[3] - s[1]) * k.two + (s[4] - s[0]);
+    } else {
+        t0 = ((s[0] + s[G - 1]) + (s[1] + s[G - 2]) * (short)6 + (s[2] + s[G - 3]) * (short)15 + s[G / 2] * (short)20) >> (short)2;
+        t1 = ((s[G - 1] - s[0]) + (s[G - 2] - s[1]) * k.four + (s[G - 3] - s[2]) * (short)5) >> (short)2;
+    }
+}
+
+// the gradients of a pair of columns from the pairs at columns -R .. R of it (canny_simd_px's, gy's sign included)
+template <int G> MVX_DEV void canny_grad2(const i16x2 (&a0)[G], const i16x2 (&a1)[G], const CannyMul &k, i16x2 &gx, i16x2 &gy)
+{
+    if constexpr (G == 3) {
+        gx = a0[2] - a0[0];
+        gy = (short)0 - (a1[1] * k.two + (a1[0] + a1[2]));
+    } else if constexpr (G == 5) {
+        gx = (a0[3] - a0[1]) * k.two + (a0[4] - a0[0]);
+        gy = (short)0 - (a1[2] * (short)6 + ((a1[1] + a1[3]) * k.four + (a1[0] + a1[4])));
+    } else {
+        gx = __builtin_elementwise_add_sat((i16x2)((a0[G - 2] - a0[1]) * k.four + (a0[G - 1] - a0[0])),
+                                           (i16x2)((a0[G - 3] - a0[2]) * (short)5));
+        const i16x2 v = __builtin_elementwise_add_sat((i16x2)((a1[1] + a1[G - 2]) * (short)6 + a1[G / 2] * (short)20 + (a1[0] + a1[G - 1])),
+                                                      (i16x2)((a1[2] + a1[G - 3]) * (short)15));
+        gy = __builtin_elementwise_sub_sat((i16x2)(short)0, v);
+    }
+}
+
+// a pixel's sector (canny_sector) given 3 or 1 for gx * gy negative or not
+MVX_DEV uint32_t canny_sector_f(float fx, float fy, uint32_t diagonal)
+{
+    uint32_t ret = fabsf(fy) <= fabsf(fx) * 0.4142135623730950488016887242097f ? 0u : diagonal;
+    return fabsf(fy) >= fabsf(fx) * 2.4142135623730950488016887242097f ? 2u : ret;
+}
+
+template <int G, bool L2> MVX_DEV uint32_t canny_pair(i16x2 gx, i16x2 gy)
+{
+    // where one of the two is zero the sector is 0 or 2 whatever the signs
+    const uint32_t diag = (((bits_of(gx) ^ bits_of(gy)) >> 14) & 0x00020002u) | 0x00010001u;
+    const uint32_t sec = canny_sector_f((float)gx.x, (float)gy.x, diag & 0xffffu) | (canny_sector_f((float)gx.y, (float)gy.y, diag >> 16) << 16);
+    uint32_t mag;
+    if (L2) {
+        uint32_t m0, m1;
+        if (G == 3) {   // the squares wrap at 16 bits
+            const u16x2 xx = pair_of(bits_of(gx)) * pair_of(bits_of(gx)), yy = pair_of(bits_of(gy)) * pair_of(bits_of(gy));
+            m0 = l2_round((float)xx.x + (float)yy.x);
+            m1 = l2_round((float)xx.y + (float)yy.y);
+        } else {
+            const i16x2 p0 = i16_pair(__builtin_amdgcn_perm(bits_of(gy), bits_of(gx), 0x05040100u));
+            const i16x2 p1 = i16_pair(__builtin_amdgcn_perm(bits_of(gy), bits_of(gx), 0x07060302u));
+            m0 = l2_round((float)__builtin_amdgcn_sdot2(p0, p0, 0, false));
+            m1 = l2_round((float)__builtin_amdgcn_sdot2(p1, p1, 0, false));
+        }
+        mag = __builtin_amdgcn_perm(m1, m0, 0x05040100u);   // at most 46341: no saturation
+    } else {
+        i16x2 m = pair_abs(gx) + pair_abs(gy);
+        if (G == 7) m = __builtin_elementwise_min(m, (i16x2)(short)0x3fff);
+        mag = bits_of(m);
+    }
+    return bits_of((u16x2)(pair_of(mag) << (unsigned short)2)) | sec;
+}
+
+constexpr int CSC_ROWS = 4;    // output rows per lane
+
+template <int G, bool L2>
+MVX_DEV void canny_columns(uint32_t h, uint16_t *dst, uint32_t dstStride, const uint8_t *src, uint32_t srcStride, uint32_t x0, uint32_t rowGroup)
+{
+    constexpr int R = G / 2;
+    const int yb = R + (int)rowGroup * CSC_ROWS, last = (int)h - 1;
+    gptr_t<const uint8_t> p = gmem(src) + (x0 - 4);
+    u32x4 raw[CSC_ROWS + 2 * R];
+#pragma unroll
+    for (int j = 0; j < CSC_ROWS + 2 * R; j++) raw[j] = *(gptr_t<const u32x4_dword>)(p + (uint64_t)(uint32_t)min(yb - R + j, last) * srcStride);
+    // here all rows have arrived: left alone the compiler moves some of the loads down to their first use
+#pragma unroll
+    for (int j = 0; j < CSC_ROWS + 2 * R; j++) asm volatile("" : "+v"(raw[j]));
+    const CannyMul mul = canny_mul();
+    i16x2 win[G][8];   // the rows' columns: [2k] = E_k, [2k + 1] = O_k
+#pragma unroll
+    for (int j = 0; j < CSC_ROWS + 2 * R; j++) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            win[j % G][2 * k] = i16_pair(bits_of(even_bytes(raw[j][k])));
+            win[j % G][2 * k + 1] = i16_pair(bits_of(odd_bytes(raw[j][k])));
+        }
+        if (j < 2 * R) continue;
+        const int y = yb + j - 2 * R;
+        i16x2 t0[8], t1[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            i16x2 s[G];
+#pragma unroll
+            for (int i = 0; i < G; i++) s[i] = win[(j + 1 + i) % G][c];   // oldest first
+            canny_vsum2<G>(s, mul, t0[c], t1[c]);
+        }
+        uint32_t out[4];
+#pragma unroll
+        for (int c = 2; c < 6; c++) {   // E_1, O_1, E_2, O_2
+            // the pair d columns on of E_k (c even) or O_k: O_k's columns are one on from E_k's
+            const auto at = [&](const i16x2 (&t)[8], int d) -> i16x2 {
+                const int n = (c & 1) + d, k = c / 2;       // columns from E_k
+                const int q = n & 1, m = (n - q) / 2;       // pair kind (even or odd), half pairs on
+                const int i = 2 * (k + (m - (m & 1)) / 2) + q;
+                return (m & 1) ? pair_shift(t[i], t[i + 2]) : t[i];
+            };
+            i16x2 a0[G], a1[G];
+#pragma unroll
+            for (int d = -R; d <= R; d++) {
+                a0[R + d] = at(t0, d);
+                a1[R + d] = at(t1, d);
+            }
+            i16x2 gx, gy;
+            canny_grad2<G>(a0, a1, mul, gx, gy);
+            out[c - 2] = canny_pair<G, L2>(gx, gy);
+        }
+        u32x4 o;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            o[2 * k] = __builtin_amdgcn_perm(out[2 * k + 1], out[2 * k], 0x05040100u);
+            o[2 * k + 1] = __builtin_amdgcn_perm(out[2 * k + 1], out[2 * k], 0x07060302u);
+        }
+        // the rows past the last are computed and dropped: a branch around them would hold their loads back
+        if (y <= last - R) *(gptr_t<u32x4>)((gptr_t<uint8_t>)gmem(dst) + (uint64_t)(uint32_t)y * dstStride + 2 * x0) = o;
+    }
+}
+
+// The first `edge` workgroups' waves take the left and right edge of CSW_ROWS rows each (first, since theirs are the
+// longest chains); the others 8-column units of the columns between, row group after row group.
+// 3840x2160, gradient 5, L2: 30.5 us with a lane a column and shifts between lanes (83 lane operations a pixel), 18.0 now
+// (41): half of it vector instructions, the rest the waits for memory at either end of four rows.
+template <int G, bool L2>
+__global__ void __launch_bounds__(256)
+k_canny_sobel_g(uint32_t w, uint32_t h, uint16_t *__restrict__ dst, uint32_t dstStride, const uint8_t *__restrict__ src,
+                uint32_t srcStride, uint32_t edge, uint32_t units, uint32_t rowGroups)
+{
+    constexpr int R = G / 2;
+    const uint32_t aligned = w & ~15u;
+    if (blockIdx.x >= edge) {
+        const uint32_t u = (blockIdx.x - edge) * 256 + threadIdx.x, g = u / units;
+        if (g < rowGroups) canny_columns<G, L2>(h, dst, dstStride, src, srcStride, 8 + 8 * (u - g * units), g);
+        return;
+    }
+    const int e = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int yb = R + (e >> 1) * CSW_ROWS, ye = min(yb + CSW_ROWS, (int)h - R);
+    if (yb >= ye) return;
+    if (e & 1) canny_strip<G, L2>(w, h, dst, dstStride, src, srcStride, (int)aligned - 8, (int)w, yb, ye);
+    else canny_strip<G, L2>(w, h, dst, dstStride, src, srcStride, 0, 8, yb, ye);
 }
 
 // widths below 16: only the scalar loop runs, from x = -1 (the slot before each row), rows in order
@@ -485,9 +569,6 @@ struct CtArgs {
     uint16_t *border;   // tiles * 2 * CT_NB: top row, bottom row (CT_W each), left, right column (CT_H each), seeds (CT_NB)
     uint32_t *ucount;   // tiles: undecided components of the tile
 };
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_dword __attribute__((ext_vector_type(2), aligned(4)));   // at a 4-byte aligned address
 
 // a lane's row of its tile; lanes past the image hold no pixel
 struct CtRow {
@@ -784,9 +865,10 @@ int canny_sobel_g(mvx_stream_t stream, uint32_t w, uint32_t h, uint16_t *dst, ui
     if (w < 16) {
         hipLaunchKernelGGL((k_canny_sobel_g_narrow<G, L2>), dim3(1), dim3(64), 0, stream_of(stream), w, h, dst, dstStride, src, srcStride);
     } else {
-        const uint32_t strips = (w + (64 - 2 * (G / 2)) - 1) / (64 - 2 * (G / 2));
-        hipLaunchKernelGGL((k_canny_sobel_g<G, L2>), dim3((strips + CSW_WAVES - 1) / CSW_WAVES, (h - 2 * (G / 2) + CSW_ROWS - 1) / CSW_ROWS),
-                           dim3(64 * CSW_WAVES), 0, stream_of(stream), w, h, dst, dstStride, src, srcStride, strips);
+        const uint32_t rows = h - 2 * (G / 2), units = ((w & ~15u) - 16) / 8, rowGroups = (rows + CSC_ROWS - 1) / CSC_ROWS;
+        const uint32_t inner = (uint32_t)(((uint64_t)units * rowGroups + 255) / 256), edge = ((rows + CSW_ROWS - 1) / CSW_ROWS + 1) / 2;
+        hipLaunchKernelGGL((k_canny_sobel_g<G, L2>), dim3(inner + edge), dim3(256), 0, stream_of(stream), w, h, dst, dstStride, src,
+                           srcStride, edge, units, rowGroups);
     }
     MVX_LAUNCH_CHECK();
     return MVX_SUCCESS;
@@ -799,28 +881,13 @@ int canny_sobel_g(mvx_stream_t stream, uint32_t w, uint32_t h, uint16_t *dst, ui
     {                                                                                                                     \
         return canny_sobel_g<G, L2>(stream, w, h, dst, dstStride, src, srcStride);                                         \
     }
+MVX_CANNY_SOBEL(mvx_CannySobel_U16_U8_3x3_L1NORM, 3, false)
 MVX_CANNY_SOBEL(mvx_CannySobel_U16_U8_5x5_L1NORM, 5, false)
 MVX_CANNY_SOBEL(mvx_CannySobel_U16_U8_7x7_L1NORM, 7, false)
 MVX_CANNY_SOBEL(mvx_CannySobel_U16_U8_3x3_L2NORM, 3, true)
 MVX_CANNY_SOBEL(mvx_CannySobel_U16_U8_5x5_L2NORM, 5, true)
 MVX_CANNY_SOBEL(mvx_CannySobel_U16_U8_7x7_L2NORM, 7, true)
 #undef MVX_CANNY_SOBEL
-
-extern "C" int mvx_CannySobel_U16_U8_3x3_L1NORM(mvx_stream_t stream, uint32_t w, uint32_t h, uint16_t *dst,
-                                                uint32_t dstStride, const uint8_t *src, uint32_t srcStride)
-{
-    if (w == 0 || h == 0) return MVX_SUCCESS;
-    if (!plane_ok_c(dst, w, dstStride, 2) || !plane_ok_c(src, w, srcStride, 1)) return MVX_ERROR_INVALID_PARAMETERS;
-    if (h < 3) return MVX_SUCCESS;
-    if (w < 16) {
-        hipLaunchKernelGGL(k_canny_sobel_narrow, dim3(1), dim3(64), 0, stream_of(stream), w, h, dst, dstStride, src, srcStride);
-    } else {
-        dim3 grid(((w + 7) / 8 + 255) / 256, h - 2);
-        hipLaunchKernelGGL(k_canny_sobel, grid, dim3(256), 0, stream_of(stream), w, h, dst, dstStride, src, srcStride);
-    }
-    MVX_LAUNCH_CHECK();
-    return MVX_SUCCESS;
-}
 
 extern "C" int mvx_CannySuppThreshold_U8XY_U16_3x3(mvx_stream_t stream, uint32_t w, uint32_t h, uint8_t *dst,
                                                    uint32_t dstStride, const uint16_t *mag, uint32_t magStride,

@@ -72,3 +72,16 @@ def test_canny_node_variants(gpu, orc, w, h, g, l2):
     finally:
         cc = ctypes.c_void_p(ctx)
         L.vxReleaseContext(ctypes.byref(cc))
+
+
+@pytest.mark.parametrize("w,h", [(16, 9), (17, 12), (24, 8), (31, 10), (32, 7), (33, 11), (47, 13), (512, 14), (1283, 10)])
+@pytest.mark.parametrize("g,l2", [(3, 0)] + VARIANTS)
+def test_canny_sobel_edge_and_column_units(gpu, orc, w, h, g, l2):
+    """widths around one, two and three 16-column blocks (edge columns only, then the first 8-column units between
+    them), rows that do not fill a lane's four; 0/255 noise reaches the gradient-7 sums' saturation"""
+    src = (synth.uniform_u8(w, h, 5 * w + h) >= 128).astype(np.uint8) * 255
+    s = Plane.from_array(src)
+    d = Plane(w, h, "U16")
+    call(f"CannySobel_U16_U8_{g}x{g}_{'L2' if l2 else 'L1'}NORM", w, h, d, d.stride, s, s.stride)
+    got = d.t.cpu().numpy().view(np.uint16)
+    assert_same(got, orc.canny_sobel_ex(src, g, l2, padded=True), f"canny sobel units {g} l2={l2} {w}x{h}")
