@@ -85,3 +85,18 @@ def test_canny_sobel_edge_and_column_units(gpu, orc, w, h, g, l2):
     call(f"CannySobel_U16_U8_{g}x{g}_{'L2' if l2 else 'L1'}NORM", w, h, d, d.stride, s, s.stride)
     got = d.t.cpu().numpy().view(np.uint16)
     assert_same(got, orc.canny_sobel_ex(src, g, l2, padded=True), f"canny sobel units {g} l2={l2} {w}x{h}")
+
+
+@pytest.mark.parametrize("w,h", [(3, 3), (8, 4), (9, 7), (10, 8), (17, 6), (64, 11), (333, 77)])
+@pytest.mark.parametrize("lower,upper", [(0, 0), (100, 3000), (-1, 50), (-5, -2), (16382, 16383), (16383, 40000), (3000, 100)])
+def test_canny_supp_pairs(gpu, orc, w, h, lower, upper):
+    """the suppression's packed comparisons: every sector, equal neighbours, magnitudes up to 14 bits, thresholds below
+    0, at and past the largest magnitude, and in the wrong order"""
+    rng = np.random.default_rng(w * h + lower)
+    mag = np.where(rng.random((h, w)) < 0.5, rng.integers(0, 65536, (h, w)), rng.integers(0, 4, (h, w)) * 4096 + rng.integers(0, 4, (h, w)))
+    mag = mag.astype(np.uint16)
+    m, d = Plane.from_array(mag, "U16"), Plane(w, h)
+    stack = torch.zeros(w * h * 4, dtype=torch.uint8, device="cuda")
+    call("CannySuppThreshold_U8XY_U16_3x3", w, h, d, d.stride, m, m.stride, ctypes.c_void_p(stack.data_ptr()), w * h,
+         lower & 0xffffffff, upper & 0xffffffff)
+    assert_same(d.download(), orc.canny_supp_threshold(mag, lower, upper)[0], f"canny supp {w}x{h} {lower} {upper}")
