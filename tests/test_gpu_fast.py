@@ -124,3 +124,15 @@ def test_fast_unaligned_source(gpu, orc, nonmax):
     want, wc = orc.fast(src, 20.0, nonmax, 5000)
     assert int(num.item()) == wc and n == len(want)
     assert np.array_equal(kp.view(np.uint8), want.view(np.uint8))
+
+
+@pytest.mark.parametrize("w,h", [(4096, 9), (4112, 8), (4100, 10), (4099, 9), (20, 1030), (19, 1029), (16, 1031)])
+def test_fast_write_rows(gpu, orc, w, h):
+    """rows at and past the 4096 columns one sweep of a row's workgroup covers, with and without whole words, and more
+    rows than one load of the counts above covers; most pixels are corners"""
+    src = synth.uniform_u8(w, h, w + h)
+    for nonmax in (0, 1):
+        kp, n, total = _run(src, 1.0, nonmax, 3 * w * h // 4)
+        want, wc = orc.fast(src, 1.0, nonmax, 3 * w * h // 4)
+        assert total == wc and n == len(want) and n > 0
+        assert np.array_equal(kp.view(np.uint8), want.view(np.uint8))
