@@ -398,33 +398,83 @@ k_extract_u8(uint32_t w, uint32_t h, uint8_t *__restrict__ dst, uint32_t dstStri
 // ------------------------------------------------------------------ ColorConvert RGB <- YUV ------
 // HafCpu_ColorConvert_RGB_IYUV / _RGB_NV12 (ago_haf_cpu_color_convert.cpp:472-768), BT.709: one chroma
 // sample per 2x2 block, u = U - 128, v = V - 128; R = Y + v*1.5748, G = Y - (u*0.1873 + v*0.4681),
-// B = Y + u*1.8556, each truncated and clamped to [0, 255].  One thread: 4 consecutive pixels of a row.
-template <bool NV12>
+// B = Y + u*1.8556, each truncated and clamped to [0, 255].
+MVX_DEV void rgb_of_chroma(float U, float V, float &R, float &G, float &B)
+{
+    G = (U * 0.1873f) + (V * 0.4681f);
+    R = V * 1.5748f;
+    B = U * 1.8556f;
+}
+MVX_DEV uint32_t rgb_byte(float f) { return (uint32_t)fminf(fmaxf(f, 0.0f), 255.0f); }
+
+// One thread: 8 columns of 2 rows, their chroma read and scaled once.  Where every plane and stride is a multiple of
+// 4 bytes (DWORDS) and the 8 columns are in the image it loads and stores words, else bytes.
+// Bound by memory at large sizes, by latency at small ones.  NV12, a byte at a time and 4 pixels a thread against now:
+// 1920x1080 7.0 and 4.3 us, 3840x2160 18.7 and 8.8 us.
+typedef uint32_t rgb_u32x2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t rgb_u32x3 __attribute__((ext_vector_type(3), aligned(4)));
+
+template <bool NV12, bool DWORDS>
 __global__ void __launch_bounds__(256)
 k_rgb_from_yuv(uint32_t w, uint32_t h, uint8_t *__restrict__ dst, uint32_t dstStride, const uint8_t *__restrict__ ys, uint32_t yStride,
                const uint8_t *__restrict__ us, uint32_t uStride, const uint8_t *__restrict__ vs, uint32_t vStride)
 {
-    const uint32_t x0 = (blockIdx.x * 256 + threadIdx.x) * 4, r = blockIdx.y;
-    if (x0 >= w || r >= h) return;
-    uint8_t *d = dst + (size_t)r * dstStride + 3ull * x0;
-#pragma unroll
-    for (uint32_t k = 0; k < 4; k++) {
-        const uint32_t x = x0 + k;
-        if (x >= w) break;
-        const float Y = (float)ys[(size_t)r * yStride + x];
-        float U, V;
+    const uint32_t x0 = (blockIdx.x * 64 + threadIdx.x) * 8, r2 = blockIdx.y * 4 + threadIdx.y;
+    if (x0 >= w || 2 * r2 >= h) return;
+    const uint32_t cols = min(w - x0, 8u);   // w and h are even
+    const uint8_t *y[2] = {ys + (size_t)(2 * r2) * yStride + x0, ys + (size_t)(2 * r2 + 1) * yStride + x0};
+    const uint8_t *u = us + (size_t)r2 * uStride + (NV12 ? x0 : x0 / 2), *v = NV12 ? u + 1 : vs + (size_t)r2 * vStride + x0 / 2;
+    uint8_t *d[2] = {dst + (size_t)(2 * r2) * dstStride + 3ull * x0, dst + (size_t)(2 * r2 + 1) * dstStride + 3ull * x0};
+    if (DWORDS && cols == 8) {
+        const rgb_u32x2 Y[2] = {*(const rgb_u32x2 *)y[0], *(const rgb_u32x2 *)y[1]};
+        uint32_t c[2];   // U0 V0 U1 V1, ..
         if (NV12) {
-            const uint8_t *c = us + (size_t)(r / 2) * uStride + 2 * (x / 2);
-            U = (float)c[0] - 128.0f;
-            V = (float)c[1] - 128.0f;
+            const rgb_u32x2 q = *(const rgb_u32x2 *)u;
+            c[0] = q.x;
+            c[1] = q.y;
         } else {
-            U = (float)us[(size_t)(r / 2) * uStride + x / 2] - 128.0f;
-            V = (float)vs[(size_t)(r / 2) * vStride + x / 2] - 128.0f;
+            const uint32_t U = *(const uint32_t *)u, V = *(const uint32_t *)v;
+            c[0] = __builtin_amdgcn_perm(V, U, 0x05010400u);
+            c[1] = __builtin_amdgcn_perm(V, U, 0x07030602u);
         }
-        const float G = (U * 0.1873f) + (V * 0.4681f), R = V * 1.5748f, B = U * 1.8556f;
-        d[3 * k + 0] = (uint8_t)fminf(fmaxf(Y + R, 0.0f), 255.0f);
-        d[3 * k + 1] = (uint8_t)fminf(fmaxf(Y - G, 0.0f), 255.0f);
-        d[3 * k + 2] = (uint8_t)fminf(fmaxf(Y + B, 0.0f), 255.0f);
+        float R[4], G[4], B[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t q = c[i >> 1] >> (16 * (i & 1));
+            rgb_of_chroma((float)(q & 0xffu) - 128.0f, (float)((q >> 8) & 0xffu) - 128.0f, R[i], G[i], B[i]);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+#pragma unroll
+            for (int k = 0; k < 2; k++) {   // four columns: twelve bytes
+                uint32_t o[12];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float f = (float)((Y[j][k] >> (8 * i)) & 0xffu);
+                    const int m = 2 * k + i / 2;
+                    o[3 * i] = rgb_byte(f + R[m]);
+                    o[3 * i + 1] = rgb_byte(f - G[m]);
+                    o[3 * i + 2] = rgb_byte(f + B[m]);
+                }
+                rgb_u32x3 q;
+#pragma unroll
+                for (int i = 0; i < 3; i++) q[i] = o[4 * i] | (o[4 * i + 1] << 8) | (o[4 * i + 2] << 16) | (o[4 * i + 3] << 24);
+                *(rgb_u32x3 *)(d[j] + 12 * k) = q;
+            }
+        }
+        return;
+    }
+    for (uint32_t k = 0; k < cols; k++) {
+        const uint32_t c = NV12 ? (k & ~1u) : k / 2;
+        float R, G, B;
+        rgb_of_chroma((float)u[c] - 128.0f, (float)v[c] - 128.0f, R, G, B);
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float f = (float)y[j][k];
+            d[j][3 * k + 0] = (uint8_t)rgb_byte(f + R);
+            d[j][3 * k + 1] = (uint8_t)rgb_byte(f - G);
+            d[j][3 * k + 2] = (uint8_t)rgb_byte(f + B);
+        }
     }
 }
 
@@ -441,13 +491,11 @@ int rgb_from_yuv(mvx_stream_t stream, uint32_t w, uint32_t h, uint8_t *dst, uint
     if (!dst || !y || !u || (!nv12 && !v) || dstStride < 3 * w || yStride < w || uStride < (nv12 ? w : w / 2) ||
         (!nv12 && vStride < w / 2))
         return MVX_ERROR_INVALID_PARAMETERS;
-    dim3 grid(((w + 3) / 4 + 255) / 256, h);
-    if (nv12)
-        hipLaunchKernelGGL(k_rgb_from_yuv<true>, grid, dim3(256), 0, stream_of(stream), w, h, dst, dstStride, y, yStride, u, uStride, u,
-                           uStride);
-    else
-        hipLaunchKernelGGL(k_rgb_from_yuv<false>, grid, dim3(256), 0, stream_of(stream), w, h, dst, dstStride, y, yStride, u, uStride, v,
-                           vStride);
+    const bool dwords = (((uintptr_t)dst | dstStride | (uintptr_t)y | yStride | (uintptr_t)u | uStride | (nv12 ? 0 : (uintptr_t)v | vStride)) & 3u) == 0;
+    const auto kernel = nv12 ? (dwords ? k_rgb_from_yuv<true, true> : k_rgb_from_yuv<true, false>)
+                             : (dwords ? k_rgb_from_yuv<false, true> : k_rgb_from_yuv<false, false>);
+    hipLaunchKernelGGL(kernel, dim3((w + 511) / 512, (h / 2 + 3) / 4), dim3(64, 4), 0, stream_of(stream), w, h, dst, dstStride, y, yStride, u,
+                       uStride, nv12 ? u : v, nv12 ? uStride : vStride);
     MVX_LAUNCH_CHECK();
     return MVX_SUCCESS;
 }

@@ -67,3 +67,30 @@ def test_yuv_nodes(gpu, orc):
     finally:
         cc = ctypes.c_void_p(ctx)
         L.vxReleaseContext(ctypes.byref(cc))
+
+
+@pytest.mark.parametrize("w,h", [(2, 2), (6, 4), (8, 2), (10, 6), (14, 10), (512, 4), (514, 8), (1034, 2)])
+@pytest.mark.parametrize("off,pad", [(0, 0), (4, 4), (1, 2), (2, 3)])
+def test_rgb_from_yuv_addresses(gpu, orc, w, h, off, pad):
+    """planes at any address and stride: word accesses only where every plane and stride allows them, widths around the
+    8 columns of a thread and the 512 of a workgroup's row; nothing is written past a row's 3w bytes"""
+    y, u, v = _planes(w, h, w + 7 * h)
+    uv = np.stack([u, v], -1).reshape(h // 2, w)
+
+    def place(a):
+        rows, n = a.shape
+        stride = (n + 3) // 4 * 4 + pad
+        host = np.zeros(off + rows * stride + 8, np.uint8)
+        host[off:off + rows * stride].reshape(rows, stride)[:, :n] = a
+        t = torch.from_numpy(host).cuda()
+        return t, ctypes.c_void_p(t.data_ptr() + off), stride
+
+    planes = [place(a) for a in (y, u, v, uv)]
+    (_, Y, ys), (_, U, us), (_, V, vs), (_, UV, uvs) = planes
+    for name, args, want in (("IYUV", (Y, ys, U, us, V, vs), orc.color_rgb_yuv(y, u, v)), ("NV12", (Y, ys, UV, uvs), orc.color_rgb_yuv(y, uv))):
+        t, d, ds = place(np.full((h, 3 * w), 77, np.uint8))
+        before = t.clone()
+        call(f"ColorConvert_RGB_{name}", w, h, d, ds, *args)
+        expect = before.cpu().numpy()
+        expect[off:off + h * ds].reshape(h, ds)[:, :3 * w] = want.reshape(h, 3 * w)
+        assert_same(t.cpu().numpy(), expect, f"{name}->RGB {w}x{h} at {off}, strides + {pad}")
