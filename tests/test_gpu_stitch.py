@@ -92,3 +92,79 @@ def test_loom_stitch_config_size(gpu, orc):
     assert_same(one, want, "stitch vs oracle")
     sel = rig["camId0"].cpu().numpy()
     assert (sel < 31).any() and (sel == 31).any() and (sel > 31).any()
+
+
+def _dev(a, off, stride):
+    """rows of `a` (bytes) in device memory at byte `off`, `stride` bytes apart"""
+    rows = a.reshape(a.shape[0], -1)
+    host = np.zeros(off + rows.shape[0] * stride, np.uint8)
+    host[off:].reshape(rows.shape[0], stride)[:, :rows.shape[1]] = rows
+    t = torch.from_numpy(host).cuda()
+    return t, ctypes.c_void_p(t.data_ptr() + off)
+
+
+def _entries(rng, h, w, sw, sh):
+    """raw 13.3 entries: inside, in the last column and row, past them, and marked invalid"""
+    e = np.stack([rng.integers(0, 8 * sw + 24, (h, w)), rng.integers(0, 8 * sh + 24, (h, w))], -1).astype(np.uint16)
+    e[rng.random((h, w)) < 0.2] = 0xffff
+    return e
+
+
+@pytest.mark.parametrize("sw,sh", [(2, 2), (3, 2), (37, 21), (64, 3)])
+@pytest.mark.parametrize("off,pad", [(0, 0), (1, 1), (3, 6)])
+@pytest.mark.parametrize("constant", [False, True])
+def test_remap_u24_raw_entries(gpu, sw, sh, off, pad, constant):
+    """the packed pixel pairs: sources at any address and stride that end with their last pixel, entries whose left pixel
+    is the last column (its own right neighbour), against the formula in numpy"""
+    rng = np.random.default_rng(sw * sh + off)
+    w, h = 101, 13
+    src = rng.integers(0, 256, (sh, sw, 3), dtype=np.uint8)
+    e = _entries(rng, h, w, sw, sh)
+    keep, S = _dev(src, off, 3 * sw + pad)
+    fixed = torch.from_numpy(e.view(np.uint8).reshape(h, 4 * w).copy()).cuda()
+    d = torch.zeros(h * (3 * w + 5), dtype=torch.uint8, device="cuda")
+    args = [w, h, ctypes.c_void_p(d.data_ptr()), 3 * w + 5, sw, sh, S, 3 * sw + pad, ctypes.c_void_p(fixed.data_ptr()), 4 * w]
+    if constant:
+        call("Remap_U24_U24_Bilinear_Constant", *args, ctypes.c_uint8(201))
+    else:
+        call("Remap_U24_U24_Bilinear", *args)
+    bad = e[..., 0] == 0xffff
+    m = np.where(e == 0xffff, 0 if constant else 8, e).astype(np.int64)
+    fx, fy = (m[..., 0] & 7)[..., None], (m[..., 1] & 7)[..., None]
+    xi, yi = np.minimum(m[..., 0] >> 3, sw - 1), np.minimum(m[..., 1] >> 3, sh - 1)
+    x1, y1 = np.minimum(xi + 1, sw - 1), np.minimum(yi + 1, sh - 1)
+    s = src.astype(np.int64)
+    t = (s[yi, xi] * (8 - fx) * (8 - fy) + s[yi, x1] * fx * (8 - fy) + s[y1, xi] * (8 - fx) * fy + s[y1, x1] * fx * fy + 32) >> 6
+    if constant:
+        t[bad] = 201
+    got = d.cpu().numpy().reshape(h, 3 * w + 5)
+    assert_same(got[:, :3 * w].reshape(h, w, 3).copy(), t.astype(np.uint8), f"remap {sw}x{sh} at {off}")
+    assert not got[:, 3 * w:].any()
+
+
+@pytest.mark.parametrize("w,h", [(8, 3), (4, 2), (3, 2), (203, 9), (257, 5), (1030, 3)])
+@pytest.mark.parametrize("off", [0, 1, 2])
+def test_loom_fused_addresses(gpu, orc, w, h, off):
+    """four pixels a thread: widths that leave one to three pixels over, output rows, weights and cameras at any address"""
+    rng = np.random.default_rng(w * h + off)
+    n, sw, sh, g = 5, 37, 21, (w + 7) // 8
+    cams = [rng.integers(0, 256, (sh, sw, 3), dtype=np.uint8) for _ in range(n)]
+    fixed = np.stack([rng.integers(0, 8 * (sw - 1), (n * h, w)), rng.integers(0, 8 * (sh - 1), (n * h, w))], -1).astype(np.uint16)
+    fixed[rng.random((n * h, w)) < 0.1] = 0xffff
+    wts = rng.integers(0, 256, (n * h, w), dtype=np.uint8)
+    id0 = rng.choice(np.array([0, 1, 4, 7, 31, 40, 128, 129, 130, 131, 132, 250], np.uint8), (h, g))
+    pick = lambda: (rng.choice(np.array([0, 1, 2, 3, 4, 31]), (h, g, 3)) << np.array([0, 5, 10])).sum(-1).astype(np.uint16)
+    id1, id2 = pick(), pick()
+    devs = [_dev(c, off + k, 3 * sw + k) for k, c in enumerate(cams)]
+    fd = torch.from_numpy(fixed.view(np.uint8).reshape(n * h, 4 * w).copy()).cuda()
+    wk, W = _dev(wts, off, w + off)
+    I = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (id0, id1.view(np.int16), id2.view(np.int16))]
+    base = np.full((h, 3 * w), 77, np.uint8)
+    out, O = _dev(base, off, 3 * w + off)
+    vp = lambda t: ctypes.c_void_p(t.data_ptr())
+    call("Stitch_Loom_RGB", w, h, O, 3 * w + off, n, (ctypes.c_void_p * n)(*[d[1].value for d in devs]),
+         (ctypes.c_uint32 * n)(*[3 * sw + k for k in range(n)]), sw, sh, vp(fd), 4 * w, W, w + off, vp(I[0]), g, vp(I[1]), 2 * g, vp(I[2]), 2 * g)
+    want = orc.stitch_loom_remap(cams, fixed, wts, id0, id1, id2, dst=np.full((h, w, 3), 77, np.uint8))
+    got = out.cpu().numpy()[off:].reshape(h, 3 * w + off)
+    assert_same(got[:, :3 * w].reshape(h, w, 3).copy(), want, f"fused stitch {w}x{h} at {off}")
+    assert not got[:, 3 * w:].any()
