@@ -152,10 +152,24 @@ MVX_DEV WarpBox warp_box(float xlo, float xhi, float ylo, float yhi, uint32_t sw
     return b;
 }
 
-// stage rows r0..r1, columns cA..cA+4nd-1 (linear-address coordinates) into lds, row pitch 4nd bytes
+// stage rows r0..r1, columns cA..cA+4nd-1 (linear-address coordinates) into lds, row pitch 4nd bytes.  A box inside the
+// image lies in the plane whole (its last dword ends at or before the stride): its dwords are dealt to all threads one
+// after the other, without a check.  (A row of a 64-pixel tile is 18 dwords or so: 16 threads a row took two trips for
+// it.  With one corner a lane in place of four, 3840x2160: perspective 21.2 -> 19.4 us, affine 17.5 -> 15.7.)
 MVX_DEV void warp_stage(uint32_t *lds, const WarpBox &b, const uint8_t *src, uint32_t stride, uint64_t n)
 {
     const int rows = b.r1 - b.r0 + 1;
+    if (b.inside) {
+        const uint32_t total = (uint32_t)(rows * b.nd);
+        const float inv = __builtin_amdgcn_rcpf((float)b.nd);   // i + 1/2 is at least 1/(2 nd) of a row from a row's end, and i at most WLDS_DW
+        const uint8_t *p = src + ((uint32_t)b.r0 * stride + (uint32_t)b.cA);   // planes are below 2^31 bytes
+#pragma unroll 2
+        for (uint32_t i = threadIdx.y * (WTW / 4) + threadIdx.x; i < total; i += (WTW / 4) * WTH) {
+            const uint32_t r = (uint32_t)(((float)i + 0.5f) * inv);
+            lds[i] = *reinterpret_cast<const uint32_t *>(p + (r * stride + 4 * (i - r * (uint32_t)b.nd)));
+        }
+        return;
+    }
     for (int rr = (int)threadIdx.y; rr < rows; rr += (int)blockDim.y) {
         const int64_t base = (int64_t)(b.r0 + rr) * stride + b.cA;
         for (int k = (int)threadIdx.x; k < b.nd; k += (int)blockDim.x) {
@@ -163,6 +177,24 @@ MVX_DEV void warp_stage(uint32_t *lds, const WarpBox &b, const uint8_t *src, uin
             lds[rr * b.nd + k] = (lin >= 0 && (uint64_t)lin + 4 <= n) ? *reinterpret_cast<const uint32_t *>(src + lin) : 0u;
         }
     }
+}
+
+// the value of the lane whose number differs by 1 (quad_perm 1,0,3,2) or by 2 (quad_perm 2,3,0,1)
+MVX_DEV float lane_xor1(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, true)); }
+MVX_DEV float lane_xor2(float v) { return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4e, 0xf, 0xf, true)); }
+MVX_DEV float quad_min(float v) { v = fminf(v, lane_xor1(v)); return fminf(v, lane_xor2(v)); }
+MVX_DEV float quad_max(float v) { v = fmaxf(v, lane_xor1(v)); return fmaxf(v, lane_xor2(v)); }
+
+// the same box in every lane (scalar registers)
+MVX_DEV WarpBox wave_box(WarpBox b)
+{
+    b.r0 = __builtin_amdgcn_readfirstlane(b.r0);
+    b.r1 = __builtin_amdgcn_readfirstlane(b.r1);
+    b.cA = __builtin_amdgcn_readfirstlane(b.cA);
+    b.nd = __builtin_amdgcn_readfirstlane(b.nd);
+    b.on = __builtin_amdgcn_readfirstlane((int)b.on);
+    b.inside = __builtin_amdgcn_readfirstlane((int)b.inside);
+    return b;
 }
 
 // the bytes at LDS offsets o and o+1 (o >= 0) in bits 0..15, from two dword-aligned reads and a byte
@@ -207,6 +239,7 @@ k_warp_affine_lds(uint32_t dw, uint32_t dh, uint8_t *__restrict__ dst, uint32_t 
                              m.r10 * xb + (yb * m.r11 + m.c2)};
         b = warp_box(fminf(fminf(sx[0], sx[1]), fminf(sx[2], sx[3])), fmaxf(fmaxf(sx[0], sx[1]), fmaxf(sx[2], sx[3])),
                      fminf(fminf(sy[0], sy[1]), fminf(sy[2], sy[3])), fmaxf(fmaxf(sy[0], sy[1]), fmaxf(sy[2], sy[3])), sw, sh);
+        b = wave_box(b);
     }
     if (b.on) warp_stage(stage, b, src, srcStride, n);
     __syncthreads();
@@ -272,22 +305,15 @@ k_warp_perspective_lds(uint32_t dw, uint32_t dh, uint8_t *__restrict__ dst, uint
     const uint64_t n = (uint64_t)sh * srcStride;
     const int32_t limit = (int32_t)(sh * srcStride - 1u);
     const uint32_t tx0 = blockIdx.x * WTW, ty0 = blockIdx.y * WTH;
-    WarpBox b{0, -1, 0, 0, false};
+    WarpBox b{0, -1, 0, 0, false, false};
     {
-        float sx[4], sy[4], sz[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const float xf = (float)(tx0 + ((c & 1) ? WTW - 1 : 0)), yf = (float)(ty0 + ((c & 2) ? WTH - 1 : 0));
-            sz[c] = m.g * xf + (yf * m.h + m.i);
-            const float z = 1.0f / sz[c];
-            sx[c] = (m.a * xf + (yf * m.b + m.c)) * z;
-            sy[c] = (m.d * xf + (yf * m.e + m.f)) * z;
-        }
-        const bool pos = sz[0] > 0.0f && sz[1] > 0.0f && sz[2] > 0.0f && sz[3] > 0.0f;
-        const bool neg = sz[0] < 0.0f && sz[1] < 0.0f && sz[2] < 0.0f && sz[3] < 0.0f;
-        if (pos || neg)
-            b = warp_box(fminf(fminf(sx[0], sx[1]), fminf(sx[2], sx[3])), fmaxf(fmaxf(sx[0], sx[1]), fmaxf(sx[2], sx[3])),
-                         fminf(fminf(sy[0], sy[1]), fminf(sy[2], sy[3])), fmaxf(fmaxf(sy[0], sy[1]), fmaxf(sy[2], sy[3])), sw, sh);
+        // each lane maps one corner, four lanes have all
+        const uint32_t c = threadIdx.x;
+        const float xf = (float)(tx0 + ((c & 1) ? WTW - 1 : 0)), yf = (float)(ty0 + ((c & 2) ? WTH - 1 : 0));
+        const float sz = m.g * xf + (yf * m.h + m.i);
+        const float z = 1.0f / sz;
+        const float sx = (m.a * xf + (yf * m.b + m.c)) * z, sy = (m.d * xf + (yf * m.e + m.f)) * z;
+        if (__all(sz > 0.0f) || __all(sz < 0.0f)) b = wave_box(warp_box(quad_min(sx), quad_max(sx), quad_min(sy), quad_max(sy), sw, sh));
     }
     if (b.on) warp_stage(stage, b, src, srcStride, n);
     __syncthreads();

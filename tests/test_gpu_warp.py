@@ -309,3 +309,23 @@ def test_remap_rgb_is_three_u8_remaps(gpu, orc, w, h):
             for c in range(3):
                 want = orc.remap(np.ascontiguousarray(rgb[..., c]), mp, border is not None, border or 0)
                 assert_same(got[..., c], want, f"RGB remap {w}x{h} k1 {k1} border {border} channel {c}")
+
+
+@pytest.mark.parametrize("sx,sy", [(0.02, 0.02), (0.5, 1.7), (1.0, 1.0), (1.9, 1.9), (0.05, 3.5), (3.5, 0.05), (2.3, 2.3)])
+@pytest.mark.parametrize("w", [512, 500])
+def test_warp_staged_box_shapes(gpu, orc, sx, sy, w):
+    """boxes inside the image from a few dwords to the whole staging array, narrow and wide, and too large for it;
+    sources whose stride equals their width, so a box's last dword ends with its row"""
+    h, dw, dh = 240, 128, 48
+    src = synth.uniform_u8(w, h, 43)
+    s = Plane.from_array(src)
+    for tx, ty, rot in ((3.25, 2.5, 0.0), (w - 1 - sx * (dw - 1) - 3.5, h - 1 - sy * (dh - 1) - 3.5, 0.0), (9.0, 20.0, 0.01)):
+        m = np.array([sx, rot, -rot, sy, tx, ty], np.float32)
+        p = np.array([sx, rot, 1e-5, -rot, sy, 2e-5, tx, ty, 1], np.float32)
+        for border in (None, 9):
+            d = _run_warp(0, s, dw, dh, m, border)
+            want, _ = orc.warp_affine(src, dw, dh, m, border is not None, border or 0, padded=True)
+            assert_same(_padded(d), want, f"affine {m.tolist()} {border}")
+            d = _run_warp(1, s, dw, dh, p, border)
+            want, _ = orc.warp_perspective(src, dw, dh, p, border or 0, padded=True)
+            assert_same(_padded(d), want, f"perspective {p.tolist()} {border}")
