@@ -280,6 +280,7 @@ MVX_DEV uint32_t block_scan(uint32_t v, uint32_t &total)
 // 3840x2160 with suppression: a count a load and marks a byte a load 12.5 us, 6.3 now.
 typedef uint32_t fast_u32x4 __attribute__((ext_vector_type(4)));
 typedef fast_u32x4 fast_u32x4_dword __attribute__((aligned(4)));
+typedef fast_u32x4 fast_u32x4_any __attribute__((aligned(1)));
 
 template <bool SUPP>
 __global__ void __launch_bounds__(256)
@@ -288,10 +289,9 @@ k_fast_write(FastArgs a, const uint8_t *__restrict__ marks, const uint32_t *__re
 {
     const int y = 3 + (int)blockIdx.x;
     const uint8_t *row = marks + (long)y * a.w;
-    const bool words = (((uintptr_t)marks | a.w) & 3u) == 0;   // rows start at whole words
     const auto load = [&](int xs) {
         fast_u32x4 v = {0u, 0u, 0u, 0u};
-        if (words && xs + 16 <= (int)a.w) return (fast_u32x4) * (const fast_u32x4_dword *)(row + xs);
+        if (xs + 16 <= (int)a.w) return (fast_u32x4) * (const fast_u32x4_any *)(row + xs);   // rows start at any address
 #pragma unroll
         for (int k = 0; k < 16; k++) v[k >> 2] |= (xs + k < (int)a.w ? (uint32_t)row[xs + k] : 0u) << (8 * (k & 3));
         return v;
