@@ -184,10 +184,11 @@ MVX_DEV void canny_strip(uint32_t w, uint32_t h, uint16_t *dst, uint32_t dstStri
     const int col = xs - R + lane;
     int sc = col;
     const int kind = canny_slot(col, aligned, a16, sc);
-    const __amdgpu_buffer_rsrc_t sR = plane_rsrc(src), dR = plane_rsrc(dst);
+    gptr_t<const uint8_t> sp = gmem(src);
+    gptr_t<uint8_t> dp = (gptr_t<uint8_t>)gmem(dst);
     // a zero slot still loads an in-plane byte (column 0) and drops it, so the loads stay unconditional
     auto load = [&](int r) -> int {
-        const int v = (int)__builtin_amdgcn_raw_buffer_load_b8(sR, sc, (int)((uint32_t)r * srcStride), 0);
+        const int v = sp[(uint64_t)(uint32_t)r * srcStride + (uint32_t)sc];
         return kind == 0 ? 0 : v;
     };
     // every source row of the strip is loaded before the first is used: the loads are all in flight
@@ -221,7 +222,7 @@ MVX_DEV void canny_strip(uint32_t w, uint32_t h, uint16_t *dst, uint32_t dstStri
         uint16_t out = canny_simd_px<G, L2>(a0, a1);
         if (outLane) {
             if (x >= aligned - 1) out = canny_scalar<G, L2>(src, (long)h * srcStride, srcStride, x, y);
-            __builtin_amdgcn_raw_buffer_store_b16(out, dR, 2 * x, (int)((uint32_t)y * dstStride), 0);
+            *(gptr_t<uint16_t>)(dp + (uint64_t)(uint32_t)y * dstStride + 2 * (uint32_t)x) = out;
         }
     }
 }
@@ -890,8 +891,8 @@ int canny_sobel_g(mvx_stream_t stream, uint32_t w, uint32_t h, uint16_t *dst, ui
     if (w == 0 || h == 0) return MVX_SUCCESS;
     if (!plane_ok_c(dst, w, dstStride, 2) || !plane_ok_c(src, w, srcStride, 1)) return MVX_ERROR_INVALID_PARAMETERS;
     if ((int)h < G) return MVX_SUCCESS;
-    // buffer offsets (row * stride + column) stay below 2^32
-    if ((uint64_t)h * dstStride > 0xffffffffull || (uint64_t)h * srcStride > 0xffffffffull) return MVX_ERROR_INVALID_PARAMETERS;
+    // (the 3x3 L1 form takes larger planes too)
+    if ((G != 3 || L2) && ((uint64_t)h * dstStride > 0xffffffffull || (uint64_t)h * srcStride > 0xffffffffull)) return MVX_ERROR_INVALID_PARAMETERS;
     if (w < 16) {
         hipLaunchKernelGGL((k_canny_sobel_g_narrow<G, L2>), dim3(1), dim3(64), 0, stream_of(stream), w, h, dst, dstStride, src, srcStride);
     } else {
