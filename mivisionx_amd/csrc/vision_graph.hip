@@ -95,6 +95,9 @@ template <class Ptr> MVX_DEV uint32_t luma(Ptr p)
     return (uint32_t)min(max(iv, 0), 255);
 }
 
+// four bytes at any address
+struct __attribute__((packed, aligned(1))) RgbDword { uint32_t v; };
+
 // the virtual luma plane at linear position (r, c): stride yStride, padding and guard bytes zero
 MVX_DEV uint32_t yflat(const FrameDesc &F, const GraphParams &P, int r, int c)
 {
@@ -185,6 +188,7 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
     // two rows ahead, from a row clamped into the image; the last column's dword starts one byte early.
     // Images narrower than a tile's window may wrap more than once: they go through yflat.
     const bool wide = w >= 64;
+    const uint64_t rgbAddr = (uint64_t)F.rgb;
     int edgeRow = 0, edgeCol = tx0 - HY + lane;
     if (edgeCol < 0) { edgeRow = -1; edgeCol += P.yStride; }
     else if (edgeCol >= P.yStride) { edgeRow = 1; edgeCol -= P.yStride; }
@@ -192,8 +196,12 @@ MVX_DEV void front_tile(uint64_t *cand, const FrameDesc &F, const GraphParams &P
     const uint32_t edgeOff = edgeColOk ? 3u * (uint32_t)edgeCol - (edgeCol == w - 1 ? 1u : 0u) : 0u, edgeShift = edgeCol == w - 1 ? 8u : 0u;
     auto fetch = [&](int k) -> uint32_t {
         if (INNER) return __builtin_amdgcn_raw_buffer_load_b32(rgbR, rgbCol, (int)((uint32_t)(ty0 - HY + k) * rgbStride), 0);
-        const uint32_t r = (uint32_t)min(max(ty0 - HY + k + edgeRow, 0), h - 1);
-        return __builtin_amdgcn_raw_buffer_load_b32(rgbR, (int)(__umul24(r, rgbStride) + edgeOff), 0, 0);
+        // 64-bit row addresses, since a frame can be a narrow view of a wide buffer; the three that a lane chooses
+        // from are scalar arithmetic
+        const auto row = [&](int r) { return rgbAddr + (uint64_t)(uint32_t)min(max(r, 0), h - 1) * rgbStride; };
+        const int r = ty0 - HY + k;
+        const uint64_t above = row(r - 1), same = row(r), below = row(r + 1);
+        return ((gptr_t<const RgbDword>)((edgeRow < 0 ? above : edgeRow > 0 ? below : same) + edgeOff))->v;
     };
     // luma row k from its fetched dwords
     auto luma_of = [&](int k, uint32_t p) -> int {

@@ -1,15 +1,17 @@
 """The fused tile pass where its rows change path -- Harris rows with and without a score, scores at and
 around zero, negative thresholds and sensitivities, Canny thresholds from 0 to above every magnitude, the
-scaled image's scalar tail, tiles cut at every edge -- and the half-size pyramid step at the edges of its
-62-chunk waves.  The per-node kernels are the reference for the graph (each has its own oracle tests), the
-oracle for the pyramid step; every byte has to be the same."""
+scaled image's scalar tail, tiles cut at every edge, frames inside much wider buffers -- and the half-size
+pyramid step at the edges of its 62-chunk waves.  The per-node kernels are the reference for the graph (each
+has its own oracle tests), the oracle for the pyramid step; every byte has to be the same."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from mivisionx_amd import synth
+from mivisionx_amd import kernels, synth
 from mivisionx_amd.device import Plane, call
-from mivisionx_amd.pipelines import FusedVisionGraph, VisionGraph4K
+from mivisionx_amd.pipelines import FusedVisionGraph, VisionGraph4K, _ptr, _stream
 from util import assert_same
 
 pytestmark = pytest.mark.gpu
@@ -62,6 +64,33 @@ def _compare(rgb, lower, upper, k, thr):
             assert_same(got["pyramid"][l], want["pyramid"][l], f"frame {i} level {l}")
         assert got["count"] == want["count"]
         assert got["corners"].tobytes() == want["corners"].tobytes(), f"frame {i} corners"
+
+
+@pytest.mark.parametrize("w,h,stride", [(128, 66, 1 << 24), (128, 66, (1 << 26) + 16), (180, 98, (1 << 24) + 4096), (64, 16, (1 << 28) + 16)])
+def test_frame_is_a_narrow_view(gpu, w, h, stride):
+    """rows 16 MiB and more apart: the same bytes as for the packed frame (the planes above 4 GiB have
+    border tiles only)"""
+    print(f"fused graph: {w}x{h}, RGB stride {stride}", flush=True)
+    rgb = _rgb("noise", w, h)
+    f = FusedVisionGraph(w, h, w // 2, h // 2, levels=2)
+    f.frames[0].rgb.upload(rgb)
+    f.run()
+    torch.cuda.synchronize()
+    want = f.frames[0].results()
+    wide = torch.empty((h, stride), dtype=torch.uint8, device="cuda")
+    wide[:, :3 * w].copy_(torch.from_numpy(rgb.reshape(h, 3 * w)))
+    f._arr[0].rgb, f._arr[0].rgbStride = wide.data_ptr(), stride
+    assert kernels().mvx_VisionGraph_prepare(_stream(), ctypes.byref(f.params), f._arr, 1, _ptr(f.ws), ctypes.c_size_t(f.ws_size)) == 0
+    f.run()
+    torch.cuda.synchronize()
+    got = f.frames[0].results()
+    del wide
+    torch.cuda.empty_cache()
+    for k in ("edges", "scaled"):
+        assert_same(got[k], want[k], k)
+    for l in range(2):
+        assert_same(got["pyramid"][l], want["pyramid"][l], f"level {l}")
+    assert got["count"] == want["count"] and got["corners"].tobytes() == want["corners"].tobytes()
 
 
 @pytest.mark.parametrize("w,h", [(5, 5), (6, 5), (15, 6), (17, 7), (990, 9), (991, 11), (992, 12), (993, 13), (994, 7), (1008, 6), (1985, 10)])
