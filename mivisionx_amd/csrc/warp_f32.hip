@@ -293,8 +293,8 @@ k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t ti
         s.ok = true;
         s.x0 = x + (int)fu; s.y0 = y + (int)fv;
         const bool usual = (z >= 0x1p-60f) & (z <= 0x1p60f);
-        const auto accumulate = [&](auto check) {
-            constexpr bool CHECK = decltype(check)::value;
+        const auto accumulate = [&](auto check, auto quotients) {
+            constexpr bool CHECK = decltype(check)::value, QUOTIENTS = decltype(quotients)::value;
             s.fx = du - fu; s.fy = dv - fv;
             const float gx = 1.f - s.fx, gy = 1.f - s.fy;
             const float Iu = fmaf(s.fy, s.p11 - s.p10, gy * (s.p01 - s.p00)), Iv = fmaf(s.fx, s.p11 - s.p01, gx * (s.p10 - s.p00));
@@ -308,8 +308,9 @@ k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t ti
             }
             const bool take = (!CHECK || s.ok) & (g != 0.f);
             if (take) {
-                const float gz = g * rz;
-                const float a = gz * Iu, b = gz * Iv, c = -fmaf(a, X + du, b * (Y + dv));
+                // (rz, or g rz, may overflow where the quotients do not)
+                const float gz = QUOTIENTS ? g : g * rz;
+                const float a = QUOTIENTS ? gz * Iu / z : gz * Iu, b = QUOTIENTS ? gz * Iv / z : gz * Iv, c = -fmaf(a, X + du, b * (Y + dv));
                 sa += a; sb += b; sc += c;
                 saY = fmaf(a, Y, saY); sbY = fmaf(b, Y, sbY); scY = fmaf(c, Y, scY);
             }
@@ -319,10 +320,10 @@ k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t ti
             const uint32_t off = __umul24((uint32_t)s.y0, S.stride) + 4u * (uint32_t)s.x0;
             const float2a t = *(const float2a *)(sbase + off), b = *(const float2a *)(sbase + S.stride + off);
             s.p00 = t.x; s.p01 = t.y; s.p10 = b.x; s.p11 = b.y;
-            accumulate(std::false_type());
+            accumulate(std::false_type(), std::false_type());
         } else {
-            if (!wave_all(usual & (fabsf(du) < 1.0e7f) & (fabsf(dv) < 1.0e7f))) {
-                rz = 1.f / z;
+            const bool plain = !wave_all(usual & (fabsf(du) < 1.0e7f) & (fabsf(dv) < 1.0e7f));
+            if (plain) {
                 du = nu / z;
                 dv = nv / z;
                 s.ok = (z > 0.f) & (fabsf(du) < 1.0e7f) & (fabsf(dv) < 1.0e7f);   // also false for NaN
@@ -338,7 +339,8 @@ k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t ti
             const bool ia = xa == s.x0, ib = xb == s.x0 + 1, ja = ya == s.y0, jb = yb == s.y0 + 1;
             s.p00 = (ia & ja) ? t0 : 0.f; s.p01 = (ib & ja) ? t1 : 0.f;
             s.p10 = (ia & jb) ? t2 : 0.f; s.p11 = (ib & jb) ? t3 : 0.f;
-            accumulate(std::true_type());
+            if (plain) accumulate(std::true_type(), std::true_type());
+            else accumulate(std::true_type(), std::false_type());
         }
     }
     if (SCAT) sg.finish();

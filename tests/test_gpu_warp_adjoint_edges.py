@@ -78,3 +78,24 @@ def test_adjoint_paths(gpu, src_wh, dst_wh, name):
     assert float((loss - 1.5 - want).abs().max()) <= 1e-4 * max(1.0, float(want.abs().max()))
     assert float((gsl.double() - ws).abs().max()) <= 1e-4 * max(1.0, float(ws.abs().max()))
     _check_gH(gHl, wH, H, 0.5 * res.detach(), "dL/dH of the loss")
+
+
+@pytest.mark.parametrize("scale,gscale,sscale", [(2.0 ** -133, 2.0 ** -40, 1.0), (2.0 ** -126, 8.0, 2.0 ** -30), (2.0 ** 126, 8.0, 1.0)])
+def test_adjoint_z_at_the_ends_of_f32(gpu, scale, gscale, sscale):
+    """1 / z, or dL/d(out) / z, outgrows an F32 but dL/d(out) dI/du / z does not.  The shift by (1.5, -2.5) is
+    exact in F32, so what is left is the sums' rounding: below 130 * 70 terms of one size, 1e-5 of the largest."""
+    print(f"adjoint, z = {scale}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    src = (torch.rand((1, 37, 130), generator=gen, device="cuda") > 0.5).float() * sscale
+    src[:, :, 64:] = 0.0                                     # no slope: dL/d(out) / z meets 0
+    g = (torch.randint(1, 3, (1, 35, 127), generator=gen, device="cuda")).float() * gscale
+    H = torch.tensor([[1, 0, 1.5, 0, 1, -2.5, 0, 0, 1]], dtype=torch.float64, device="cuda") * scale
+    s64, H64 = src.double().requires_grad_(True), H.clone().requires_grad_(True)
+    out = warp64(s64, H64.reshape(-1, 3, 3), (35, 127))
+    ws, wH = torch.autograd.grad((out * g.double()).sum(), (s64, H64))
+    for want_src in (True, False):
+        gs, gH = align.warp_adjoint(g, src, H, want_src=want_src)
+        assert torch.isfinite(gH).all(), f"dL/dH {gH}"
+        assert float((gH - wH).abs().max()) <= 1e-5 * float(wH.abs().max()), f"{gH}\n{wH}"
+        if want_src:
+            assert float((gs.double() - ws).abs().max()) <= 1e-5 * float(ws.abs().max())
