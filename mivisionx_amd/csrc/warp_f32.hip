@@ -261,8 +261,8 @@ __global__ void __launch_bounds__(WF_BX * WF_BY, SCAT ? 7 : 8)
 k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t tilesX, const double *Hs, float weight,
                    float *gsrc, uint32_t gsStride, size_t gsBatch, float *partials)
 {
-    const uint32_t tiles = gridDim.x;
-    const uint32_t id = xcd_order(blockIdx.y * tiles + blockIdx.x, tiles * gridDim.y);
+    const uint32_t tiles = gridDim.x * gridDim.y;   // a 1-D grid but for the largest images
+    const uint32_t id = xcd_order((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x, tiles * gridDim.z);
     const uint32_t img = id / tiles, tile = id - img * tiles;
     const uint32_t ty = tile / tilesX, tx = tile - ty * tilesX;
     const int yw = (int)((ty * WF_BY + __builtin_amdgcn_readfirstlane(threadIdx.y)) * ROWS);
@@ -520,9 +520,11 @@ static int warp_adjoint_common(mvx_stream_t stream, int mode, uint32_t count, ui
     // two rounds of waves or more for the 1024 SIMDs, else four (sixteen was no faster for 64 x 1024x1024)
     const uint32_t rows = tiles_of(8) * count >= 2048 ? 8 : 4;
     const uint64_t tiles = tiles_of(rows);
-    if (tiles > 0xffffffull || tiles * count > 0xffffffffull) return MVX_ERROR_INVALID_PARAMETERS;   // the launch's own limits
+    if (tiles * count > 0xffffffffull) return MVX_ERROR_INVALID_PARAMETERS;   // the kernel's 32-bit tile numbers
+    // a launch takes below 2^32 threads in x; images of more than 34 Gpixel have a row of tiles there
+    const dim3 grid = tiles <= 0xffffffull ? dim3((uint32_t)tiles, 1, count) : dim3(tilesX, (uint32_t)(tiles / tilesX), count);
     const auto run = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3((uint32_t)tiles, count), dim3(WF_BX, WF_BY), 0, stream_of(stream), S, G, dw, dh, tilesX, H, weight,
+        hipLaunchKernelGGL(kern, grid, dim3(WF_BX, WF_BY), 0, stream_of(stream), S, G, dw, dh, tilesX, H, weight,
                            gradSrc, gsStride, gsBatch, part);
     };
     const auto pick = [&](auto m) {

@@ -1,12 +1,14 @@
 """Host-side checks of the alignment parameterisation (no GPU): the chain rule from dL/dH to dL/dp
 and from a pyramid level's dL/dH_l to the base level, against float64 autograd of the same maps,
 and the synthetic homographies' ranges."""
+import ctypes as c
 import math
 
 import numpy as np
+import pytest
 import torch
 
-from mivisionx_amd import align
+from mivisionx_amd import align, kernels
 
 
 def test_identity_and_true_parameter_ranges():
@@ -57,3 +59,17 @@ def test_corner_error_is_zero_for_equal_and_exact_for_a_shift():
     T[:, 1, 2] = 4.0
     assert float(align.corner_error(H, H, 100, 80).max()) == 0.0
     assert np.allclose(align.corner_error(H, T, 100, 80).numpy(), 5.0)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the arguments are no device memory: without a GPU nothing is launched")
+@pytest.mark.parametrize("dw,dh", [(64, 64), (1 << 18, 1 << 17), ((1 << 18) + 1, 1 << 17), (1 << 18, (1 << 17) + 1), (1 << 20, 1 << 16)])
+def test_adjoint_takes_images_of_any_size_that_fits(dw, dh):
+    """images of 34 Gpixel (137 GB, which one card holds) and more are no invalid parameter: here their launch
+    fails for want of a GPU, as that of a small one does"""
+    K = kernels()
+    K.mvx_warp_perspective_f32_workspace_size.restype = c.c_size_t
+    size = K.mvx_warp_perspective_f32_workspace_size(1, dw, dh)
+    p = c.c_void_p(1 << 20)
+    rc = K.mvx_warp_perspective_f32_adjoint(None, 1, dw, dh, p, 4 * dw, c.c_size_t(0), 16, 16, p, 64, c.c_size_t(0), p, None, 64,
+                                            c.c_size_t(0), p, p, c.c_size_t(size))
+    assert rc == -1    # MVX_ERROR_LAUNCH, not MVX_ERROR_INVALID_PARAMETERS
