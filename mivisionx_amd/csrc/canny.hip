@@ -849,7 +849,7 @@ __global__ void __launch_bounds__(256) k_ct_resolve(CtArgs a)
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     for (uint32_t k = (uint32_t)t.row; k < count; k += CT_H) {
         const uint32_t p = gmem((const uint16_t *)a.border)[(long)t.tile * 2 * CT_NB + CT_NB + k];
-        if (gfind(gmem((const uint32_t *)a.parent), 1u + (uint32_t)t.tile * CT_NB + k) == 0u)
+        if (gfind_settled<__HIP_MEMORY_SCOPE_WAVEFRONT>(gmem(a.parent), 1u + (uint32_t)t.tile * CT_NB + k) == 0u)
             atomicOr(&seeds[(t.lane & 48) + (int)(p / CT_W)][(p % CT_W) >> 5], 1u << (p & 31u));
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

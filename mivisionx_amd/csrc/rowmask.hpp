@@ -15,10 +15,36 @@ MVX_DEV uint32_t gfind(gptr_t<const uint32_t> par, uint32_t p)
     return p;
 }
 
+// One step of a find once all unions are done: p's parent is l, which is no root unless the answer is l.  The
+// links it passes are shortened by half: p now hangs under l's parent.  Roots are never written and every
+// value written is an ancestor, so finds of other waves may run beside it, whichever value they see.  (Only
+// then: beside a union, which counts on an id keeping the parent it was given, it would lose links.)
+template <int SCOPE> MVX_DEV uint32_t gstep(gptr_t<uint32_t> par, uint32_t p, uint32_t l)
+{
+    const uint32_t up = __hip_atomic_load(par + l, __ATOMIC_RELAXED, SCOPE);
+    if (up != l) __hip_atomic_store(par + p, up, __ATOMIC_RELAXED, SCOPE);
+    return up;
+}
+
+// the root of p once all unions are done
+template <int SCOPE> MVX_DEV uint32_t gfind_settled(gptr_t<uint32_t> par, uint32_t p)
+{
+    uint32_t l = par[p];
+    while (l != p) {
+        const uint32_t up = gstep<SCOPE>(par, p, l);
+        p = l;
+        l = up;
+    }
+    return p;
+}
+
 // The larger id hangs under the smaller at once, without finding the roots first: when it was a root (most
 // ids are) that is the whole union, one trip to memory instead of three.  When it was not, its old parent
 // still has to join b's set, and the loop goes on with those two; ids only fall, so it ends.  An id may so
-// hang under one that is no root: chains are as correct as stars for gfind.
+// hang under one that is no root: chains are as correct as stars for the finds, and where one component
+// winds through many tiles the settled finds shorten them for one another (16 frames of 3840x2160: border
+// pass 39 us, 52 with the roots found first; a serpentine of 16-row steps through 3840x2160 in the Canny
+// trace: 508 us with plain finds, 332 with the roots found first, 73 now).
 MVX_DEV void gunion(gptr_t<uint32_t> par, uint32_t a, uint32_t b)
 {
     while (a != b) {

@@ -40,21 +40,41 @@ def test_trace_random_maps(gpu, orc, w, h, p127, p255):
     assert_same(_trace(m), orc.canny_trace(m), f"trace {w}x{h} {p127}/{p255}")
 
 
+def _serpentine(w, h, step):
+    m = np.zeros((h, w), np.uint8)
+    for y in range(2, h - 2, step):
+        m[y, 2:w - 2] = 127
+        x = w - 3 if (y // step) % 2 == 0 else 2
+        if y + step < h - 2:
+            m[y:y + step, x] = 127
+    return m
+
+
 @pytest.mark.parametrize("w,h", [(300, 200), (1000, 700)])
 def test_trace_long_paths(gpu, orc, w, h):
     """a one-pixel serpentine of 127s through the whole image with a single 255 at its far end (every
     tile it crosses depends on the last one), and a second serpentine with no 255 (all of it -> 0)"""
-    m = np.zeros((h, w), np.uint8)
-    for y in range(2, h - 2, 4):
-        m[y, 2:w - 2] = 127
-        x = w - 3 if (y // 4) % 2 == 0 else 2
-        if y + 4 < h - 2:
-            m[y:y + 4, x] = 127
+    m = _serpentine(w, h, 4)
     m2 = m.copy()
     ys = np.nonzero(m[:, 2])[0]
     m[ys[-1], 2] = 255
     assert_same(_trace(m), orc.canny_trace(m), f"serpentine {w}x{h}")
     assert_same(_trace(m2), orc.canny_trace(m2), f"serpentine without a strong pixel {w}x{h}")
+
+
+@pytest.mark.parametrize("down", [False, True])
+@pytest.mark.parametrize("w,h,step", [(640, 480, 16), (1920, 1080, 40), (1920, 1080, 8)])
+def test_trace_chains_of_tiles(gpu, orc, w, h, step, down):
+    """one component through hundreds of tiles, along rows or down columns: the finds that shorten one
+    another's links see the strong end, or none"""
+    print(f"trace {w}x{h}, steps of {step}, {'down' if down else 'along'}", flush=True)
+    m = _serpentine(h, w, step).T.copy() if down else _serpentine(w, h, step)
+    for strong in (True, False):
+        if strong:
+            m[2, 2] = 255
+        else:
+            m[2, 2] = 127
+        assert_same(_trace(m), orc.canny_trace(m), f"serpentine, strong end {strong}")
 
 
 def test_trace_stack_alignment(gpu, orc):

@@ -1,8 +1,9 @@
 """The fused tile pass where its rows change path -- Harris rows with and without a score, scores at and
 around zero, negative thresholds and sensitivities, Canny thresholds from 0 to above every magnitude, the
-scaled image's scalar tail, tiles cut at every edge, frames inside much wider buffers -- and the half-size
-pyramid step at the edges of its 62-chunk waves.  The per-node kernels are the reference for the graph (each
-has its own oracle tests), the oracle for the pyramid step; every byte has to be the same."""
+scaled image's scalar tail, tiles cut at every edge, components that wind through all tiles, frames inside
+much wider buffers -- and the half-size pyramid step at the edges of its 62-chunk waves.  The per-node kernels
+are the reference for the graph (each has its own oracle tests), the oracle for the pyramid step; every byte
+has to be the same."""
 import ctypes
 
 import numpy as np
@@ -22,6 +23,15 @@ def _rgb(kind, w, h):
         return synth.u32(11, 3, w * h * 3).astype(np.uint8).reshape(h, w, 3)
     if kind == "flat":        # no gradient at all
         return np.full((h, w, 3), 77, np.uint8)
+    if kind in ("winding", "winding down"):  # one weak line through all tiles, strong at one end
+        a, b = (w, h) if kind == "winding" else (h, w)
+        img = np.zeros((b, a), np.uint8)
+        for y in range(4, b - 4, 12):
+            img[y, 4:a - 4] = 23
+            if y + 12 < b - 4:
+                img[y:y + 12, a - 5 if (y // 12) % 2 == 0 else 4] = 23
+        img[4, 4:7] = 60
+        return np.repeat((img if kind == "winding" else img.T)[:, :, None], 3, 2)
     img = np.zeros((h, w, 3), np.uint8)      # sparse corners: most rows have no score
     img[h // 3:h // 3 + 9, w // 4:w // 2] = 200
     img[2 * h // 3:, 5:9] = (10, 250, 60)
@@ -40,6 +50,13 @@ def test_harris_rows(gpu, kind, k, thr):
 def test_canny_thresholds_and_sizes(gpu, w, h, lower, upper):
     print(f"fused graph: {w}x{h}, Canny {lower}/{upper}", flush=True)
     _compare(_rgb("noise", w, h), lower, upper, 0.04, 0.0005)
+
+
+@pytest.mark.parametrize("kind", ["winding", "winding down"])
+@pytest.mark.parametrize("w,h", [(244, 106), (1284, 726)])
+def test_components_through_many_tiles(gpu, kind, w, h):
+    print(f"fused graph: {kind}, {w}x{h}", flush=True)
+    _compare(_rgb(kind, w, h), 80, 100, 0.04, 0.0005)
 
 
 def _compare(rgb, lower, upper, k, thr):
