@@ -641,7 +641,7 @@ typedef struct mvx_chain_image {
 
 typedef struct mvx_chain_plan {
     void *table;                                 /* device plan (in the caller's workspace) */
-    uint32_t count, numTiles, tile, workgroups;  /* images, tiles, tile shape index, persistent grid */
+    uint32_t count, numTiles, tile, workgroups;  /* images, tiles (up to whole waves), tile shape index, persistent grid */
     uint32_t tileWidth, tileHeight;
 } mvx_chain_plan_t;
 

@@ -18,16 +18,16 @@
 // not written (the Sobel node leaves them); Magnitude and Phase of those rows are computed from zero
 // gradients, which is what the nodes compute from the zeroed rows.  The half-size image comes from the same
 // input rows.
-// An output tile is TW x TH pixels of one image, TW / 8 lanes; a wave takes tiles that follow each other, and an
-// image's tiles are counted up to whole waves, so a wave's lanes share one image.  Where all tiles together
-// leave SIMDs idle, a tile's rows are split among several waves (the two rows above and below a lane's rows
-// are read and blurred again: small batches have the room).
+// An output tile is TW pixels of at most TH rows of one image, TW / 8 lanes; a wave takes tiles that follow each
+// other, and an image's tiles are counted up to whole waves, so a wave's lanes share one image.  Tiles are
+// lower where all together would leave SIMDs idle, and where an image has too few to fill its waves' lanes
+// (the two rows above and below a lane's rows are read and blurred again).
 //
 // Bound by memory and VALU issue alike: 8.25 bytes and 53 lane operations a pixel.  48 uneven images of
 // 118 Mpixel: 349 us with tiles in LDS (73 operations a pixel, a third of them blurring halos and unpacking
 // bytes twice), 283 us now.
 //
-// Schedule.  The waves' units of all images form one sequence (image after image, row-major inside an
+// Schedule.  The waves' tiles of all images form one sequence (image after image, row-major inside an
 // image).  The grid is persistent: it is a multiple of 8 workgroups, workgroup b runs on XCD b%8
 // (MI355X dispatches workgroups round-robin over its 8 XCDs), the sequence is cut into 8 equal
 // contiguous ranges, one per XCD, and the waves of an XCD stride through its range, so tiles
@@ -47,7 +47,8 @@ struct ChainRow {  // device plan: one 128-byte row per image
     uint32_t w, h;
     uint32_t srcStride, gxStride, gyStride, magStride, phaseStride, halfStride;
     uint32_t tilesX, tileBegin;  // tiles per row; index of the image's first tile in the sequence
-    uint32_t pad[10];
+    uint32_t rows;               // of a tile: even, a divisor of TH
+    uint32_t pad[9];
 };
 static_assert(sizeof(ChainRow) == 128, "plan row is 128 bytes");
 
@@ -251,22 +252,21 @@ struct ChainLane {
     }
 };
 
-// `rows` per lane (even, a divisor of TH); `units` waves' worth of work, TH / rows of them per wave of tiles
-template <int TW, int TH>
+// `units` waves' worth of tiles
+template <int TW>
 __global__ void __launch_bounds__(CHAIN_THREADS)
-k_chain_batch(const ChainRow *__restrict__ plan, uint32_t count, uint32_t units, uint32_t rows)
+k_chain_batch(const ChainRow *__restrict__ plan, uint32_t count, uint32_t units)
 {
     constexpr uint32_t LPT = TW / 8, TPW = 64 / LPT;   // lanes per tile, tiles per wave
     const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3, step = (gridDim.x >> 3) * (CHAIN_THREADS / 64);
     const uint32_t span = (units + 7u) / 8u;
     const uint32_t uBegin = xcd * span, uEnd = min(units, uBegin + span);
-    const uint32_t parts = TH / rows;
     for (uint32_t u = uBegin + slot * (CHAIN_THREADS / 64) + wave; u < uEnd; u += step) {
-        const uint32_t group = u / parts, part = u - group * parts;
-        const ChainRow &d = plan[find_image(plan, count, group * TPW)];
-        const uint32_t tile = group * TPW - d.tileBegin + lane / LPT, ty = tile / d.tilesX, tx = tile - ty * d.tilesX;
-        const int x = (int)(tx * TW + 8 * (lane % LPT)), y0 = (int)(ty * TH + part * rows);
+        const ChainRow &d = plan[find_image(plan, count, u * TPW)];
+        const uint32_t rows = d.rows;
+        const uint32_t tile = u * TPW - d.tileBegin + lane / LPT, ty = tile / d.tilesX, tx = tile - ty * d.tilesX;
+        const int x = (int)(tx * TW + 8 * (lane % LPT)), y0 = (int)(ty * rows);
         const int w = (int)d.w, h = (int)d.h, stride = (int)d.srcStride;
         if (x >= w || y0 >= h) continue;
         ChainLane L{d, w, h, stride, h * stride, x};
@@ -324,23 +324,44 @@ k_chain_batch(const ChainRow *__restrict__ plan, uint32_t count, uint32_t units,
 struct TileShape { int tw, th; };
 constexpr TileShape kShapes[MVX_CHAIN_TILE_COUNT] = {{16, 16}, {32, 16}, {32, 32}, {64, 16}, {64, 32}};
 
-typedef void (*ChainKernel)(const ChainRow *, uint32_t, uint32_t, uint32_t);
-constexpr ChainKernel kKernels[MVX_CHAIN_TILE_COUNT] = {k_chain_batch<16, 16>, k_chain_batch<32, 16>, k_chain_batch<32, 32>,
-                                                        k_chain_batch<64, 16>, k_chain_batch<64, 32>};
+typedef void (*ChainKernel)(const ChainRow *, uint32_t, uint32_t);
+constexpr ChainKernel kKernels[MVX_CHAIN_TILE_COUNT] = {k_chain_batch<16>, k_chain_batch<32>, k_chain_batch<32>, k_chain_batch<64>,
+                                                        k_chain_batch<64>};
 // tiles one wave takes side by side
 constexpr uint32_t tiles_per_wave(uint32_t tile) { return 64u / ((uint32_t)kShapes[tile].tw / 8u); }
 
-// Rows a lane streams: the tile's, halved down to 2 while the whole batch is fewer than 8192 waves (eight for each of
+// an image's waves with tiles of `rows` rows
+inline uint64_t image_waves(uint32_t w, uint32_t h, uint32_t rows, uint32_t tile)
+{
+    const uint32_t tw = (uint32_t)kShapes[tile].tw, per = tiles_per_wave(tile);
+    return ((uint64_t)((w + tw - 1) / tw) * ((h + rows - 1) / rows) + per - 1) / per;
+}
+
+// Rows a lane streams at most: the tile shape's, halved down to 2 while the whole batch (`waves` of tiles of the
+// shape's height) is fewer than 8192 waves (eight for each of
 // the 1024 SIMDs, of which about four run at a time, so that no SIMD ends long after the others: 48 uneven images with
 // 64x32 tiles took 294 us at 2048, 283 at 8192); a lane's rows cost one more load and blur above and below them each.
 // A small batch is bound by the chain of a lane's rows, each a wait for memory: one 320x240 image 9.8 us with no fewer
 // than 4 rows, 6.7 with 2, 4096x2160 10.6 and 9.0.
-inline uint32_t rows_per_lane(uint32_t numTiles, uint32_t tile)
+inline uint32_t batch_rows(uint64_t waves, uint32_t tile)
 {
     uint32_t rows = (uint32_t)kShapes[tile].th;
-    uint64_t waves = numTiles / tiles_per_wave(tile);
     while (rows > 2 && waves < 8192) { rows /= 2; waves *= 2; }
     return rows;
+}
+
+// Rows a lane streams of one image: of those up to the batch's the ones with the least work, a wave's being its rows
+// and the four more that it loads.  An image much smaller than a wave of tiles so gets more, lower ones that fill
+// the wave's lanes (64x32 tiles: 4096 images of 64x64 36 us, 112 with all at the batch's rows; 1024 of them 14 and 36).
+inline uint32_t image_rows(uint32_t w, uint32_t h, uint32_t most, uint32_t tile)
+{
+    uint32_t best = most;
+    uint64_t least = image_waves(w, h, most, tile) * (most + 4);
+    for (uint32_t rows = most / 2; rows >= 2; rows /= 2) {
+        const uint64_t work = image_waves(w, h, rows, tile) * (rows + 4);
+        if (work < least) { least = work; best = rows; }
+    }
+    return best;
 }
 
 inline bool plane_ok_cb(const void *p, uint32_t w, uint32_t stride, uint32_t bpp)
@@ -417,10 +438,15 @@ extern "C" int mvx_ChainBatch_prepare(const mvx_chain_image_t *images, uint32_t 
         return MVX_ERROR_INVALID_PARAMETERS;
     const TileShape s = kShapes[tile];
     std::vector<ChainRow> rows(count);
+    uint64_t waves = 0;
+    for (uint32_t i = 0; i < count; i++) {
+        if (!image_ok(images[i])) return MVX_ERROR_INVALID_PARAMETERS;
+        waves += image_waves(images[i].width, images[i].height, (uint32_t)s.th, tile);
+    }
+    const uint32_t most = batch_rows(waves, tile);
     uint64_t tiles = 0;
     for (uint32_t i = 0; i < count; i++) {
         const mvx_chain_image_t &im = images[i];
-        if (!image_ok(im)) return MVX_ERROR_INVALID_PARAMETERS;
         ChainRow &r = rows[i];
         std::memset(&r, 0, sizeof(r));
         r.src = im.src; r.gx = im.gx; r.gy = im.gy; r.mag = im.mag; r.phase = im.phase; r.half = im.half;
@@ -429,8 +455,8 @@ extern "C" int mvx_ChainBatch_prepare(const mvx_chain_image_t *images, uint32_t 
         r.magStride = im.magStride; r.phaseStride = im.phaseStride; r.halfStride = im.halfStride;
         r.tilesX = (im.width + s.tw - 1) / s.tw;
         r.tileBegin = (uint32_t)tiles;
-        const uint64_t own = (uint64_t)r.tilesX * ((im.height + s.th - 1) / s.th), per = tiles_per_wave(tile);
-        tiles += (own + per - 1) / per * per;   // whole waves: a wave's lanes share one image
+        r.rows = image_rows(im.width, im.height, most, tile);
+        tiles += image_waves(im.width, im.height, r.rows, tile) * tiles_per_wave(tile);   // a wave's lanes share one image
         if (tiles >= (1ull << 31)) return MVX_ERROR_INVALID_PARAMETERS;
     }
     int occ = 0;
@@ -442,7 +468,7 @@ extern "C" int mvx_ChainBatch_prepare(const mvx_chain_image_t *images, uint32_t 
     const uint32_t perCu = workgroupsPerCU == 0 ? (uint32_t)occ : std::min<uint32_t>(workgroupsPerCU, (uint32_t)occ);
     uint32_t wgs = (uint32_t)cus * perCu;
     // no more workgroups than there are waves' units for (rounded to a multiple of the 8 XCDs)
-    const uint64_t units = tiles / tiles_per_wave(tile) * ((uint32_t)s.th / rows_per_lane((uint32_t)tiles, tile));
+    const uint64_t units = tiles / tiles_per_wave(tile);
     const uint64_t perXcd = ((units + 7) / 8 + CHAIN_THREADS / 64 - 1) / (CHAIN_THREADS / 64);
     wgs = (uint32_t)std::min<uint64_t>(wgs, perXcd * 8);
     wgs = std::max<uint32_t>(8u, wgs & ~7u);
@@ -464,11 +490,8 @@ extern "C" int mvx_ChainBatch_run(mvx_stream_t stream, const mvx_chain_plan_t *p
         (plan->workgroups & 7u))
         return MVX_ERROR_INVALID_PARAMETERS;
     if (plan->numTiles == 0) return MVX_SUCCESS;
-    const uint32_t rows = rows_per_lane(plan->numTiles, plan->tile);
-    const uint64_t units = (uint64_t)(plan->numTiles / tiles_per_wave(plan->tile)) * ((uint32_t)kShapes[plan->tile].th / rows);
-    if (units > UINT32_MAX) return MVX_ERROR_INVALID_PARAMETERS;   // not a plan of mvx_ChainBatch_prepare
     hipLaunchKernelGGL(kKernels[plan->tile], dim3(plan->workgroups), dim3(CHAIN_THREADS), 0, stream_of(stream),
-                       (const ChainRow *)plan->table, plan->count, (uint32_t)units, rows);
+                       (const ChainRow *)plan->table, plan->count, plan->numTiles / tiles_per_wave(plan->tile));
     MVX_LAUNCH_CHECK();
     return MVX_SUCCESS;
 }

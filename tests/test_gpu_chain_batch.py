@@ -1,7 +1,7 @@
 """GPU parity of the batched fused chain (Gaussian3x3 -> Sobel GXY -> Magnitude + Phase, ScaleImage
 to half size) over images of uneven sizes in one persistent launch: bit-exact against the oracle's
 node-by-node chain, against the per-node HIP kernels, against hashes of the reference CPU engine
-(tests/golden/vision_golden_chain_batch.json), for every tile shape, through a captured HIP graph
+(tests/golden/vision_golden_chain_batch.json), for every tile shape and height, through a captured HIP graph
 replayed several times, and after the autotuner's pick."""
 import json
 import os
@@ -12,7 +12,7 @@ import torch
 
 from mivisionx_amd import synth
 from mivisionx_amd.device import Plane
-from mivisionx_amd.pipelines import CHAIN_TILES, ChainBatch
+from mivisionx_amd.pipelines import CHAIN_TILES, ChainBatch, ChainImage
 from util import assert_same, sha
 
 pytestmark = pytest.mark.gpu
@@ -52,6 +52,39 @@ def test_small_uneven_every_tile_vs_oracle(small_batch, tile):
     b = ChainBatch([Plane.from_array(a) for a in imgs]).prepare(tile)
     b.run()
     _check(b, want, f"tile {CHAIN_TILES[tile]}")
+
+
+# sizes whose waves are full at the tallest tiles, so that they keep them, cut off at every remainder
+TALL = [(510, 130), (512, 158), (256, 66), (1022, 34), (254, 16)]
+
+
+@pytest.fixture(scope="module")
+def tall_batch(small_batch, orc):
+    imgs = [synth.scene_u8(w, h, seed=90 + i) for i, (w, h) in enumerate(TALL)]
+    return small_batch[0] + imgs, small_batch[1] + [_oracle(orc, a) for a in imgs]
+
+
+@pytest.mark.parametrize("tile,most", [(t, m) for t, (_, th) in enumerate(CHAIN_TILES) for m in (32, 16, 8, 4, 2) if m <= th])
+def test_rows_per_lane_vs_oracle(tall_batch, tile, most):
+    """every height of the tiles of every shape: the height follows from the size of the batch (8192 waves of tiles
+    of the shape's height, or of ones half as high, ..), so the images come as often as that takes; a repeated
+    image writes the same bytes to the same planes"""
+    imgs, want = tall_batch
+    tw, th = CHAIN_TILES[tile]
+    waves = sum(-(-(-(-a.shape[1] // tw) * -(-a.shape[0] // th)) // (512 // tw)) for a in imgs)
+    times = -(-8192 * most // th // waves) if most > 2 else 1
+    b = ChainBatch([Plane.from_array(a) for a in imgs])
+    n = len(imgs)
+    b._arr = (ChainImage * (n * times))(*[b._arr[i % n] for i in range(n * times)])
+    b.src = b.src * times
+    b.ws = torch.zeros(b.ws_size * times, dtype=torch.uint8, device="cuda")
+    b.ws_size = b.ws.numel()
+    b.prepare(tile)
+    rows = b.ws.view(n * times, 128)[:n, 88:92].contiguous().view(torch.int32).flatten().tolist()    # the plan's table
+    print(f"chain batch: tile {tw}x{th}, {n * times} images, rows per lane {rows}", flush=True)
+    assert max(rows) == most
+    b.run()
+    _check(b, want, f"tile {CHAIN_TILES[tile]}, at most {most} rows")
 
 
 @pytest.mark.parametrize("per_cu", [1, 2, 0])
