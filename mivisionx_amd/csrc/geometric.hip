@@ -407,14 +407,15 @@ MVX_DEV void rgb_of_chroma(float U, float V, float &R, float &G, float &B)
 }
 MVX_DEV uint32_t rgb_byte(float f) { return (uint32_t)fminf(fmaxf(f, 0.0f), 255.0f); }
 
-// One thread: 8 columns of 2 rows, their chroma read and scaled once.  Where every plane and stride is a multiple of
-// 4 bytes (DWORDS) and the 8 columns are in the image it loads and stores words, else bytes.
+// One thread: 8 columns of 2 rows, their chroma read and scaled once, in words at whatever address the planes and
+// strides put them; the last columns of a row, where fewer than 8 are left, in bytes.
 // Bound by memory at large sizes, by latency at small ones.  NV12, a byte at a time and 4 pixels a thread against now:
-// 1920x1080 7.0 and 4.3 us, 3840x2160 18.7 and 8.8 us.
-typedef uint32_t rgb_u32x2 __attribute__((ext_vector_type(2), aligned(4)));
-typedef uint32_t rgb_u32x3 __attribute__((ext_vector_type(3), aligned(4)));
+// 1920x1080 7.0 and 4.3 us, 3840x2160 18.7 and 8.8 us, also at odd addresses and strides.
+typedef uint32_t rgb_u32_any __attribute__((aligned(1)));
+typedef uint32_t rgb_u32x2 __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t rgb_u32x3 __attribute__((ext_vector_type(3), aligned(1)));
 
-template <bool NV12, bool DWORDS>
+template <bool NV12>
 __global__ void __launch_bounds__(256)
 k_rgb_from_yuv(uint32_t w, uint32_t h, uint8_t *__restrict__ dst, uint32_t dstStride, const uint8_t *__restrict__ ys, uint32_t yStride,
                const uint8_t *__restrict__ us, uint32_t uStride, const uint8_t *__restrict__ vs, uint32_t vStride)
@@ -425,7 +426,7 @@ k_rgb_from_yuv(uint32_t w, uint32_t h, uint8_t *__restrict__ dst, uint32_t dstSt
     const uint8_t *y[2] = {ys + (size_t)(2 * r2) * yStride + x0, ys + (size_t)(2 * r2 + 1) * yStride + x0};
     const uint8_t *u = us + (size_t)r2 * uStride + (NV12 ? x0 : x0 / 2), *v = NV12 ? u + 1 : vs + (size_t)r2 * vStride + x0 / 2;
     uint8_t *d[2] = {dst + (size_t)(2 * r2) * dstStride + 3ull * x0, dst + (size_t)(2 * r2 + 1) * dstStride + 3ull * x0};
-    if (DWORDS && cols == 8) {
+    if (cols == 8) {
         const rgb_u32x2 Y[2] = {*(const rgb_u32x2 *)y[0], *(const rgb_u32x2 *)y[1]};
         uint32_t c[2];   // U0 V0 U1 V1, ..
         if (NV12) {
@@ -433,7 +434,7 @@ k_rgb_from_yuv(uint32_t w, uint32_t h, uint8_t *__restrict__ dst, uint32_t dstSt
             c[0] = q.x;
             c[1] = q.y;
         } else {
-            const uint32_t U = *(const uint32_t *)u, V = *(const uint32_t *)v;
+            const uint32_t U = *(const rgb_u32_any *)u, V = *(const rgb_u32_any *)v;
             c[0] = __builtin_amdgcn_perm(V, U, 0x05010400u);
             c[1] = __builtin_amdgcn_perm(V, U, 0x07030602u);
         }
@@ -491,9 +492,7 @@ int rgb_from_yuv(mvx_stream_t stream, uint32_t w, uint32_t h, uint8_t *dst, uint
     if (!dst || !y || !u || (!nv12 && !v) || dstStride < 3 * w || yStride < w || uStride < (nv12 ? w : w / 2) ||
         (!nv12 && vStride < w / 2))
         return MVX_ERROR_INVALID_PARAMETERS;
-    const bool dwords = (((uintptr_t)dst | dstStride | (uintptr_t)y | yStride | (uintptr_t)u | uStride | (nv12 ? 0 : (uintptr_t)v | vStride)) & 3u) == 0;
-    const auto kernel = nv12 ? (dwords ? k_rgb_from_yuv<true, true> : k_rgb_from_yuv<true, false>)
-                             : (dwords ? k_rgb_from_yuv<false, true> : k_rgb_from_yuv<false, false>);
+    const auto kernel = nv12 ? k_rgb_from_yuv<true> : k_rgb_from_yuv<false>;
     hipLaunchKernelGGL(kernel, dim3((w + 511) / 512, (h / 2 + 3) / 4), dim3(64, 4), 0, stream_of(stream), w, h, dst, dstStride, y, yStride, u,
                        uStride, nv12 ? u : v, nv12 ? uStride : vStride);
     MVX_LAUNCH_CHECK();

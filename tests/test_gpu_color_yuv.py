@@ -72,7 +72,7 @@ def test_yuv_nodes(gpu, orc):
 @pytest.mark.parametrize("w,h", [(2, 2), (6, 4), (8, 2), (10, 6), (14, 10), (512, 4), (514, 8), (1034, 2)])
 @pytest.mark.parametrize("off,pad", [(0, 0), (4, 4), (1, 2), (2, 3)])
 def test_rgb_from_yuv_addresses(gpu, orc, w, h, off, pad):
-    """planes at any address and stride: word accesses only where every plane and stride allows them, widths around the
+    """planes at any address and stride, words read and written wherever they lie: widths around the
     8 columns of a thread and the 512 of a workgroup's row; nothing is written past a row's 3w bytes"""
     y, u, v = _planes(w, h, w + 7 * h)
     uv = np.stack([u, v], -1).reshape(h // 2, w)
