@@ -1,13 +1,16 @@
 """All pyramid levels in one tracking launch against one launch per level (which a workspace without room
 for a derivative image per level still takes): the same keypoints, call after call, at level widths with
 and without whole 8-column chunks -- the cells no level writes keep the last call's values in both -- and
-windows on both sides of the small-window kernel.  The per-level form is the oracle-tested one."""
+windows on both sides of the small-window kernel.  With the workspace of the queried size pyramids of halved
+levels take the single launch, which the other LK tests so compare with the oracle; the launch per level is
+compared with it here."""
 import pytest
 import torch
 
 from mivisionx_amd import synth
 from mivisionx_amd.device import Plane, call
 from mivisionx_amd.pipelines import PyrLKTracker, pyramid_dims
+from test_gpu_lk import BOTH, EPS, ITER, GpuLK, _estimate, _same
 
 pytestmark = pytest.mark.gpu
 
@@ -27,6 +30,28 @@ def _align256(n):
     return (n + 255) // 256 * 256
 
 
+def _level_at_a_time_size(w, h, n):
+    """row scratch + one derivative image + positions"""
+    return _align256(_align256(_align256((2 * w + 64) * 2) + w * h * 4) + 8 * n)
+
+
+@pytest.mark.parametrize("w,h,levels,n,win,term,use", [(320, 240, 3, 400, 9, BOTH, 0), (640, 480, 4, 1000, 9, ITER, 0),
+                                                       (333, 200, 3, 300, 7, BOTH, 1), (256, 128, 2, 300, 15, BOTH, 0),
+                                                       (200, 96, 2, 256, 12, EPS, 1)])
+def test_level_at_a_time_matches_oracle(gpu, orc, w, h, levels, n, win, term, use):
+    print(f"LK {w}x{h}, {levels} levels one launch each, window {win}", flush=True)
+    old, new, _ = synth.lk_pair(w, h, 21)
+    kp = synth.lk_keypoints(w, h, n, 22, margin=4)
+    kp["tracking_status"][::13] = 0
+    op, np_ = orc.pyramid(old, levels), orc.pyramid(new, levels)
+    g = GpuLK(op, np_, n)
+    assert _level_at_a_time_size(w, h, n) < g.ws_size
+    g.ws_size = _level_at_a_time_size(w, h, n)
+    got = g.run(kp, _estimate(kp), term, 0.01, 20, use, win)
+    want = orc.lk(op, np_, kp, _estimate(kp), term, 0.01, 20, use, win)
+    _same(got, want, f"lk {w}x{h} L{levels} win{win} term {term:x} est {use}")
+
+
 @pytest.mark.parametrize("w,h,levels", [(96, 64, 2), (157, 101, 3), (203, 90, 3), (334, 250, 4), (640, 480, 4)])
 @pytest.mark.parametrize("win", [3, 5, 8, 9, 11, 12, 15])
 def test_together_equals_level_at_a_time(gpu, w, h, levels, win):
@@ -41,8 +66,8 @@ def test_together_equals_level_at_a_time(gpu, w, h, levels, win):
     for together in (True, False):
         results = []
         t = PyrLKTracker(pyrs[0], pyrs[1], n)
-        if not together:     # row scratch + one derivative image + positions
-            t.ws_size = _align256(_align256(_align256((2 * w + 64) * 2) + w * h * 4) + 8 * n)
+        if not together:
+            t.ws_size = _level_at_a_time_size(w, h, n)
         t.set_points(kp)
         for old, new in ((0, 1), (1, 2), (2, 1), (1, 2)):     # successive calls on one workspace
             for lv in range(levels):

@@ -99,3 +99,53 @@ def test_adjoint_z_at_the_ends_of_f32(gpu, scale, gscale, sscale):
         assert float((gH - wH).abs().max()) <= 1e-5 * float(wH.abs().max()), f"{gH}\n{wH}"
         if want_src:
             assert float((gs.double() - ws).abs().max()) <= 1e-5 * float(ws.abs().max())
+
+
+# u and v are exact in F32 and no sample lies on a cell boundary: multiples of 1/4 (1/8) plus 1/8 (1/16)
+EXACT = {"shift": [1, 0, 3.125, 0, 1, -2.375, 0, 0, 1], "shrink_rotate": [1.5, 0.5, 0.125, -0.75, 1.25, 30.375, 0, 0, 1],
+         "enlarge": [0.25, 0, 0.125, 0, 0.375, 0.0625, 0, 0, 1]}
+
+
+@pytest.mark.parametrize("name", EXACT)
+@pytest.mark.parametrize("n,w,h", [(4, 1021, 1003), (350, 130, 37), (704, 63, 83)])
+def test_adjoint_batches_of_eight_rows(gpu, n, w, h, name):
+    """batches of 2048 tiles and more, whose waves take eight rows each: last row groups cut off, all four kernels.
+    Positions and weights are exact, so what is left is the rounding of terms and F32 partial sums (of at most 8
+    rows and 64 columns): dL/dH within 1e-6 of the sum of its terms' sizes, a gradient of the source, a sum of at
+    most 16 terms below 1, within 1e-5, the loss within 1e-5 of itself."""
+    print(f"adjoint of eight-row waves, {name}: {n} images of {w}x{h}", flush=True)
+    assert n * -(-w // 64) * -(-h // 32) >= 2048
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    src = torch.rand((n, h, w), generator=gen, device="cuda")
+    g = torch.rand((n, h, w), generator=gen, device="cuda") - 0.3
+    g[:, ::3, ::5] = 0.0
+    H = torch.tensor([EXACT[name]], dtype=torch.float64, device="cuda").repeat(n, 1)
+    H[:, 2] += torch.arange(n, device="cuda") % 7                  # each image its own
+    H[:, 5] -= torch.arange(n, device="cuda") % 5
+    s64, H64 = src.double().requires_grad_(True), H.clone().requires_grad_(True)
+    out = warp64(s64, H64.reshape(-1, 3, 3), (h, w))
+    ys, xs = torch.meshgrid(torch.arange(h, dtype=torch.float64, device="cuda"), torch.arange(w, dtype=torch.float64, device="cuda"),
+                            indexing="ij")
+    u, v = (H[:, k, None, None] * xs + H[:, k + 1, None, None] * ys + H[:, k + 2, None, None] for k in (0, 3))
+    inside = (u > -1) & (u < w) & (v > -1) & (v < h)
+    terms = (torch.sqrt(1 + xs * xs + ys * ys) * torch.sqrt(1 + u * u + v * v)) * inside
+
+    def close(gH, gs, loss, what, gout):
+        wantS, wantH = torch.autograd.grad(loss, (s64, H64), retain_graph=True)
+        err, bound = (gH - wantH).abs().amax(1), 1e-6 * (terms * gout.abs()).sum((1, 2))
+        print(f"  {what}: {float((err / wantH.abs().amax(1)).max()):.1e} of dL/dH off, bound {float((bound / wantH.abs().amax(1)).max()):.1e}", flush=True)
+        assert (err <= bound).all(), f"{what}: image {int((err / bound).argmax())}"
+        if gs is not None:
+            assert float((gs.double() - wantS).abs().max()) <= 1e-5, what
+
+    for want_src in (True, False):
+        gs, gH = align.warp_adjoint(g, src, H, want_src=want_src)
+        close(gH, gs, (out * g.double()).sum(), f"dL/dH, dL/dsource {want_src}", g.double())
+    res = out - g.double()
+    want = 0.25 * (res ** 2).sum(dim=(1, 2))
+    l2 = align.L2Grad(src, g)
+    for gsrc in (torch.zeros_like(src), None):
+        loss, gH = torch.zeros(n, dtype=torch.float64, device="cuda"), torch.zeros((n, 9), dtype=torch.float64, device="cuda")
+        l2(H, 0.25, loss, gH, accumulate=False, gsrc=gsrc)
+        assert float(((loss - want.detach()) / want.detach()).abs().max()) <= 1e-5
+        close(gH, gsrc, want.sum(), f"the loss, dL/dsource {gsrc is not None}", 0.5 * res.detach())
