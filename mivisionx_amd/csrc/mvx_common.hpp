@@ -100,6 +100,23 @@ MVX_DEV float div_by_const_rn(float a, float b, float y)
     return r == 0.0f ? q : fmaf(r, y, q);
 }
 
+// 1 / z for z in [2^-60, 2^60], correctly rounded: the hardware's reciprocal and one Newton step (checked for every
+// mantissa, tests/hip/probe_arith.hip; powers of two only shift the exponents)
+MVX_DEV float recip_usual(float z)
+{
+    const float r = __builtin_amdgcn_rcpf(z);
+    return fmaf(fmaf(-z, r, 1.f), r, r);
+}
+
+// n / z given r = recip_usual(z): the product, its exact remainder, one correction.  With r correctly rounded that
+// is the correctly rounded quotient (Markstein) where the product and the remainder neither overflow nor
+// underflow, as for any n of a sample position.
+MVX_DEV float div_by(float n, float z, float r)
+{
+    const float q = n * r;
+    return fmaf(fmaf(-q, z, n), r, q);
+}
+
 // RN(1/b) in single precision: the double quotient is within half a double ulp of 1/b, and 1/b
 // (b a float) is never a single-precision rounding midpoint, so rounding it to float is exact
 inline float recip_rn(float b) { return (float)(1.0 / (double)b); }

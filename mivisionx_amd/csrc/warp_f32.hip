@@ -186,13 +186,6 @@ MVX_DEV void block_sum_store(const float (&acc)[WF_SLOTS], float *out, uint32_t 
     }
 }
 
-// n / z from a reciprocal r of z that is good to an ulp: the product, its exact remainder, one correction
-MVX_DEV float div_by(float n, float z, float r)
-{
-    const float q = n * r;
-    return fmaf(fmaf(-q, z, n), r, q);
-}
-
 MVX_DEV bool wave_all(bool v) { return __builtin_amdgcn_ballot_w64(v) == __builtin_amdgcn_ballot_w64(true); }
 
 // dL/dsrc of one wave's samples, taken row by row.  Four atomics a pixel were the larger part of the
@@ -249,10 +242,10 @@ struct SrcGrad {
 // of a lane's rows, so only the sums of a, b, c and of a Y, b Y, c Y are kept and the X sums formed once;
 // rows whose samples all lie inside the source, in front and with z in [2^-60, 2^60] (the usual case) take
 // their four pixels with two unchecked loads off one 32-bit offset, others clamped loads, and where z or a
-// position is out of the ordinary the plain divisions.  The sample positions follow project() operation by
-// operation, so forward and adjoint sample the same cells.  Eight waves a SIMD hide the loads better than
-// more loads in flight per wave: with two and four rows at a time (58 to 96 and 115 to 155 registers) the
-// batch below took 236 and 286 us in all, with one row 232.
+// position is out of the ordinary the plain divisions.  The sample positions are project()'s, operation by
+// operation and with quotients rounded as its divisions are, so forward and adjoint sample the same cells.
+// Eight waves a SIMD hide the loads better than more loads in flight per wave: with two and four rows at a time
+// (58 to 96 and 115 to 155 registers) the batch below took 236 and 286 us in all, with one row 232.
 // 64 pairs of 1024x1024 and their two smaller levels (L2, no source gradient), reductions included: 417 us
 // with four divisions, checked loads, ten sums a pixel and shuffle reductions; 232 us now.  With dL/dsrc, 8
 // images of 509x387: 42.7 us with four atomics a pixel, 20.5 us now.
@@ -285,8 +278,7 @@ k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t ti
         const float Y = (float)y;
         const float q = q0 + H.h7 * Y, z = q + H.h8;
         const float nu = (u0 + H.h1 * Y + H.h2) - X * q, nv = (v0 + H.d4 * Y + H.h5) - Y * q;
-        float rz = __builtin_amdgcn_rcpf(z);
-        rz = fmaf(fmaf(-z, rz, 1.f), rz, rz);
+        const float rz = recip_usual(z);
         float du = div_by(nu, z, rz), dv = div_by(nv, z, rz);
         float fu = floorf(du), fv = floorf(dv);
         Sample s;
@@ -352,8 +344,8 @@ k_warp_f32_adjoint(F32Plane S, F32Plane G, uint32_t dw, uint32_t dh, uint32_t ti
 }
 
 // dH[img][0..8] (and loss[img]) = F64 sums of the per-workgroup partials, in a fixed order; one workgroup
-// per image and slot (64 images, 1024 partials a slot: 18 us when one workgroup took all ten slots in turn,
-// ? us now)
+// per image and slot (64 images, 512 partials a slot: 18 us when one workgroup took all ten slots in turn,
+// 5 us now)
 __global__ void __launch_bounds__(256)
 k_reduce_partials(const float *partials, uint32_t blocks, double *gradH, double *loss, int accumulate)
 {

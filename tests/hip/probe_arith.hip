@@ -11,6 +11,8 @@
 //     integer-valued float below 2^32;
 //   * mag_sobel, mag_sobel_trunc and phase_sobel vs mag_body and mag_tail, mag_trunc and phase_px, for every
 //     pair of 3x3 Sobel gradients (-1020..1020 each);
+//   * recip_usual(z) vs IEEE single division 1 / z, every mantissa at three exponents, and div_by(n, z, .) vs n / z,
+//     every mantissa of z with a few hundred million dividends;
 //   * the lane mapping of the DPP wave_shl:1 control.
 #include "../../mivisionx_amd/csrc/arith.hpp"
 
@@ -88,6 +90,25 @@ __global__ void k_div_const(float b, float y, uint32_t *out)
     }
 }
 
+// every mantissa of z in [2^e, 2^(e+1)): the reciprocal, and 64 quotients each
+__global__ void k_recip(uint32_t e, uint32_t *out)
+{
+    const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= 1u << 23) return;
+    const float z = __uint_as_float((e << 23) | m), r = recip_usual(z);
+    bool same = __float_as_uint(r) == __float_as_uint(__fdiv_rn(1.f, z));
+    uint32_t s = m * 2654435761u + e;
+    for (int k = 0; k < 64; k++) {
+        s = s * 1664525u + 1013904223u;
+        const float n = __uint_as_float((s & 0x807fffffu) | ((100u + ((s >> 23) & 0x3fu)) << 23));   // 2^-27 .. 2^36, both signs
+        same = same && div_by(n, z, r) == __fdiv_rn(n, z);
+    }
+    if (!same) {
+        atomicAdd(out, 1u);
+        atomicCAS(out + 1, 0u, m);
+    }
+}
+
 // l2_pack_simd(f) against _mm_cvtps_epi32(_mm_sqrt_ps(f)) + unsigned 16-bit pack restated in double
 // (the float square root is the double one rounded to float: double rounding is innocuous for sqrt),
 // for f = (float)i, every integer 0 <= i < 2^32 (every integer-valued float below 2^32)
@@ -115,6 +136,7 @@ __global__ void k_dpp(int32_t *out)
 
 // result[0] = mismatches, result[1] = first mismatch packed as (b << 16) | a (b, a <= 32768)
 extern "C" int probe_div_small(uint32_t maxB, uint32_t *result) { return run(k_div, maxB, maxB, result); }
+extern "C" int probe_recip(uint32_t e, uint32_t *result) { return run(k_recip, 1u << 15, e, result); }
 extern "C" int probe_sobel_px(uint32_t maxG, uint32_t *result) { return run(k_sobel_px, 2 * maxG + 1, maxG, result); }
 extern "C" int probe_mag_body(uint32_t maxA, uint32_t *result) { return run(k_mag, maxA + 1, maxA, result); }
 

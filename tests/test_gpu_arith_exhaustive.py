@@ -44,6 +44,14 @@ def test_sobel_magnitude_and_phase_all_pairs(probe):
     assert bad == 0, f"{bad} pixels differ; first (gx + 1020, gy + 1020) = {first}"
 
 
+@pytest.mark.parametrize("exponent", [67, 126, 127, 186])
+def test_refined_reciprocal_all_mantissas(probe, exponent):
+    """the F32 warp adjoint's reciprocal is the correctly rounded one, and its quotients are the division's"""
+    out = (ctypes.c_uint32 * 2)()
+    assert probe.probe_recip(ctypes.c_uint32(exponent), out) == 0
+    assert out[0] == 0, f"{out[0]} mantissas differ; first {out[1]:#08x}"
+
+
 @pytest.mark.parametrize("gradient", [3])
 def test_harris_norm_division_all_floats(probe, gradient):
     """the Harris score divides by the fixed norm (255 * 2^(g-1) * 3)^4; the reciprocal-and-FMA
