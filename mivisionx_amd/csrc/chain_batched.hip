@@ -23,7 +23,7 @@
 // lower where all together would leave SIMDs idle, and where an image has too few to fill its waves' lanes
 // (the two rows above and below a lane's rows are read and blurred again).
 //
-// Bound by memory and VALU issue alike: 8.25 bytes and 53 lane operations a pixel.  48 uneven images of
+// Bound by memory and VALU issue alike: 8.25 bytes and 55 lane operations a pixel.  48 uneven images of
 // 118 Mpixel: 349 us with tiles in LDS (73 operations a pixel, a third of them blurring halos and unpacking
 // bytes twice), 283 us now.
 //

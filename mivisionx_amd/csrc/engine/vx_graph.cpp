@@ -587,10 +587,10 @@ vx_status verify_graph(_vx_graph *g)
             const bool written = n->kernel->params[i].dir != VX_INPUT;
             if (r->type == VX_TYPE_IMAGE) {
                 _vx_image *im = (_vx_image *)r;
-                // the fused supernode keeps the virtual YUV image and luma in LDS: nothing to allocate
+                // the fused supernode keeps the virtual YUV image and luma in registers: nothing to allocate
                 if (g->fused && im->isVirtual && (r == g->fused->cc->params[1] || r == g->fused->ex->params[2])) continue;
                 if (im->isVirtual && unallocated.count(r)) continue;
-                // the chain batch keeps each blurred image in LDS
+                // the chain batch keeps each blurred image in registers
                 if (g->chains && im->isVirtual && n->fused == FUSED_CHAIN) {
                     bool blur = false;
                     for (const ChainNodes &c : g->chains->chains) blur = blur || r == c.blur;

@@ -8,12 +8,6 @@ namespace mvx {
 
 // union-find with atomicMin linking (the larger root hangs under the smaller): the final root of a
 // component is its smallest index, whatever the order of the unions
-MVX_DEV uint32_t gfind(gptr_t<const uint32_t> par, uint32_t p)
-{
-    uint32_t l = par[p];
-    while (l != p) { p = l; l = par[p]; }
-    return p;
-}
 
 // One step of a find once all unions are done: p's parent is l, which is no root unless the answer is l.  The
 // links it passes are shortened by half: p now hangs under l's parent.  Roots are never written and every

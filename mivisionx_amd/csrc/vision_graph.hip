@@ -44,14 +44,10 @@ namespace mvx {
 
 constexpr int TW = 58, TH = 32;                  // luma tile
 constexpr int HY = 3;                            // luma halo: Sobel 1 + Harris window 1 + NMS 1
-constexpr int TP = 64;                           // LDS row pitch (one wave row)
+constexpr int TP = 64;                           // row pitch of pixel indices in a tile (one wave row)
 constexpr int YH = TH + 2 * HY;                  // luma window rows (columns: TW + 6 = 64)
-constexpr int GH = TH + 4, GW = TW + 4;          // gradients, halo 2
-constexpr int MH = TH + 2, MW = TW + 2;          // Canny magnitude / Harris score, halo 1
 constexpr int TS = TH * TP;                      // tile-local pixel index space, p = ly * TP + lx
 constexpr int TNB = 2 * (TW + TH);               // union-find slots per tile: one per border pixel, at most
-constexpr int FT = 256;                          // threads of the tile kernels (4 waves)
-constexpr int NW = FT / 64;
 
 struct FrameDesc {
     const uint8_t *rgb; uint32_t rgbStride;
@@ -112,28 +108,6 @@ MVX_DEV uint32_t yflat(const FrameDesc &F, const GraphParams &P, int r, int c)
 
 // the value of lane + 1 of the wave (DPP wave_shl:1; lane 63 reads 0)
 MVX_DEV int lane_next(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, true); }
-
-// union-find with atomicMin linking (the larger root hangs under the smaller): the final root of
-// a component is its smallest index, whatever the order of the unions
-MVX_DEV int lfind(const int *L, int p)
-{
-    int l = L[p];
-    while (l != p) { p = l; l = L[p]; }
-    return p;
-}
-
-MVX_DEV void lunion(int *L, int a, int b)
-{
-    while (true) {
-        a = lfind(L, a);
-        b = lfind(L, b);
-        if (a == b) return;
-        if (a < b) { int t = a; a = b; b = t; }
-        const int old = atomicMin(&L[a], b);
-        if (old == a) return;
-        a = old;
-    }
-}
 
 MVX_DEV float lane_next_f(float v) { return __int_as_float(lane_next(__float_as_int(v))); }
 
@@ -873,9 +847,10 @@ static int lane_init(mvx_vision_lane *L)
 }
 
 // frames per chunk of the pipelined run: by default all frames in one chunk.  Smaller chunks overlap a
-// chunk's later stages with the next chunk's tile pass, but measured slower on MI355X at 4K (16 frames:
-// 0.834 ms per batch in one chunk, 0.893 in two, 1.065 in four): the tile pass is bound by VALU issue,
-// and the latency-bound union-find and pick waves resident beside it slow it by more than they hide.
+// chunk's later stages with the next chunk's tile pass, but measured slower on MI355X (16 frames in one chunk,
+// in two, in four: 540, 569 and 633 us at 3840x2160, 183, 221 and 276 at 1920x1080, 124, 150 and 231 at
+// 1284x726): the tile pass is bound by VALU issue, and the latency-bound union-find and pick waves resident
+// beside it slow it by more than they hide.
 static uint32_t mvx_vision_default_chunk(uint32_t nframes) { return nframes; }
 
 static void lane_free(mvx_vision_lane *L)
